@@ -49,6 +49,39 @@ def test_sample_matches_oracle(hip, n, t, k, p, ties):
     buf.free()
 
 
+def _edge_logits(kind, n):
+    x = _logits(n, n)
+    if kind == "equal":          # only the indices rank them
+        x[:] = 0.25
+    elif kind == "sorted":       # the largest side by side, in few groups
+        x = np.sort(x)
+    elif kind == "outliers":     # the whole range of values
+        x[::3] = np.finfo(np.float32).min
+        x[n // 2] = np.finfo(np.float32).max
+        x[1::5] = -np.inf
+    elif kind == "zeros":        # both zeros, and values that differ in the last bit
+        x = np.where(x > 0, np.float32(0.0), np.float32(-0.0)).astype(np.float32)
+        x[::7] = np.float32(1e-45)
+    return x
+
+
+@pytest.mark.parametrize("kind", ["normal", "equal", "sorted", "outliers", "zeros"])
+@pytest.mark.parametrize("n,k", [(1, 1), (15, 15), (17, 3), (256 * 16, 256), (256 * 16 + 1, 256), (4111, 255),
+                                 (32 * 8192, 256), (32 * 8192, 1)])
+def test_sample_edges(hip, kind, n, k):
+    """Group and block remainders, the smallest and largest vocabulary, and
+    values whose words crowd into few groups or few leading bits. Values of
+    few kinds over a wide softmax, so that every candidate can be drawn: the
+    probabilities of equal values are equal to the last bit on both sides."""
+    x = _edge_logits(kind, n)
+    buf = hip.alloc(n)
+    hip.write(buf, x)
+    dev, cpu = Sampler(1.5, k, 1.0, 7), ref.Sampler(1.5, k, 1.0, 7)
+    assert [dev.sample(hip, buf) for _ in range(24)] == [cpu.sample(x) for _ in range(24)]
+    assert dev.rng == cpu.state
+    buf.free()
+
+
 def test_sample_temperature_zero_is_argmax(hip):
     x = _logits(5000, 3)
     x[[10, 4000]] = x.max() + 1.0

@@ -496,7 +496,8 @@ int enqueue_step(th_state *s, bool chunked) {
                                   s->logits->ptr, s->s_part, &np));
     if (s->graph_keep) TH_HIP(th::launch_keep_logits(st, s->logits->ptr, (size_t)V, s->step));
     if (s->sampling)
-        TH_HIP(th::launch_sample(st, s->logits->ptr, (size_t)V, s->s_cand, s->s_sample, s->step, 1, step_embed(s)));
+        TH_HIP(th::launch_sample(st, s->logits->ptr, (size_t)V, s->s_cand, s->s_sample, s->step, 1, step_embed(s),
+                                 s->s_part));
     else
         TH_HIP(th::launch_pick_partials(st, s->s_part, (size_t)np, s->step, 1, step_embed(s)));
     return TH_OK;

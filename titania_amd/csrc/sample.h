@@ -24,13 +24,16 @@ struct SampleState {
     uint32_t token;     // the draw, when no StepState records it
 };
 
-// Device scratch the sampler needs for a vocabulary (candidate keys).
+// Device scratch the sampler needs for a vocabulary (the maxima below).
 size_t sample_scratch_bytes(size_t vocab);
 
 // Draws a token from `logits`: into st (recorded like launch_pick, with the
 // embedding row written for the next step) when st is not null, else into
-// ss->token. Advances ss->rng by one draw.
+// ss->token. Advances ss->rng by one draw. `maxima`, if not null, holds the
+// largest argmax_pack word of every 16 consecutive logits (the partials of
+// launch_step_logits); otherwise a launch of its own puts them in scratch.
 hipError_t launch_sample(hipStream_t s, const float *logits, size_t vocab, void *scratch, SampleState *ss,
-                         StepState *st, int advance, const PickEmbed &emb = PickEmbed());
+                         StepState *st, int advance, const PickEmbed &emb = PickEmbed(),
+                         const uint64_t *maxima = nullptr);
 
 }  // namespace th
