@@ -249,6 +249,36 @@ def test_qwen4b_prefill_gemm(hip, name, n):
     assert np.all(np.abs(got.astype(np.float64) - expected) <= 3e-5 * bound + 1e-6)
 
 
+@pytest.mark.parametrize("n", [2, 3, 4, 15, 16, 17, 50])
+@pytest.mark.parametrize("rows,cols", [(1, 8), (15, 24), (16, 504), (17, 512), (100, 520), (33, 768), (40, 1032),
+                                       (257, 1528), (16, 2056), (48, 2568), (5000, 1096), (24, 9736)])
+def test_few_token_matmul(hip, rows, cols, n):
+    """Row, column and token counts around the few-token kernel's tiles (16
+    rows, 32 columns a step, 2 to 10 steps a wave and eight waves a block,
+    chunks past them; one or several token tiles; K split or not), some
+    tokens 1e6 times the others and one infinite. An f32 sum of the products
+    in any order is within cols * 2^-24 of sum |w x|; three times that leaves
+    room for the terms that sum apart."""
+    rng = np.random.default_rng(rows * cols + n)
+    w = normal_bf16(rows * cols, 3, "few", 0.05)
+    x = rng.standard_normal((n, cols)).astype(np.float32)
+    x[::3] *= np.float32(1e6)
+    x[n - 1, cols // 2] = np.inf
+    wf = bf16_to_f32(w).astype(np.float64).reshape(rows, cols)
+    with np.errstate(invalid="ignore"):
+        exp = x.astype(np.float64) @ wf.T
+        bound = 3 * cols * 2.0**-24 * (np.abs(x).astype(np.float64) @ np.abs(wf).T)
+    bx, out = hip.alloc(x.size), hip.alloc(n * rows)
+    hip.write(bx, x)
+    hip.write(out, np.full(n * rows, np.nan, np.float32))
+    hip.matmul(out, hip.upload(Tensor((rows, cols), w)), bx)
+    got = hip.read(out).reshape(n, rows)
+    fine = np.isfinite(exp)
+    assert np.array_equal(np.isinf(exp), np.isinf(got)) and np.array_equal(exp[np.isinf(exp)], got[np.isinf(got)])
+    assert np.array_equal(np.isnan(exp), np.isnan(got))
+    assert np.all(np.abs(got[fine] - exp[fine]) <= bound[fine])
+
+
 @pytest.mark.parametrize("rows,cols,n", [(6144, 1024, 2000), (4096, 6144, 1024), (6144, 512, 8000),
                                          (2560, 1024, 8000)])
 def test_large_tile_gemm(hip, rows, cols, n):
@@ -441,7 +471,7 @@ def test_qkv_rope_append(hip, n, pos, shape):
                                                                                kc[(pos + n) * kvd:])
 
 
-@pytest.mark.parametrize("n,H,I", [(1, 1024, 3072), (1, 2560, 9728), (4, 1024, 3072), (32, 1024, 3072),
+@pytest.mark.parametrize("n,H,I", [(2, 1024, 3072), (15, 520, 1000), (1, 1024, 3072), (1, 2560, 9728), (4, 1024, 3072), (32, 1024, 3072),
                                    (2, 256, 512)])
 def test_gate_up_silu(hip, n, H, I):
     """th_gate_up_silu (the trait extension's gate_up_silu) against the

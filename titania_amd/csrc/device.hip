@@ -9,6 +9,7 @@
 #include <string>
 
 #include "common.h"
+#include "few.h"
 #include "gemm.h"
 #include "sample.h"
 #include "step.h"
@@ -101,6 +102,7 @@ int th_device_create(int ordinal, th_device **out) {
     }
     hipError_t e = hipStreamCreateWithFlags(&dev->stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipMalloc(&dev->token_out, 256);
+    if (e == hipSuccess) e = hipMalloc(&dev->few_part, th::kFewPartFloats * sizeof(float));
     if (e == hipSuccess) e = hipEventCreate(&dev->ev_begin);
     if (e == hipSuccess) e = hipEventCreate(&dev->ev_end);
     if (e != hipSuccess) {
@@ -123,6 +125,7 @@ void th_device_destroy(th_device *dev) {
     if (dev->tokens) (void)hipFree(dev->tokens);
     if (dev->scratch) (void)hipFree(dev->scratch);
     if (dev->token_out) (void)hipFree(dev->token_out);
+    if (dev->few_part) (void)hipFree(dev->few_part);
     if (dev->ev_begin) (void)hipEventDestroy(dev->ev_begin);
     if (dev->ev_end) (void)hipEventDestroy(dev->ev_end);
     if (dev->stream) (void)hipStreamDestroy(dev->stream);
@@ -362,7 +365,8 @@ int th_matmul(th_device *dev, th_buffer *out, const th_weight *w, const th_buffe
     if (n == 1 && th::step_gemv_supported((int)cols) && rows < ((size_t)1 << 30))
         TH_HIP(th::launch_step_gemv(dev->stream, w->ptr, (int)rows, (int)cols, x->ptr, out->ptr));
     else
-        TH_HIP(th::launch_matmul(dev->stream, out->ptr, w->ptr, rows, cols, x->ptr, n));
+        TH_HIP(th::launch_matmul(dev->stream, out->ptr, w->ptr, rows, cols, x->ptr, n, dev->few_part,
+                                 th::kFewPartFloats));
     return TH_OK;
 }
 
@@ -520,6 +524,10 @@ int th_qkv_rope_append(th_device *dev, th_buffer *q, th_buffer *k, th_buffer *v,
         TH_NOT_CAPTURING(dev, "a projection of 16 or more tokens (stream-ordered scratch)");
         const th::GemmOut o[3] = {{wq->ptr, qd, q->ptr}, {wk->ptr, kvd, k->ptr}, {wv->ptr, kvd, v->ptr}};
         TH_HIP(th::launch_gemm_outs(dev->stream, xb->ptr, n, H, o, 3));
+    } else if (n > 1 && th::few_supported(n, qd, H)) {
+        if (n >= th::kGemmMinTokens) TH_NOT_CAPTURING(dev, "a projection of 16 or more tokens (stream-ordered scratch)");
+        const th::GemmOut o[3] = {{wq->ptr, qd, q->ptr}, {wk->ptr, kvd, k->ptr}, {wv->ptr, kvd, v->ptr}};
+        TH_HIP(th::launch_few(dev->stream, xb->ptr, n, H, o, 3, nullptr, 1));
     } else {
         if (n >= th::kGemmMinTokens) TH_NOT_CAPTURING(dev, "a projection of 16 or more tokens (stream-ordered scratch)");
         TH_HIP(th::launch_matmul(dev->stream, q->ptr, wq->ptr, qd, H, xb->ptr, n));
@@ -568,6 +576,11 @@ int th_gate_up_silu(th_device *dev, th_buffer *gate, th_buffer *up, const th_wei
         TH_NOT_CAPTURING(dev, "a projection of 16 or more tokens (stream-ordered scratch)");
         const th::GemmOut o[2] = {{w_gate->ptr, I, gate->ptr}, {w_up->ptr, I, up->ptr}};
         TH_HIP(th::launch_gemm_outs(dev->stream, xb->ptr, n, H, o, 2));
+    } else if (n > 1 && th::few_supported(n, I, H)) {
+        if (n >= th::kGemmMinTokens) TH_NOT_CAPTURING(dev, "a projection of 16 or more tokens (stream-ordered scratch)");
+        // Both projections and silu(gate) * up in one launch; up unused.
+        TH_HIP(th::launch_few_silu(dev->stream, xb->ptr, n, H, w_gate->ptr, w_up->ptr, I, gate->ptr));
+        return TH_OK;
     } else {
         if (n >= th::kGemmMinTokens) TH_NOT_CAPTURING(dev, "a projection of 16 or more tokens (stream-ordered scratch)");
         TH_HIP(th::launch_matmul(dev->stream, gate->ptr, w_gate->ptr, I, H, xb->ptr, n));

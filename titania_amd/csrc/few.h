@@ -1,0 +1,35 @@
+// Matmuls of a few tokens (2 to 16 a tile) on the matrix cores.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstddef>
+#include <cstdint>
+
+#include "gemm.h"
+
+namespace th {
+
+// Partials of up to 15 tokens in four parts, up to 8192 rows (more rows do
+// not split: few_ksplit).
+constexpr size_t kFewPartFloats = (size_t)4 * 15 * 8192;
+
+// Whether launch_few takes rows of `cols` columns for n tokens: whole 16-byte
+// chunks, and offsets that fit its buffer descriptors.
+bool few_supported(size_t n, size_t rows, size_t cols);
+
+// out[t * rows + r] = w[r] . x[t] for t < n, for 1-3 matrices of `cols`
+// columns that share x. With ksplit > 1 (one matrix) the partial products go
+// to part[ksplit][n][rows], to be summed in order.
+hipError_t launch_few(hipStream_t s, const float *x, size_t n, size_t cols, const GemmOut *outs, int n_outs,
+                      float *part, int ksplit);
+
+// Ways launch_few's caller should split K for one [rows, cols] matrix, when
+// the consumer sums the partials (1: no split), at most kGemmMaxSplitK.
+int few_ksplit(size_t n, size_t rows, size_t cols);
+
+// h[t * inter + j] = silu(gate[j] . x[t]) * (up[j] . x[t]) (model/cpu.rs:151-155).
+hipError_t launch_few_silu(hipStream_t s, const float *x, size_t n, size_t cols, const uint16_t *gate,
+                           const uint16_t *up, size_t inter, float *h);
+
+}  // namespace th

@@ -78,6 +78,10 @@ bool gemm_qkv_huge_fused(size_t n, size_t q_rows, size_t kv_rows, size_t cols, s
 hipError_t launch_gemm_qkv_huge(hipStream_t s, const uint16_t *hi, const uint16_t *lo, size_t cols,
                                 const uint16_t *wq, const uint16_t *wk, const uint16_t *wv, const QkvPostArgs &a);
 
+// out[i] = part[i] + part[m + i] + ... over ksplit partials of m values, in
+// order (m a multiple of 4).
+hipError_t launch_splitk_sum(hipStream_t s, const float *part, float *out, size_t m, int ksplit);
+
 // Bytes of scratch launch_gemm_multi needs for n tokens of `cols` columns and
 // single-matrix outputs of up to `rows` rows (room for the split-K partials).
 size_t gemm_scratch_bytes(size_t n, size_t cols, size_t rows);

@@ -830,6 +830,15 @@ hipError_t launch_gemm_qkv(hipStream_t s, const uint16_t *hi, const uint16_t *lo
     return hipGetLastError();
 }
 
+hipError_t launch_splitk_sum(hipStream_t s, const float *part, float *out, size_t m, int ksplit) {
+    if (m == 0) return hipSuccess;
+    if (m % 4 || ((uintptr_t)part | (uintptr_t)out) % 16) return hipErrorInvalidValue;
+    const size_t m4 = m / 4;
+    splitk_sum_kernel<<<(unsigned)std::min<size_t>((m4 + 255) / 256, 4096), 256, 0, s>>>(
+        reinterpret_cast<const float4 *>(part), reinterpret_cast<float4 *>(out), m4, ksplit);
+    return hipGetLastError();
+}
+
 hipError_t launch_gemm_multi(hipStream_t s, const float *x, size_t n, size_t cols, const GemmOut *outs, int n_outs,
                              void *scratch, size_t scratch_bytes) {
     if (n == 0) return hipSuccess;
@@ -845,10 +854,7 @@ hipError_t launch_gemm_multi(hipStream_t s, const float *x, size_t n, size_t col
     hipError_t e = launch_gemm_split(s, x, n, cols, hi, lo);
     if (e == hipSuccess) e = launch_gemm_hl(s, hi, lo, n, cols, outs, n_outs, part, ksplit);
     if (e != hipSuccess || ksplit == 1) return e;
-    const size_t m4 = n * total / 4;
-    splitk_sum_kernel<<<(unsigned)std::min<size_t>((m4 + 255) / 256, 4096), 256, 0, s>>>(
-        reinterpret_cast<const float4 *>(part), reinterpret_cast<float4 *>(outs[0].out), m4, ksplit);
-    return hipGetLastError();
+    return launch_splitk_sum(s, part, outs[0].out, n * total, ksplit);
 }
 
 hipError_t launch_gemm_outs(hipStream_t s, const float *x, size_t n, size_t cols, const GemmOut *outs, int n_outs) {

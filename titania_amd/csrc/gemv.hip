@@ -1,12 +1,14 @@
 // Device::matmul (model/cpu.rs:49-77): out[t][r] = w[r] . x[t] with bf16
 // weights and f32 activations, fp32 accumulation.
 //
-// For the few-token case (decode, n <= 8 per pass) this is a bandwidth-bound
-// GEMV: each wave owns ROWS weight rows, every lane streams 16-byte chunks
-// (8 bf16) of each row, and a wave64 shuffle reduction finishes each dot
-// product. Larger batches go to the MFMA GEMM (gemm.hip).
+// For up to three tokens this is a bandwidth-bound GEMV: each wave owns ROWS
+// weight rows, every lane streams 16-byte chunks (8 bf16) of each row, and a
+// wave64 shuffle reduction finishes each dot product. More tokens go to the
+// matrix cores: few.hip below 16 tokens and for matrices that are not whole
+// tiles, the MFMA GEMM (gemm.hip) otherwise.
 #include "common.h"
 #include "device_util.h"
+#include "few.h"
 #include "gemm.h"
 
 namespace th {
@@ -93,7 +95,7 @@ static hipError_t gemv(hipStream_t s, float *out, const uint16_t *w, size_t rows
 }
 
 hipError_t launch_matmul(hipStream_t s, float *out, const uint16_t *w, size_t rows, size_t cols, const float *x,
-                         size_t n) {
+                         size_t n, float *part, size_t part_floats) {
     if (n == 0 || rows == 0) return hipSuccess;
     if (cols % 8 != 0) {
         gemv_scalar_kernel<<<dim3((unsigned)((rows + 3) / 4)), 256, 0, s>>>(out, w, rows, cols, x, n);
@@ -106,15 +108,24 @@ hipError_t launch_matmul(hipStream_t s, float *out, const uint16_t *w, size_t ro
         if (rows >= 4096) return gemv<2, 1>(s, out, w, rows, cols, x, 1, rows);
         return gemv<1, 1>(s, out, w, rows, cols, x, 1, rows);
     }
-    for (size_t t0 = 0; t0 < n; t0 += 8) {
-        int nt = (int)std::min<size_t>(8, n - t0);
-        hipError_t e;
-        if (nt <= 2) e = gemv<2, 2>(s, out + t0 * rows, w, rows, cols, x + t0 * cols, nt, rows);
-        else if (nt <= 4) e = gemv<2, 4>(s, out + t0 * rows, w, rows, cols, x + t0 * cols, nt, rows);
-        else e = gemv<2, 8>(s, out + t0 * rows, w, rows, cols, x + t0 * cols, nt, rows);
-        if (e != hipSuccess) return e;
+    // Two and three tokens stay here (x 4096 x 1024, 2 / 4 / 8 tokens: 4.2 /
+    // 5.6 / 8.7 us against few.hip's 5.5 / 5.6 / 5.7; 19456 x 2560, 2 / 3 / 4 /
+    // 8: 21.4 / 25.9 / 29.8 / 46.8 against 25.8 / 25.7 / 25.9 / 26.1).
+    if (n == 2) return gemv<2, 2>(s, out, w, rows, cols, x, 2, rows);
+    if (n == 3 || !few_supported(n, rows, cols)) {
+        for (size_t t0 = 0; t0 < n; t0 += 4) {
+            const hipError_t e = gemv<2, 4>(s, out + t0 * rows, w, rows, cols, x + t0 * cols,
+                                            (int)std::min<size_t>(4, n - t0), rows);
+            if (e != hipSuccess) return e;
+        }
+        return hipSuccess;
     }
-    return hipSuccess;
+    int ksplit = n < kGemmMinTokens ? few_ksplit(n, rows, cols) : 1;
+    if (!part || n * rows % 4 || (size_t)ksplit * n * rows > part_floats) ksplit = 1;
+    const GemmOut o{w, rows, out};
+    const hipError_t e = launch_few(s, x, n, cols, &o, 1, part, ksplit);
+    if (e != hipSuccess || ksplit == 1) return e;
+    return launch_splitk_sum(s, part, out, n * rows, ksplit);
 }
 
 }  // namespace th

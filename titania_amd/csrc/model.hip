@@ -19,6 +19,7 @@
 #include <cstdlib>
 
 #include "common.h"
+#include "few.h"
 #include "fused.h"
 #include "gemm.h"
 #include "sample.h"
@@ -548,6 +549,30 @@ int enqueue_fused(th_state *s, const uint32_t *tokens, size_t n, size_t pos, con
         return TH_OK;
     };
 
+    // The projections of a few tokens (and of shapes the GEMM does not take):
+    // q/k/v and gate/up in a launch each; o and down may split K, their
+    // partials (in the GEMM's scratch) summed by the norm that follows.
+    auto few = [&](size_t rows, size_t cols) { return n > 1 && th::few_supported(n, rows, cols); };
+    auto one_residual = [&]() {
+        res = s->fy;
+        nres = 1;
+        res_stride = 0;
+    };
+    auto single_few = [&](const uint16_t *w, size_t cols, const float *x) -> int {
+        one_residual();
+        const int ks = part && n < th::kGemmMinTokens && few(H, cols) ? th::few_ksplit(n, H, cols) : 1;
+        const th::GemmOut o{w, H, s->fy};
+        if (ks > 1) {
+            TH_HIP(th::launch_few(st, x, n, cols, &o, 1, part, ks));
+            res = part;
+            nres = ks;
+            res_stride = n * H;
+        } else {
+            TH_HIP(th::launch_matmul(st, s->fy, w, H, cols, x, n));
+        }
+        return TH_OK;
+    };
+
     TH_HIP(th::launch_embed(st, s->fx, m->embed->ptr, H, tokens, n));
     for (size_t i = 0; i < m->layers.size(); ++i) {
         const Layer &L = m->layers[i];
@@ -629,11 +654,16 @@ int enqueue_fused(th_state *s, const uint32_t *tokens, size_t n, size_t pos, con
                 TH_HIP(th::launch_qk_norm_rope_append(st, qa));
             }
         } else {
-            TH_HIP(th::launch_add_rmsnorm(st, s->fx, i ? s->fy : nullptr, s->fxb, n, L.attn_norm->ptr, H, eps));
+            TH_HIP(th::launch_add_rmsnorm_parts(st, s->fx, res, nres, res_stride, s->fxb, nullptr, nullptr, n,
+                                                L.attn_norm->ptr, H, eps));
             if (use_gemm(H) && th::gemm_supported(qd, H) && th::gemm_supported(nkv * hd, H)) {
                 const th::GemmOut o[3] = {
                     {L.q->ptr, qd, s->fq}, {L.k->ptr, nkv * hd, s->fk}, {L.v->ptr, nkv * hd, s->fv}};
                 TH_HIP(th::launch_gemm_multi(st, s->fxb, n, H, o, 3, s->fsplit, s->fsplit_bytes));
+            } else if (few(qd, H)) {
+                const th::GemmOut o[3] = {
+                    {L.q->ptr, qd, s->fq}, {L.k->ptr, nkv * hd, s->fk}, {L.v->ptr, nkv * hd, s->fv}};
+                TH_HIP(th::launch_few(st, s->fxb, n, H, o, 3, nullptr, 1));
             } else {
                 TH_HIP(th::launch_matmul(st, s->fq, L.q->ptr, qd, H, s->fxb, n));
                 TH_HIP(th::launch_matmul(st, s->fk, L.k->ptr, nkv * hd, H, s->fxb, n));
@@ -669,27 +699,30 @@ int enqueue_fused(th_state *s, const uint32_t *tokens, size_t n, size_t pos, con
         if (use_gemm(qd) && th::gemm_supported(H, qd)) {
             const th::GemmOut o{L.o->ptr, H, s->fy};
             TH_HIP(th::launch_gemm_multi(st, s->fatt, n, qd, &o, 1, s->fsplit, s->fsplit_bytes));
+            one_residual();
         } else {
-            TH_HIP(th::launch_matmul(st, s->fy, L.o->ptr, H, qd, s->fatt, n));
+            TRY(single_few(L.o->ptr, qd, s->fatt));
         }
-        TH_HIP(th::launch_add_rmsnorm(st, s->fx, s->fy, s->fxb, n, L.mlp_norm->ptr, H, eps));
+        TH_HIP(th::launch_add_rmsnorm_parts(st, s->fx, res, nres, res_stride, s->fxb, nullptr, nullptr, n,
+                                            L.mlp_norm->ptr, H, eps));
         if (use_gemm(H) && th::gemm_supported(I, H)) {
             const th::GemmOut o[2] = {{L.gate->ptr, I, s->fgate}, {L.up->ptr, I, s->fup}};
             TH_HIP(th::launch_gemm_multi(st, s->fxb, n, H, o, 2, s->fsplit, s->fsplit_bytes));
+            TH_HIP(th::launch_silu_mul(st, s->fgate, s->fup, n * I));
+        } else if (few(I, H)) {
+            TH_HIP(th::launch_few_silu(st, s->fxb, n, H, L.gate->ptr, L.up->ptr, I, s->fgate));
         } else {
             TH_HIP(th::launch_matmul(st, s->fgate, L.gate->ptr, I, H, s->fxb, n));
             TH_HIP(th::launch_matmul(st, s->fup, L.up->ptr, I, H, s->fxb, n));
+            TH_HIP(th::launch_silu_mul(st, s->fgate, s->fup, n * I));
         }
-        TH_HIP(th::launch_silu_mul(st, s->fgate, s->fup, n * I));
         if (use_gemm(I) && th::gemm_supported(H, I)) {
             const th::GemmOut o{L.down->ptr, H, s->fy};
             TH_HIP(th::launch_gemm_multi(st, s->fgate, n, I, &o, 1, s->fsplit, s->fsplit_bytes));
+            one_residual();
         } else {
-            TH_HIP(th::launch_matmul(st, s->fy, L.down->ptr, H, I, s->fgate, n));
+            TRY(single_few(L.down->ptr, I, s->fgate));
         }
-        res = s->fy;
-        nres = 1;
-        res_stride = 0;
     }
     // Only the last token's logits are wanted (model.rs:143-147).
     float *xl = s->fx + (n - 1) * H;
