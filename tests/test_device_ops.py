@@ -249,6 +249,46 @@ def test_qwen4b_prefill_gemm(hip, name, n):
     assert np.all(np.abs(got.astype(np.float64) - expected) <= 3e-5 * bound + 1e-6)
 
 
+@pytest.mark.parametrize("n", [16, 33, 64, 65, 130])
+@pytest.mark.parametrize("rows,cols", [(64, 64), (64, 1088), (192, 1280), (1088, 2048), (2560, 1152), (64, 4160)])
+def test_split_k_matmul(hip, rows, cols, n):
+    """Whole-tile matrices around the small GEMM tile's split of K (1 to 16
+    parts, uneven ones, one K step), one and several token tiles, tokens past
+    a tile's edge. Two bf16 terms of x are within 2^-17 of it; the f32 sums
+    add cols * 2^-24 of sum |w x| at most."""
+    rng = np.random.default_rng(rows + cols + n)
+    w = normal_bf16(rows * cols, 4, "splitk", 0.05)
+    x = rng.standard_normal((n, cols)).astype(np.float32)
+    wf = bf16_to_f32(w).astype(np.float64).reshape(rows, cols)
+    exp, size = x.astype(np.float64) @ wf.T, np.abs(x).astype(np.float64) @ np.abs(wf).T
+    bx, out = hip.alloc(x.size), hip.alloc(n * rows)
+    hip.write(bx, x)
+    hip.write(out, np.full(n * rows, np.nan, np.float32))
+    hip.matmul(out, hip.upload(Tensor((rows, cols), w)), bx)
+    got = hip.read(out).reshape(n, rows)
+    assert np.all(np.abs(got - exp) <= (2.0**-17 + cols * 2.0**-24) * size)
+
+
+@pytest.mark.parametrize("rows,dim,parts", [(1, 260, 0), (3, 896, 1), (1024, 1024, 1), (1025, 1024, 1), (5, 2560, 1),
+                                            (2, 3076, 1), (7, 4096, 1)])
+def test_add_rmsnorm_rows(hip, rows, dim, parts):
+    """Rows around the block-a-row norm's reach: lengths that are not whole
+    spans, one to four float4 a lane, row counts at the edge. Four roundings
+    of each factor: 8 * 2^-24 relative."""
+    rng = np.random.default_rng(rows + dim)
+    x, y = (rng.standard_normal((rows, dim)).astype(np.float32) for _ in range(2))
+    g = f32_to_bf16((1 + 0.1 * rng.standard_normal(dim)).astype(np.float32))
+    bx, by, xb = (hip.alloc(rows * dim) for _ in range(3))
+    hip.write(bx, x)
+    hip.write(by, y)
+    hip.add_rmsnorm(bx, by if parts else None, xb, hip.upload(Tensor((dim,), g)), 1e-6)
+    s = x + y if parts else x
+    assert np.array_equal(hip.read(bx).reshape(rows, dim), s)
+    s = s.astype(np.float64)
+    exp = s / np.sqrt((s * s).mean(1, keepdims=True) + 1e-6) * bf16_to_f32(g).astype(np.float64)
+    assert np.all(np.abs(hip.read(xb).reshape(rows, dim) - exp) <= 8 * 2.0**-24 * np.abs(exp))
+
+
 @pytest.mark.parametrize("n", [2, 3, 4, 15, 16, 17, 50])
 @pytest.mark.parametrize("rows,cols", [(1, 8), (15, 24), (16, 504), (17, 512), (100, 520), (33, 768), (40, 1032),
                                        (257, 1528), (16, 2056), (48, 2568), (5000, 1096), (24, 9736)])

@@ -24,10 +24,10 @@ struct th_device {
     // The device address of the no-alloc entry points' fixed array (looked up
     // once, at th_device_create, with this device current).
     void *noalloc_scratch = nullptr;
-    // Split-K partials of a few-token matmul: kFewPartFloats, for the device's
-    // life (a matmul of fewer than 16 tokens allocates nothing, so that it can
-    // be captured).
-    float *few_part = nullptr;
+    // Split-K partials of a matmul: th::kPartFloats, for the device's life (a
+    // matmul of fewer than 16 tokens allocates nothing, so that it can be
+    // captured, and an allocation costs more than most matmuls).
+    float *part = nullptr;
     // One u32 the argmax kernels leave their result in.
     uint32_t *token_out = nullptr;
     // th_timer_begin / th_timer_end.
@@ -124,10 +124,10 @@ size_t argmax_partials(size_t n);
 hipError_t launch_argmax(hipStream_t s, const float *x, size_t n, uint64_t *partials, uint32_t *token);
 hipError_t launch_argmax_partials(hipStream_t s, const float *x, size_t n, uint64_t *partials);
 
-// out[t*rows + r] = dot(w[r], x[t]) for t < n. A product of a few tokens may
-// split K, its partials in part (part_floats long; null: it does not split).
+// out[t*rows + r] = dot(w[r], x[t]) for t < n. Where it splits K, the partials
+// go to part (kPartFloats long; null: it does not split).
 hipError_t launch_matmul(hipStream_t s, float *out, const uint16_t *w, size_t rows, size_t cols, const float *x,
-                         size_t n, float *part = nullptr, size_t part_floats = 0);
+                         size_t n, float *part = nullptr);
 
 // Attention over caches addressed as base + pos * pos_stride + head * head_stride
 // (elements), f32 or bf16. The position is *pos_dev when pos_dev is not null.

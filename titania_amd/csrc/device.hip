@@ -102,7 +102,7 @@ int th_device_create(int ordinal, th_device **out) {
     }
     hipError_t e = hipStreamCreateWithFlags(&dev->stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipMalloc(&dev->token_out, 256);
-    if (e == hipSuccess) e = hipMalloc(&dev->few_part, th::kFewPartFloats * sizeof(float));
+    if (e == hipSuccess) e = hipMalloc(&dev->part, th::kPartFloats * sizeof(float));
     if (e == hipSuccess) e = hipEventCreate(&dev->ev_begin);
     if (e == hipSuccess) e = hipEventCreate(&dev->ev_end);
     if (e != hipSuccess) {
@@ -125,7 +125,7 @@ void th_device_destroy(th_device *dev) {
     if (dev->tokens) (void)hipFree(dev->tokens);
     if (dev->scratch) (void)hipFree(dev->scratch);
     if (dev->token_out) (void)hipFree(dev->token_out);
-    if (dev->few_part) (void)hipFree(dev->few_part);
+    if (dev->part) (void)hipFree(dev->part);
     if (dev->ev_begin) (void)hipEventDestroy(dev->ev_begin);
     if (dev->ev_end) (void)hipEventDestroy(dev->ev_end);
     if (dev->stream) (void)hipStreamDestroy(dev->stream);
@@ -365,8 +365,7 @@ int th_matmul(th_device *dev, th_buffer *out, const th_weight *w, const th_buffe
     if (n == 1 && th::step_gemv_supported((int)cols) && rows < ((size_t)1 << 30))
         TH_HIP(th::launch_step_gemv(dev->stream, w->ptr, (int)rows, (int)cols, x->ptr, out->ptr));
     else
-        TH_HIP(th::launch_matmul(dev->stream, out->ptr, w->ptr, rows, cols, x->ptr, n, dev->few_part,
-                                 th::kFewPartFloats));
+        TH_HIP(th::launch_matmul(dev->stream, out->ptr, w->ptr, rows, cols, x->ptr, n, dev->part));
     return TH_OK;
 }
 
@@ -520,10 +519,11 @@ int th_qkv_rope_append(th_device *dev, th_buffer *q, th_buffer *k, th_buffer *v,
         const int rows[3] = {(int)qd, (int)kvd, (int)kvd};
         float *const out[3] = {q->ptr, k->ptr, v->ptr};
         TH_HIP(th::launch_step_gemv3(dev->stream, w, rows, (int)H, xb->ptr, out));
-    } else if (n >= th::kGemmMinTokens && th::gemm_supported(qd, H) && th::gemm_supported(kvd, H)) {
+    } else if (n >= th::kGemmMinTokens && th::gemm_supported(qd, H) && th::gemm_supported(kvd, H) &&
+               !th::few_preferred(n, qd + 2 * kvd, H, 3)) {
         TH_NOT_CAPTURING(dev, "a projection of 16 or more tokens (stream-ordered scratch)");
         const th::GemmOut o[3] = {{wq->ptr, qd, q->ptr}, {wk->ptr, kvd, k->ptr}, {wv->ptr, kvd, v->ptr}};
-        TH_HIP(th::launch_gemm_outs(dev->stream, xb->ptr, n, H, o, 3));
+        TH_HIP(th::launch_gemm_outs(dev->stream, xb->ptr, n, H, o, 3, dev->part));
     } else if (n > 1 && th::few_supported(n, qd, H)) {
         if (n >= th::kGemmMinTokens) TH_NOT_CAPTURING(dev, "a projection of 16 or more tokens (stream-ordered scratch)");
         const th::GemmOut o[3] = {{wq->ptr, qd, q->ptr}, {wk->ptr, kvd, k->ptr}, {wv->ptr, kvd, v->ptr}};
@@ -572,10 +572,10 @@ int th_gate_up_silu(th_device *dev, th_buffer *gate, th_buffer *up, const th_wei
         TH_HIP(th::launch_step_silu(dev->stream, w_gate->ptr, w_up->ptr, (int)I, (int)H, xb->ptr, gate->ptr));
         return TH_OK;
     }
-    if (n >= th::kGemmMinTokens && th::gemm_supported(I, H)) {
+    if (n >= th::kGemmMinTokens && th::gemm_supported(I, H) && !th::few_preferred(n, 2 * I, H, 2)) {
         TH_NOT_CAPTURING(dev, "a projection of 16 or more tokens (stream-ordered scratch)");
         const th::GemmOut o[2] = {{w_gate->ptr, I, gate->ptr}, {w_up->ptr, I, up->ptr}};
-        TH_HIP(th::launch_gemm_outs(dev->stream, xb->ptr, n, H, o, 2));
+        TH_HIP(th::launch_gemm_outs(dev->stream, xb->ptr, n, H, o, 2, dev->part));
     } else if (n > 1 && th::few_supported(n, I, H)) {
         if (n >= th::kGemmMinTokens) TH_NOT_CAPTURING(dev, "a projection of 16 or more tokens (stream-ordered scratch)");
         // Both projections and silu(gate) * up in one launch; up unused.

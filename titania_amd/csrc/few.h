@@ -10,9 +10,8 @@
 
 namespace th {
 
-// Partials of up to 15 tokens in four parts, up to 8192 rows (more rows do
-// not split: few_ksplit).
-constexpr size_t kFewPartFloats = (size_t)4 * 15 * 8192;
+// Most parts few_ksplit asks for.
+constexpr int kFewMaxSplitK = 4;
 
 // Whether launch_few takes rows of `cols` columns for n tokens: whole 16-byte
 // chunks, and offsets that fit its buffer descriptors.
@@ -25,8 +24,12 @@ hipError_t launch_few(hipStream_t s, const float *x, size_t n, size_t cols, cons
                       float *part, int ksplit);
 
 // Ways launch_few's caller should split K for one [rows, cols] matrix, when
-// the consumer sums the partials (1: no split), at most kGemmMaxSplitK.
+// the consumer sums the partials (1: no split), at most kFewMaxSplitK.
 int few_ksplit(size_t n, size_t rows, size_t cols);
+
+// Whether launch_few (and launch_few_silu) is the faster one for 1-3 matrices
+// of `rows` rows in all that the GEMM would take too.
+bool few_preferred(size_t n, size_t rows, size_t cols, int n_outs);
 
 // h[t * inter + j] = silu(gate[j] . x[t]) * (up[j] . x[t]) (model/cpu.rs:151-155).
 hipError_t launch_few_silu(hipStream_t s, const float *x, size_t n, size_t cols, const uint16_t *gate,

@@ -266,14 +266,26 @@ int few_ksplit(size_t n, size_t rows, size_t cols) {
     // 4096 17.7 / 10.1 / 8.6, 2560 x 9728 31.5 / 32.3 / 16.6).
     const size_t tiles = (rows + 15) / 16 * ((n + kTokens - 1) / kTokens), steps = (cols + 31) / 32;
     int k = 1;
-    while (k < kGemmMaxSplitK && tiles * k < 512 && steps / (2 * k) >= 16) k *= 2;
+    while (k < kFewMaxSplitK && tiles * k < 512 && steps / (2 * k) >= 16) k *= 2;
     return k;
+}
+
+bool few_preferred(size_t n, size_t rows, size_t cols, int n_outs) {
+    if (n < kGemmMinTokens) return true;
+    if (n > 64) return false;
+    // The GEMM splits the K of a single matrix, this kernel reads each weight
+    // once for every 16 tokens. Calls of 16 / 36 / 64 tokens: x 4096 x 1024
+    // 6.1 / 8.2 / 9.0 us against the GEMM's 10.3 unsplit (8.4 in four parts
+    // with their sum); x 6144 x 2560, 64 tokens, 21.9 against 23.9; but x 2560
+    // x 9728, 32 tokens, 22.8 against 17, and x 19456 x 2560, 64 tokens, 53
+    // against 45.
+    return n_outs == 1 ? cols <= 1024 : rows * cols <= ((size_t)32 << 20) || n <= 32;
 }
 
 hipError_t launch_few(hipStream_t s, const float *x, size_t n, size_t cols, const GemmOut *outs, int n_outs,
                       float *part, int ksplit) {
     if (n == 0) return hipSuccess;
-    if (n_outs < 1 || n_outs > 3 || ksplit < 1 || ksplit > kGemmMaxSplitK || (ksplit > 1 && (n_outs != 1 || !part)) ||
+    if (n_outs < 1 || n_outs > 3 || ksplit < 1 || ksplit > kFewMaxSplitK || (ksplit > 1 && (n_outs != 1 || !part)) ||
         (size_t)ksplit > (cols + 31) / 32 || (uintptr_t)x % 16)
         return hipErrorInvalidValue;
     Args a{};

@@ -16,9 +16,14 @@ constexpr size_t kGemmMinTokens = 16;
 // Whether launch_gemm handles a [rows, cols] weight.
 bool gemm_supported(size_t rows, size_t cols);
 
-// out[t*rows + r] = w[r] . x[t] for t < n, on the matrix cores.
+// Most floats of split-K partials that launch_gemm_outs takes in scratch of
+// the caller's: a small-tile launch is at most 512 tiles of 64 x 64.
+constexpr size_t kPartFloats = (size_t)512 * 64 * 64;
+
+// out[t*rows + r] = w[r] . x[t] for t < n, on the matrix cores, with its
+// partials in part (kPartFloats long) where they fit.
 hipError_t launch_gemm(hipStream_t s, float *out, const uint16_t *w, size_t rows, size_t cols, const float *x,
-                       size_t n);
+                       size_t n, float *part);
 
 // One weight matrix of a multi-matrix GEMM: out[t*rows + r] = w[r] . x[t].
 struct GemmOut {
@@ -28,12 +33,14 @@ struct GemmOut {
 };
 
 // launch_gemm for 1-3 matrices that share x (one GEMM launch over all their
-// rows), with its scratch in stream-ordered memory for the call.
-hipError_t launch_gemm_outs(hipStream_t s, const float *x, size_t n, size_t cols, const GemmOut *outs, int n_outs);
+// rows). Launches of the larger tiles keep their split activations in
+// stream-ordered memory for the call.
+hipError_t launch_gemm_outs(hipStream_t s, const float *x, size_t n, size_t cols, const GemmOut *outs, int n_outs,
+                            float *part);
 
 // Most ways a single-matrix GEMM splits its K range (into partial tiles that a
 // second kernel sums in a fixed order).
-constexpr int kGemmMaxSplitK = 4;
+constexpr int kGemmMaxSplitK = 16;
 
 // split_bf16 of x [n][cols] into hi[n * cols], lo[n * cols].
 hipError_t launch_gemm_split(hipStream_t s, const float *x, size_t n, size_t cols, uint16_t *hi, uint16_t *lo);

@@ -610,6 +610,102 @@ __global__ __launch_bounds__(Huge::NT, 1) void gemm_qkv_huge_kernel(const uint16
     gemm_tile<Huge, kQkvHeads, KV>(ty, sg, hi, lo, n, cols, nullptr, 1, PairTile{}, HeadTile{&a, role, local / 128});
 }
 
+// The small tile on f32 activations: they are staged as they are (the bytes of
+// their hi and lo terms), and each fragment is split on its way to the matrix
+// cores, with the same terms, so that a caller with f32 activations needs no
+// launch before this one to split them.
+struct alignas(16) F32Stage {
+    uint4 x[Small::BM * 16];  // [64 tokens][64 columns], 16-byte chunks XOR-swizzled by the row
+    uint4 w[Small::TB];
+};
+
+// Eight waves of 16 tokens x 64 rows, four for each half of a stage's columns
+// (their sums meet in LDS at the end): a block alone on its CU then has two
+// waves a SIMD, one of which splits while the other multiplies. 64 tokens x
+// 2560 x 9728 with the sum of its parts, from HBM: 23.7 us; four waves of 16 x
+// 64 33.4, of 32 x 32 (each fragment split twice) 34.1.
+constexpr int kF32Threads = 512;
+__global__ __launch_bounds__(kF32Threads, 2) void gemm_f32_kernel(int gxy, int rows0, const uint16_t *__restrict__ w0,
+                                                                  float *__restrict__ out0,
+                                                                  const float *__restrict__ x, int n, int cols,
+                                                                  int ksplit, float *__restrict__ part, Segs segs) {
+    using T = Small;
+    constexpr int FN = T::BN / 16, kStages = T::kStages;
+    static_assert(kF32Threads == 64 * 2 * (T::BM / 16) && T::BK == 64, "a wave for 16 tokens and half a stage");
+    constexpr int XI = T::BM * 16 / kF32Threads, WI = T::TB / kF32Threads;  // loads a lane, of each
+    __shared__ F32Stage ring[kStages];
+    int tx, ty;
+    tile_of_block<8>(tx, ty, gxy & 0xffff, gxy >> 16);
+    const SegTile sg = seg_tile(w0, out0, rows0, segs, tx * T::BN);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, t0 = ty * T::BM;
+    const int wm = (wave & 3) * 16, half = wave >> 2;
+    const int fr = lane & 15, fq = lane >> 4;
+    const int nk_all = cols / T::BK, z = blockIdx.z;
+    const int kb = (int)((long long)z * nk_all / ksplit), nk = (int)((long long)(z + 1) * nk_all / ksplit) - kb;
+    const uint16_t *w = sg.w + (size_t)sg.local * cols + (size_t)kb * T::BK;
+    const float *xk = x + (size_t)kb * T::BK;
+    // Token rows past n read row n - 1 (their results are never stored).
+    auto issue = [&](F32Stage &st, int k0) {
+#pragma unroll
+        for (int i = 0; i < XI; ++i) {
+            const int span = wave * XI + i, p = span * 64 + lane, row = p / 16, pc = p % 16;
+            dma16(xk + (size_t)min(t0 + row, n - 1) * cols + k0 + (pc ^ (row & 15)) * 4, st.x + span * 64);
+        }
+#pragma unroll
+        for (int i = 0; i < WI; ++i) {
+            const int span = wave * WI + i, p = span * 64 + lane, row = p / T::CH, pc = p % T::CH;
+            dma16(w + (size_t)row * cols + k0 + (pc ^ swz<T::CH>(row)) * 8, st.w + span * 64);
+        }
+    };
+    f32x4 acc[FN];
+#pragma unroll
+    for (int q = 0; q < FN; ++q) acc[q] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < kStages - 1; ++s)
+        if (s < nk) issue(ring[s], s * T::BK);
+    const int row = wm + fr, lc = half * 4 + fq;
+    for (int k = 0; k < nk; ++k) {
+        if (k + kStages - 2 < nk) wait_vm<(kStages - 2) * (XI + WI)>();
+        else wait_vm<0>();
+        stage_barrier();
+        const F32Stage &st = ring[k % kStages];
+        const uint4 x0 = st.x[row * 16 + ((2 * lc) ^ (row & 15))], x1 = st.x[row * 16 + ((2 * lc + 1) ^ (row & 15))];
+        bf16x8 b[FN];
+#pragma unroll
+        for (int q = 0; q < FN; ++q) b[q] = frag<T::CH>(st.w, q * 16 + fr, lc);
+        if (k + kStages - 1 < nk) issue(ring[(k + kStages - 1) % kStages], (k + kStages - 1) * T::BK);
+        uint2 h0, l0, h1, l1;
+        split_bf16x4(__builtin_bit_cast(float4, x0), h0, l0);
+        split_bf16x4(__builtin_bit_cast(float4, x1), h1, l1);
+        const bf16x8 ah = __builtin_bit_cast(bf16x8, make_uint4(h0.x, h0.y, h1.x, h1.y));
+        const bf16x8 al = __builtin_bit_cast(bf16x8, make_uint4(l0.x, l0.y, l1.x, l1.y));
+#pragma unroll
+        for (int q = 0; q < FN; ++q) acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, b[q], acc[q], 0, 0, 0);
+#pragma unroll
+        for (int q = 0; q < FN; ++q) acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, b[q], acc[q], 0, 0, 0);
+    }
+    // The second half's sums, through the ring (free once every wave is here).
+    f32x4(*ep)[FN][64] = reinterpret_cast<f32x4(*)[FN][64]>(&ring[0]);
+    static_assert(sizeof(ring) >= sizeof(f32x4) * (T::BM / 16) * FN * 64, "the sums fit the ring");
+    __syncthreads();
+    if (half == 1)
+#pragma unroll
+        for (int q = 0; q < FN; ++q) ep[wave & 3][q][lane] = acc[q];
+    __syncthreads();
+    if (half == 1) return;
+    const int rows = sg.rows;
+    float *out = ksplit > 1 ? part + (size_t)z * n * rows : sg.out;
+#pragma unroll
+    for (int q = 0; q < FN; ++q) {
+        const f32x4 s = acc[q] + ep[wave][q][lane];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int t = t0 + wm + fq * 4 + i;
+            if (t < n) out[(size_t)t * rows + sg.local + q * 16 + fr] = s[i];
+        }
+    }
+}
+
 // split_bf16 of 4 elements a thread.
 __global__ void split_kernel(const float4 *__restrict__ x, uint2 *__restrict__ hi, uint2 *__restrict__ lo, size_t n4) {
     const size_t stride = (size_t)gridDim.x * blockDim.x;
@@ -621,6 +717,7 @@ __global__ void splitk_sum_kernel(const float4 *__restrict__ part, float4 *__res
     const size_t stride = (size_t)gridDim.x * blockDim.x;
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < m4; i += stride) {
         float4 acc = part[i];
+#pragma unroll 4
         for (int z = 1; z < ksplit; ++z) {
             const float4 v = part[(size_t)z * m4 + i];
             acc.x += v.x;
@@ -679,17 +776,39 @@ Plan gemm_plan(size_t n, size_t rows, size_t cols, int n_outs, bool rows_large, 
     if (n_outs == 1 && lt >= kLargeSplitMinTiles && nk >= 96) return {true, false, 2};
     if (n_outs != 1) return {false, false, 1};
     // Small tiles: a single matrix with few row tiles (o, down) splits K so
-    // that the launch still fills the chip, keeping at least 4 K steps a split.
+    // that the launch fills the chip in whole rounds (up to 64 tiles: a block
+    // a CU; past them two), keeping at least 4 K steps a split. The GEMM alone
+    // in 1 / 2 / 4 / 6 / 8 / 12 / 16 parts: 64 tokens x 1024 x 3072 (16 tiles)
+    // 25.4 / 14.3 / 8.8 / 6.9 / 6.1 / 5.3 / 5.1 us, x 2560 x 9728 (40 tiles)
+    // 75.0 / 39.8 / 22.9 / 17.4 / 21.9 / 17.6 / 19.9; 128 tokens x 2560 x 9728
+    // in 4 / 6 / 8: 36.6 / 27.4 / 30.3; 512 x 1024 x 3072 in 2 / 4 / 6: 15.0 /
+    // 13.8 / 16.2.
     const size_t tiles = (rows / Small::BN) * ((n + Small::BM - 1) / Small::BM);
-    int ksplit = 1;
-    while (ksplit < kGemmMaxSplitK && tiles * ksplit < 512 && (size_t)ksplit * 2 * 4 <= nk) ksplit *= 2;
-    return {false, false, ksplit};
+    const size_t most = std::min<size_t>(kGemmMaxSplitK, std::max<size_t>(nk / 4, 1));
+    const size_t fill = (tiles <= 64 ? 256 : 512) / std::max<size_t>(tiles, 1);
+    return {false, false, (int)std::max<size_t>(std::min(fill, most), 1)};
+}
+
+// Whether the plan for these matrices is the small tile.
+bool small_plan(size_t n, size_t cols, const GemmOut *outs, int n_outs, int *ksplit) {
+    size_t total = 0;
+    bool rows_large = true, rows_huge = true;
+    for (int i = 0; i < n_outs; ++i) {
+        total += outs[i].rows;
+        rows_large = rows_large && outs[i].rows % Large::BN == 0;
+        rows_huge = rows_huge && outs[i].rows % Huge::BN == 0;
+    }
+    const Plan plan = gemm_plan(n, total, cols, n_outs, rows_large, rows_huge);
+    *ksplit = plan.ksplit;
+    return !plan.large && !plan.huge;
 }
 
 }  // namespace
 
 size_t gemm_scratch_bytes(size_t n, size_t cols, size_t rows) {
-    return n * cols * 2 * sizeof(uint16_t) + (size_t)kGemmMaxSplitK * n * rows * sizeof(float);
+    // The larger tiles split K in two at most, the small one into at most 512
+    // tiles in all.
+    return n * cols * 2 * sizeof(uint16_t) + std::max(2 * n * rows, kPartFloats) * sizeof(float);
 }
 
 hipError_t launch_gemm_split(hipStream_t s, const float *x, size_t n, size_t cols, uint16_t *hi, uint16_t *lo) {
@@ -857,13 +976,37 @@ hipError_t launch_gemm_multi(hipStream_t s, const float *x, size_t n, size_t col
     return launch_splitk_sum(s, part, outs[0].out, n * total, ksplit);
 }
 
-hipError_t launch_gemm_outs(hipStream_t s, const float *x, size_t n, size_t cols, const GemmOut *outs, int n_outs) {
+hipError_t launch_gemm_outs(hipStream_t s, const float *x, size_t n, size_t cols, const GemmOut *outs, int n_outs,
+                            float *part) {
     if (n == 0) return hipSuccess;
-    if (n_outs < 1 || n_outs > 3) return hipErrorInvalidValue;
-    size_t most = 0;
+    if (n_outs < 1 || n_outs > 3 || (uintptr_t)x % 16) return hipErrorInvalidValue;
+    size_t most = 0, total = 0;
     for (int i = 0; i < n_outs; ++i) {
         if (!gemm_supported(outs[i].rows, cols)) return hipErrorInvalidValue;
         most = std::max(most, outs[i].rows);
+        total += outs[i].rows;
+    }
+    // Small tiles take the f32 activations as they are, with partials in the
+    // caller's scratch: 64 tokens x 2560 x 9728, 29.6 -> 17.5 us a call (the
+    // launch that split the activations gone, K in six parts instead of four),
+    // and where a call ran for less than its stream-ordered allocation took,
+    // x 1024 x 3072, 26.0 -> 9.0.
+    int ksplit = 1;
+    const size_t tx = total / Small::BN, ty = (n + Small::BM - 1) / Small::BM;
+    if (small_plan(n, cols, outs, n_outs, &ksplit) && tx <= 0xffff && ty <= 0xffff && n <= ((size_t)1 << 24) &&
+        (ksplit == 1 || (part && (size_t)ksplit * n * total <= kPartFloats))) {
+        Segs sg{};
+        for (int i = 0; i < n_outs; ++i) {
+            sg.w[i] = outs[i].w;
+            sg.out[i] = outs[i].out;
+            sg.rows[i] = (int)outs[i].rows;
+        }
+        sg.n = n_outs;
+        const dim3 grid((unsigned)tx, (unsigned)ty, (unsigned)ksplit);
+        gemm_f32_kernel<<<grid, kF32Threads, 0, s>>>((int)(tx | ty << 16), sg.rows[0], sg.w[0], sg.out[0], x, (int)n,
+                                                   (int)cols, ksplit, part, sg);
+        const hipError_t e = hipGetLastError();
+        return e != hipSuccess || ksplit == 1 ? e : launch_splitk_sum(s, part, outs[0].out, n * total, ksplit);
     }
     void *scratch = nullptr;
     const size_t bytes = gemm_scratch_bytes(n, cols, most);
@@ -875,18 +1018,10 @@ hipError_t launch_gemm_outs(hipStream_t s, const float *x, size_t n, size_t cols
 }
 
 hipError_t launch_gemm(hipStream_t s, float *out, const uint16_t *w, size_t rows, size_t cols, const float *x,
-                       size_t n) {
+                       size_t n, float *part) {
     if (n == 0 || rows == 0) return hipSuccess;
-    if (!gemm_supported(rows, cols)) return hipErrorInvalidValue;
-    // The split activations live in stream-ordered scratch for this call.
-    void *scratch = nullptr;
-    const size_t bytes = gemm_scratch_bytes(n, cols, rows);
-    hipError_t e = hipMallocAsync(&scratch, bytes, s);
-    if (e != hipSuccess) return e;
     const GemmOut o{w, rows, out};
-    e = launch_gemm_multi(s, x, n, cols, &o, 1, scratch, bytes);
-    const hipError_t f = hipFreeAsync(scratch, s);
-    return e != hipSuccess ? e : f;
+    return launch_gemm_outs(s, x, n, cols, &o, 1, part);
 }
 
 }  // namespace th

@@ -95,13 +95,14 @@ static hipError_t gemv(hipStream_t s, float *out, const uint16_t *w, size_t rows
 }
 
 hipError_t launch_matmul(hipStream_t s, float *out, const uint16_t *w, size_t rows, size_t cols, const float *x,
-                         size_t n, float *part, size_t part_floats) {
+                         size_t n, float *part) {
     if (n == 0 || rows == 0) return hipSuccess;
     if (cols % 8 != 0) {
         gemv_scalar_kernel<<<dim3((unsigned)((rows + 3) / 4)), 256, 0, s>>>(out, w, rows, cols, x, n);
         return hipGetLastError();
     }
-    if (n >= kGemmMinTokens && gemm_supported(rows, cols)) return launch_gemm(s, out, w, rows, cols, x, n);
+    if (n >= kGemmMinTokens && gemm_supported(rows, cols) && !few_preferred(n, rows, cols, 1))
+        return launch_gemm(s, out, w, rows, cols, x, n, part);
     if (n == 1) {
         // Enough waves to cover the chip (256 CUs x 4 SIMDs) before packing rows.
         if (rows >= 16384) return gemv<4, 1>(s, out, w, rows, cols, x, 1, rows);
@@ -121,7 +122,7 @@ hipError_t launch_matmul(hipStream_t s, float *out, const uint16_t *w, size_t ro
         return hipSuccess;
     }
     int ksplit = n < kGemmMinTokens ? few_ksplit(n, rows, cols) : 1;
-    if (!part || n * rows % 4 || (size_t)ksplit * n * rows > part_floats) ksplit = 1;
+    if (!part || n * rows % 4 || (size_t)ksplit * n * rows > kPartFloats) ksplit = 1;
     const GemmOut o{w, rows, out};
     const hipError_t e = launch_few(s, x, n, cols, &o, 1, part, ksplit);
     if (e != hipSuccess || ksplit == 1) return e;

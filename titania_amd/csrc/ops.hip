@@ -201,6 +201,86 @@ __global__ __launch_bounds__(256) void add_rmsnorm_kernel(float *__restrict__ ax
     }
 }
 
+// The same with a block of four waves a row, for launches of few rows (and
+// rows that are not whole 256-element spans): bound by its round trips, so
+// every load of a row is in flight at once, NV float4 a lane and four
+// partials at a time. Rows of dim <= 1024 NV elements, whole float4.
+template <int NV>
+__global__ __launch_bounds__(256) void add_rmsnorm_row_kernel(float *__restrict__ ax, const float *__restrict__ ay,
+                                                              const uint16_t *__restrict__ aw, size_t adim,
+                                                              size_t ay_stride, int any, NormArgs a) {
+    __shared__ float red[4];
+    const size_t base = (size_t)blockIdx.x * (adim / 4);
+    const int n4 = (int)(adim / 4), tid = threadIdx.x;
+    float4 *xr = reinterpret_cast<float4 *>(ax) + base;
+    const float4 *yr = reinterpret_cast<const float4 *>(ay) + base;
+    float4 v[NV], u[NV];
+    uint2 g[NV];
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+        const int i = tid + 256 * k;
+        v[k] = u[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+        g[k] = make_uint2(0u, 0u);
+        if (i < n4) {
+            v[k] = xr[i];
+            if (any) u[k] = yr[i];
+            g[k] = reinterpret_cast<const uint2 *>(aw)[i];
+        }
+    }
+    for (int z0 = 1; z0 < any; z0 += 4) {
+        float4 t[4][NV];
+#pragma unroll
+        for (int z = 0; z < 4; ++z)
+#pragma unroll
+            for (int k = 0; k < NV; ++k) {
+                const int i = tid + 256 * k;
+                if (z0 + z < any && i < n4) t[z][k] = yr[(size_t)(z0 + z) * (ay_stride / 4) + i];
+            }
+#pragma unroll
+        for (int z = 0; z < 4; ++z)
+            if (z0 + z < any)
+#pragma unroll
+                for (int k = 0; k < NV; ++k)
+                    if (tid + 256 * k < n4) {
+                        u[k].x += t[z][k].x;
+                        u[k].y += t[z][k].y;
+                        u[k].z += t[z][k].z;
+                        u[k].w += t[z][k].w;
+                    }
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+        if (any && tid + 256 * k < n4) {
+            v[k].x = v[k].x + u[k].x;
+            v[k].y = v[k].y + u[k].y;
+            v[k].z = v[k].z + u[k].z;
+            v[k].w = v[k].w + u[k].w;
+            xr[tid + 256 * k] = v[k];
+        }
+        ss += v[k].x * v[k].x + v[k].y * v[k].y + v[k].z * v[k].z + v[k].w * v[k].w;
+    }
+    ss = wave_sum_dpp(ss);
+    if ((tid & 63) == 0) red[tid >> 6] = ss;
+    __syncthreads();
+    const float scale = 1.0f / sqrtf(((red[0] + red[1]) + (red[2] + red[3])) / (float)adim + a.eps);
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+        const int i = tid + 256 * k;
+        if (i >= n4) continue;
+        float4 o;
+        o.x = v[k].x * (scale * bf16_lo(g[k].x));
+        o.y = v[k].y * (scale * bf16_hi(g[k].x));
+        o.z = v[k].z * (scale * bf16_lo(g[k].y));
+        o.w = v[k].w * (scale * bf16_hi(g[k].y));
+        if (a.xb) reinterpret_cast<float4 *>(a.xb)[base + i] = o;
+        if (a.hi) split_bf16x4(o, reinterpret_cast<uint2 *>(a.hi)[base + i], reinterpret_cast<uint2 *>(a.lo)[base + i]);
+    }
+}
+
+// Rows up to which a launch takes a block a row.
+constexpr size_t kNormRowBlocks = 1024;
+
 hipError_t launch_add_rmsnorm_parts(hipStream_t s, float *x, const float *y, int ny, size_t y_stride, float *xb,
                                     uint16_t *hi, uint16_t *lo, size_t rows, const uint16_t *w, size_t dim,
                                     float eps) {
@@ -213,6 +293,20 @@ hipError_t launch_add_rmsnorm_parts(hipStream_t s, float *x, const float *y, int
     const bool vec = dim % 256 == 0 && y_stride % 4 == 0 &&
                      ((uintptr_t)x | (uintptr_t)xb | (uintptr_t)a.y | (uintptr_t)w) % 16 == 0 &&
                      ((uintptr_t)hi | (uintptr_t)lo) % 8 == 0;
+    const bool vec4 = dim % 4 == 0 && y_stride % 4 == 0 && ((uintptr_t)x | (uintptr_t)xb | (uintptr_t)a.y) % 16 == 0 &&
+                      ((uintptr_t)hi | (uintptr_t)lo | (uintptr_t)w) % 8 == 0;
+    if (vec4 && dim > 256 && dim <= 4096 && rows < ((size_t)1 << 31) && (rows <= kNormRowBlocks || !vec)) {
+        const dim3 rgrid((unsigned)rows);
+        if (dim <= 1024)
+            add_rmsnorm_row_kernel<1><<<rgrid, block, 0, s>>>(a.x, a.y, a.w, a.dim, a.y_stride, a.ny, a);
+        else if (dim <= 2048)
+            add_rmsnorm_row_kernel<2><<<rgrid, block, 0, s>>>(a.x, a.y, a.w, a.dim, a.y_stride, a.ny, a);
+        else if (dim <= 3072)
+            add_rmsnorm_row_kernel<3><<<rgrid, block, 0, s>>>(a.x, a.y, a.w, a.dim, a.y_stride, a.ny, a);
+        else
+            add_rmsnorm_row_kernel<4><<<rgrid, block, 0, s>>>(a.x, a.y, a.w, a.dim, a.y_stride, a.ny, a);
+        return hipGetLastError();
+    }
     switch (vec ? dim / 256 : 0) {
     case 1: add_rmsnorm_kernel<1><<<grid, block, 0, s>>>(a.x, a.y, a.w, a.rows, a.dim, a.y_stride, a.ny, a); break;
     case 2: add_rmsnorm_kernel<2><<<grid, block, 0, s>>>(a.x, a.y, a.w, a.rows, a.dim, a.y_stride, a.ny, a); break;
