@@ -430,7 +430,8 @@ def test_gemm_silu(hip, tlib, H, I, n):
     assert np.all(err <= bound), f"silu(gate) * up {shape} n={n}: worst {np.max(err / bound):.2f} of the bound"
 
 
-@pytest.mark.parametrize("dim,rows,n_parts", [(1024, 100, 0), (1024, 100, 1), (1024, 64, 3), (2560, 40, 2)])
+@pytest.mark.parametrize("dim,rows,n_parts", [(1024, 100, 0), (1024, 100, 1), (1024, 64, 3), (2560, 40, 2), (1024, 33, 5),
+                                              (512, 7, 16), (2560, 1030, 2)])
 def test_add_rmsnorm_parts(hip, tlib, dim, rows, n_parts):
     g, G = gains(hip, dim, 8, "g")
     rng = np.random.default_rng(dim + rows + n_parts)

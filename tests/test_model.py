@@ -15,7 +15,7 @@ import numpy as np
 import pytest
 
 from oracle import ref
-from titania_amd import (QWEN3_0_6B, QWEN3_TINY, TH_KV_BF16, TH_KV_F32, TH_PATH_FUSED, TH_PATH_OPS, TH_PATH_TRAIT,
+from titania_amd import (InvalidArgument, QWEN3_0_6B, QWEN3_TINY, TH_KV_BF16, TH_KV_F32, TH_PATH_FUSED, TH_PATH_OPS, TH_PATH_TRAIT,
                          Sampler)
 from titania_amd.config import Config
 from titania_amd import synth
@@ -286,6 +286,30 @@ def test_tiny8_decode_crossing(tiny8, decode_mode, n, steps, max_len, kv):
         assert float(np.std(exp)) > 0.05
         assert float(np.max(np.abs(logits[i] - exp))) <= tol, f"step {i} (position {n + i})"
     st.close()
+
+
+@pytest.mark.parametrize("n,steps,max_len,kv", [(5, 6, 11, TH_KV_F32), (1018, 10, 1037, TH_KV_F32),
+                                                (2043, 8, 2070, TH_KV_BF16)])
+def test_tiny8_forward_one_token(tiny8, monkeypatch, n, steps, max_len, kv):
+    """A forward of one token runs a decode step's kernels: fed the tokens of a
+    decode, it returns the decode's logits bit for bit, through the chunked
+    launch, the streaming one and the step between them, with a decode call in
+    the middle and one that follows picking from the logits it left."""
+    monkeypatch.setenv("TITANIA_DECODE", "eager")  # chooses the launch step by step, as the forward does
+    m, _ = tiny8
+    prompt = synth.prompt(n, QWEN3_TINY8.vocab_size, seed=n)
+    a, b = State(m, max_len, kv), State(m, max_len, kv)
+    m.forward(a, prompt, 0, TH_PATH_FUSED, want_logits=False)
+    m.forward(b, prompt, 0, TH_PATH_FUSED, want_logits=False)
+    toks, logits = m.decode(a, n, steps, keep_logits=True)
+    for i in range(steps - 2):
+        assert np.array_equal(m.forward(b, [int(toks[i])], n + i, TH_PATH_FUSED), logits[i]), f"step {i}"
+    assert list(m.decode(b, n + steps - 2, 1)) == [toks[steps - 2]]
+    assert np.array_equal(m.forward(b, [int(toks[-1])], n + steps - 1, TH_PATH_FUSED), logits[-1])
+    with pytest.raises(InvalidArgument, match="vocabulary"):
+        m.forward(b, [QWEN3_TINY8.vocab_size], 0, TH_PATH_FUSED)
+    a.close()
+    b.close()
 
 
 def _long_context_check(model, cfg, n_prompt, steps, kv, tol, seed):

@@ -32,6 +32,9 @@ struct th_device {
     uint32_t *token_out = nullptr;
     // th_timer_begin / th_timer_end.
     hipEvent_t ev_begin = nullptr, ev_end = nullptr;
+    // Pinned host memory of kPinnedFloats for the results of calls that wait
+    // (th::read_back), then kPinnedTokens token ids for the next launch.
+    float *pinned = nullptr;
     // Between th_graph_begin and th_graph_end: the stream is being captured.
     bool capturing = false;
 };
@@ -58,6 +61,14 @@ namespace th {
 // Records a printf-style message as the calling thread's last error and returns `code`.
 int fail(int code, const char *fmt, ...) __attribute__((format(printf, 2, 3)));
 void clear_error();
+
+// Floats and token ids that a device's pinned memory holds.
+constexpr size_t kPinnedFloats = (size_t)1 << 18, kPinnedTokens = 256;
+
+// Waits for the stream and copies `len` floats out, and *word (device memory;
+// may be null) to *word_out.
+int read_back(th_device *dev, const float *src, size_t len, float *out, const unsigned *word = nullptr,
+              unsigned *word_out = nullptr);
 
 // Makes sure the device scratch holds at least `bytes`; returns its pointer or null.
 void *scratch(th_device *dev, size_t bytes);
@@ -102,6 +113,9 @@ namespace th {
 hipError_t launch_embed(hipStream_t s, float *out, const uint16_t *table, size_t dim, const uint32_t *tokens,
                         size_t n);
 hipError_t launch_copy(hipStream_t s, float *dst, const float *src, size_t len);
+// dst[i] = src[i] for i < len and, if word is not null, dst[len] = *word, in
+// host memory that the device can write (both 16-byte aligned).
+hipError_t launch_copy_out(hipStream_t s, float *dst, const float *src, size_t len, const unsigned *word);
 hipError_t launch_add(hipStream_t s, float *x, const float *y, size_t len);
 hipError_t launch_silu_mul(hipStream_t s, float *gate, const float *up, size_t len);
 // silu(gate) * up as split_bf16 terms hi/lo (len a multiple of 4).

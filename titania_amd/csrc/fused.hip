@@ -109,6 +109,23 @@ __global__ __launch_bounds__(1024) void pick_kernel(const uint64_t *__restrict__
     write_embedding(emb, picked);
 }
 
+__global__ __launch_bounds__(256) void step_begin_kernel(StepState *st, long long pos, uint32_t epoch, uint32_t token,
+                                                         PickEmbed emb) {
+    if (threadIdx.x == 0) {
+        st->pos = pos;
+        st->epoch = epoch;
+        st->token = token;
+    }
+    write_embedding(emb, token);
+}
+
+hipError_t launch_step_begin(hipStream_t s, StepState *st, long long pos, uint32_t epoch, uint32_t token,
+                             const PickEmbed &emb) {
+    if (!emb.table || emb.dim % 8) return hipErrorInvalidValue;
+    step_begin_kernel<<<1, 256, 0, s>>>(st, pos, epoch, token, emb);
+    return hipGetLastError();
+}
+
 // Copies the logits into row `step` of the caller's logits array (the logits
 // after the token fed at this step), when the caller asked for them.
 __global__ void keep_logits_kernel(const float *__restrict__ logits, size_t vocab, const StepState *st) {

@@ -392,8 +392,9 @@ bool step_dual(const th_state *s) {
 // Queues one decode step with the fused step kernels: the token and position
 // come from s->step, the picked token goes back there. `chunked`: the q/k/v +
 // attention take the chunked launch, where the state allows it (step_chunked
-// for a short context), or else the streaming one.
-int enqueue_step(th_state *s, bool chunked) {
+// for a short context), or else the streaming one. Without `pick` it ends
+// with the logits.
+int enqueue_step(th_state *s, bool chunked, bool pick = true) {
     th_model *m = s->m;
     hipStream_t st = m->dev->stream;
     const th_config &c = m->c;
@@ -495,6 +496,7 @@ int enqueue_step(th_state *s, bool chunked) {
     int np = 0;
     TH_HIP(th::launch_step_logits(st, m->out_proj()->ptr, V, H, s->sx_b, y_prev, m->norm->ptr, eps,
                                   s->logits->ptr, s->s_part, &np));
+    if (!pick) return TH_OK;
     if (s->graph_keep) TH_HIP(th::launch_keep_logits(st, s->logits->ptr, (size_t)V, s->step));
     if (s->sampling)
         TH_HIP(th::launch_sample(st, s->logits->ptr, (size_t)V, s->s_cand, s->s_sample, s->step, 1, step_embed(s),
@@ -732,12 +734,20 @@ int enqueue_fused(th_state *s, const uint32_t *tokens, size_t n, size_t pos, con
     return TH_OK;
 }
 
-int stage_state_tokens(th_state *s, const uint32_t *tokens, size_t n) {
+int stage_state_tokens(th_state *s, const uint32_t *tokens, size_t n, const uint32_t **staged) {
     th_model *m = s->m;
     for (size_t i = 0; i < n; ++i)
         if (tokens[i] >= (uint32_t)m->c.vocab_size)
             return fail(TH_ERR_INVALID, "token %u at index %zu is past the vocabulary of %lld", tokens[i], i,
                         (long long)m->c.vocab_size);
+    if (n <= th::kPinnedTokens) {
+        // The embedding reads these from the host (the caller waits for the
+        // stream before it returns, and with it for that read).
+        uint32_t *pinned = reinterpret_cast<uint32_t *>(m->dev->pinned + th::kPinnedFloats);
+        memcpy(pinned, tokens, n * sizeof(uint32_t));
+        *staged = pinned;
+        return TH_OK;
+    }
     if (n > s->tokens_dev_cap) {
         TH_HIP(hipStreamSynchronize(m->dev->stream));
         free_dev(s->tokens_dev);
@@ -748,7 +758,34 @@ int stage_state_tokens(th_state *s, const uint32_t *tokens, size_t n) {
         s->tokens_dev_cap = cap;
     }
     TH_HIP(hipMemcpyAsync(s->tokens_dev, tokens, n * sizeof(uint32_t), hipMemcpyHostToDevice, m->dev->stream));
+    *staged = s->tokens_dev;
     return TH_OK;
+}
+
+// The outcome of a decode's or forward's step kernels (StepQkvAttnArgs::err).
+int step_status(unsigned poll_failures) {
+    if (poll_failures >= th::kStepReachError)
+        return fail(TH_ERR_HIP, "decode: a step's context passed its chunked attention launch's chunks");
+    if (poll_failures)
+        return fail(TH_ERR_HIP, "decode: %u attention blocks gave up waiting for their q/k/v", poll_failures);
+    return TH_OK;
+}
+
+// The fused forward of one token: a decode step's kernels without its pick
+// (12 Qwen3-0.6B layers, a token at position 100 with its logits read: 0.586 ->
+// 0.238 ms; the batched path's kernels took ten launches a layer). Launched one
+// by one: a first call needs no capture.
+int forward_one(th_state *s, uint32_t token, size_t pos, float *logits) {
+    th_model *m = s->m;
+    if (token >= (uint32_t)m->c.vocab_size)
+        return fail(TH_ERR_INVALID, "token %u at index 0 is past the vocabulary of %lld", token,
+                    (long long)m->c.vocab_size);
+    TH_HIP(th::launch_step_begin(m->dev->stream, s->step, (long long)pos, s->step_epoch, token, step_embed(s)));
+    s->step_epoch += 1;
+    TRY(enqueue_step(s, step_chunked(s, (long long)(pos + 1)), false));
+    unsigned poll_failures = 0;
+    TRY(th::read_back(m->dev, s->logits->ptr, logits ? s->logits->len : 0, logits, s->s_err, &poll_failures));
+    return step_status(poll_failures);
 }
 
 // The ops and trait paths share the reference's caches; the fused path keeps
@@ -1001,9 +1038,11 @@ int th_forward(th_model *m, th_state *s, const uint32_t *tokens, size_t n, size_
             TRY(forward_batch_trait(s, tokens + i, std::min(kBatch, n - i), pos + i));
     } else {
         TRY(ensure_fused_state(s));
-        TRY(stage_state_tokens(s, tokens, n));
+        if (n == 1 && s->step_fused) return forward_one(s, tokens[0], pos, logits);
+        const uint32_t *staged = nullptr;
+        TRY(stage_state_tokens(s, tokens, n, &staged));
         for (size_t i = 0; i < n; i += s->fb)
-            TRY(enqueue_fused(s, s->tokens_dev + i, std::min(s->fb, n - i), pos + i, nullptr));
+            TRY(enqueue_fused(s, staged + i, std::min(s->fb, n - i), pos + i, nullptr));
     }
     if (logits) return th_read(m->dev, s->logits, logits, s->logits->len);
     TH_HIP(hipStreamSynchronize(m->dev->stream));
@@ -1129,11 +1168,7 @@ int decode(th_model *m, th_state *s, size_t pos, size_t steps, uint32_t *out_tok
     if (s->s_err) TH_HIP(hipMemcpyAsync(&poll_failures, s->s_err, sizeof poll_failures, hipMemcpyDeviceToHost, st));
     if (sampling) TH_HIP(hipMemcpyAsync(sp, s->s_sample, sizeof *sp, hipMemcpyDeviceToHost, st));
     TH_HIP(hipStreamSynchronize(st));
-    if (poll_failures >= th::kStepReachError)
-        return fail(TH_ERR_HIP, "decode: a step's context passed its chunked attention launch's chunks");
-    if (poll_failures)
-        return fail(TH_ERR_HIP, "decode: %u attention blocks gave up waiting for their q/k/v", poll_failures);
-    return TH_OK;
+    return step_status(poll_failures);
 }
 
 }  // namespace

@@ -50,6 +50,23 @@ hipError_t launch_copy(hipStream_t s, float *dst, const float *src, size_t len) 
     return hipGetLastError();
 }
 
+__global__ void copy_out_kernel(float *__restrict__ dst, const float *__restrict__ src, size_t len,
+                                const unsigned *__restrict__ word) {
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (4 * i + 4 <= len) {
+        reinterpret_cast<float4 *>(dst)[i] = reinterpret_cast<const float4 *>(src)[i];
+    } else {
+        for (size_t k = 4 * i; k < len; ++k) dst[k] = src[k];
+    }
+    if (i == 0 && word) reinterpret_cast<unsigned *>(dst)[len] = *word;
+}
+
+hipError_t launch_copy_out(hipStream_t s, float *dst, const float *src, size_t len, const unsigned *word) {
+    if (len >= ((size_t)1 << 31) || ((uintptr_t)dst | (uintptr_t)src) % 16) return hipErrorInvalidValue;
+    copy_out_kernel<<<(unsigned)((len / 4 + 256) / 256), 256, 0, s>>>(dst, src, len, word);
+    return hipGetLastError();
+}
+
 __global__ void add_kernel(float *__restrict__ x, const float *__restrict__ y, size_t len) {
     size_t stride = (size_t)gridDim.x * blockDim.x;
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < len; i += stride) x[i] = x[i] + y[i];
