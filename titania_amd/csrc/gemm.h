@@ -32,6 +32,12 @@ struct GemmOut {
     float *out;
 };
 
+// The GEMM on f32 activations with the small tile, 1-3 matrices that share x:
+// with ksplit > 1 (one matrix) the partial products go to
+// part[ksplit][n][rows], to be summed by the consumer in split order.
+hipError_t launch_gemm_f32(hipStream_t s, const float *x, size_t n, size_t cols, const GemmOut *outs, int n_outs,
+                           float *part, int ksplit);
+
 // launch_gemm for 1-3 matrices that share x (one GEMM launch over all their
 // rows). Launches of the larger tiles keep their split activations in
 // stream-ordered memory for the call.

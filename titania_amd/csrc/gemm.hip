@@ -800,7 +800,8 @@ bool small_plan(size_t n, size_t cols, const GemmOut *outs, int n_outs, int *ksp
     }
     const Plan plan = gemm_plan(n, total, cols, n_outs, rows_large, rows_huge);
     *ksplit = plan.ksplit;
-    return !plan.large && !plan.huge;
+    return !plan.large && !plan.huge && total / Small::BN <= 0xffff && (n + Small::BM - 1) / Small::BM <= 0xffff &&
+           n <= ((size_t)1 << 24);
 }
 
 }  // namespace
@@ -976,6 +977,30 @@ hipError_t launch_gemm_multi(hipStream_t s, const float *x, size_t n, size_t col
     return launch_splitk_sum(s, part, outs[0].out, n * total, ksplit);
 }
 
+hipError_t launch_gemm_f32(hipStream_t s, const float *x, size_t n, size_t cols, const GemmOut *outs, int n_outs,
+                           float *part, int ksplit) {
+    if (n == 0) return hipSuccess;
+    if (n_outs < 1 || n_outs > 3 || (uintptr_t)x % 16 || ksplit < 1 || ksplit > kGemmMaxSplitK ||
+        (ksplit > 1 && (n_outs != 1 || !part)) || (size_t)ksplit > cols / BK)
+        return hipErrorInvalidValue;
+    Segs sg{};
+    size_t total = 0;
+    for (int i = 0; i < n_outs; ++i) {
+        if (!gemm_supported(outs[i].rows, cols)) return hipErrorInvalidValue;
+        sg.w[i] = outs[i].w;
+        sg.out[i] = outs[i].out;
+        sg.rows[i] = (int)outs[i].rows;
+        total += outs[i].rows;
+    }
+    sg.n = n_outs;
+    const size_t tx = total / Small::BN, ty = (n + Small::BM - 1) / Small::BM;
+    if (tx > 0xffff || ty > 0xffff || n > ((size_t)1 << 24)) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)tx, (unsigned)ty, (unsigned)ksplit);
+    gemm_f32_kernel<<<grid, kF32Threads, 0, s>>>((int)(tx | ty << 16), sg.rows[0], sg.w[0], sg.out[0], x, (int)n,
+                                               (int)cols, ksplit, part, sg);
+    return hipGetLastError();
+}
+
 hipError_t launch_gemm_outs(hipStream_t s, const float *x, size_t n, size_t cols, const GemmOut *outs, int n_outs,
                             float *part) {
     if (n == 0) return hipSuccess;
@@ -992,20 +1017,9 @@ hipError_t launch_gemm_outs(hipStream_t s, const float *x, size_t n, size_t cols
     // and where a call ran for less than its stream-ordered allocation took,
     // x 1024 x 3072, 26.0 -> 9.0.
     int ksplit = 1;
-    const size_t tx = total / Small::BN, ty = (n + Small::BM - 1) / Small::BM;
-    if (small_plan(n, cols, outs, n_outs, &ksplit) && tx <= 0xffff && ty <= 0xffff && n <= ((size_t)1 << 24) &&
+    if (small_plan(n, cols, outs, n_outs, &ksplit) &&
         (ksplit == 1 || (part && (size_t)ksplit * n * total <= kPartFloats))) {
-        Segs sg{};
-        for (int i = 0; i < n_outs; ++i) {
-            sg.w[i] = outs[i].w;
-            sg.out[i] = outs[i].out;
-            sg.rows[i] = (int)outs[i].rows;
-        }
-        sg.n = n_outs;
-        const dim3 grid((unsigned)tx, (unsigned)ty, (unsigned)ksplit);
-        gemm_f32_kernel<<<grid, kF32Threads, 0, s>>>((int)(tx | ty << 16), sg.rows[0], sg.w[0], sg.out[0], x, (int)n,
-                                                   (int)cols, ksplit, part, sg);
-        const hipError_t e = hipGetLastError();
+        const hipError_t e = launch_gemm_f32(s, x, n, cols, outs, n_outs, part, ksplit);
         return e != hipSuccess || ksplit == 1 ? e : launch_splitk_sum(s, part, outs[0].out, n * total, ksplit);
     }
     void *scratch = nullptr;

@@ -35,6 +35,13 @@ constexpr size_t kBatch = 64;          // model/model.rs:8 BATCH (the ops path)
 // scratch and attention partials, about 3 GB at the 4B shape.
 constexpr size_t kFusedBatch = 8192;
 constexpr size_t kWeightsPerLayer = 11;
+// Tokens from which the prefill attention of an f32 cache goes through the
+// bf16 planes of its keys and values: with fewer, splitting every earlier
+// position once costs more than splitting the tiles that the few token tiles
+// read (Qwen3-0.6B, us a layer at position 300: 8 / 64 / 256 tokens 62.7 /
+// 75.9 / 87.7 with the planes, 58.3 / 70.7 / 78.0 without; Qwen3-4B, position
+// 4000: 11 / 128 / 200 tokens 140.4 / 209.8 / 272.2 and 131.7 / 201.1 / 271.0).
+constexpr size_t kPlaneMinTokens = 320;
 
 struct Layer {
     const th_weight *attn_norm, *q, *k, *v, *o, *q_norm, *k_norm, *mlp_norm, *gate, *up, *down;
@@ -532,7 +539,15 @@ int enqueue_fused(th_state *s, const uint32_t *tokens, size_t n, size_t pos, con
     // produce a GEMM input (the norms, attention, silu_mul) write it as bf16
     // hi/lo terms directly, and the residual add after the o and down GEMMs
     // sums their split-K partials itself.
-    const bool hl = use_gemm(std::max(std::max(H, qd), I)) && th::gemm_supported(qd, H) &&
+    // Up to 32 tokens the few-token kernel takes q/k/v and gate/up, and the
+    // GEMM on f32 activations o and down (us a layer, GEMMs on split
+    // activations -> these: Qwen3-0.6B, 16 / 32 / 48 tokens, 54.8 / 59.3 / 61.2
+    // -> 52.4 / 55.1 / 59.5; Qwen3-4B at position 700 126.6 / 136.3 / 140.8 ->
+    // 118.7 / 134.4 / 143.7).
+    const bool few_path = n >= th::kGemmMinTokens && n <= 32 && th::few_preferred(n, qd + 2 * nkv * hd, H, 3) &&
+                          th::few_preferred(n, 2 * I, H, 2) && th::few_supported(n, qd, H) &&
+                          th::few_supported(n, I, H);
+    const bool hl = !few_path && use_gemm(std::max(std::max(H, qd), I)) && th::gemm_supported(qd, H) &&
                     th::gemm_supported(nkv * hd, H) && th::gemm_supported(H, qd) && th::gemm_supported(I, H) &&
                     th::gemm_supported(H, I);
     uint16_t *hi = static_cast<uint16_t *>(s->fsplit), *lo = hi ? hi + s->fb * s->fsplit_cols : nullptr;
@@ -562,13 +577,19 @@ int enqueue_fused(th_state *s, const uint32_t *tokens, size_t n, size_t pos, con
     };
     auto single_few = [&](const uint16_t *w, size_t cols, const float *x) -> int {
         one_residual();
-        const int ks = part && n < th::kGemmMinTokens && few(H, cols) ? th::few_ksplit(n, H, cols) : 1;
+        // 16 tokens or more: the GEMM on f32 activations, as th_matmul.
+        const bool gemm = few_path && part && th::gemm_supported(H, cols) && !th::few_preferred(n, H, cols, 1);
+        const int ks = gemm ? th::gemm_ksplit(n, H, cols, 1)
+                       : part && n < th::kGemmMinTokens && few(H, cols) ? th::few_ksplit(n, H, cols) : 1;
         const th::GemmOut o{w, H, s->fy};
-        if (ks > 1) {
-            TH_HIP(th::launch_few(st, x, n, cols, &o, 1, part, ks));
-            res = part;
-            nres = ks;
-            res_stride = n * H;
+        if (gemm || ks > 1) {
+            TH_HIP(gemm ? th::launch_gemm_f32(st, x, n, cols, &o, 1, part, ks)
+                        : th::launch_few(st, x, n, cols, &o, 1, part, ks));
+            if (ks > 1) {
+                res = part;
+                nres = ks;
+                res_stride = n * H;
+            }
         } else {
             TH_HIP(th::launch_matmul(st, s->fy, w, H, cols, x, n));
         }
@@ -621,7 +642,8 @@ int enqueue_fused(th_state *s, const uint32_t *tokens, size_t n, size_t pos, con
         // The attention through bf16 planes of the keys and values (f32
         // caches); the fused q/k/v GEMM writes the new positions' planes in
         // its epilogue.
-        const bool use_planes = s->kv_planes && th::attention_planes_supported(aa, n, hd);
+        const bool use_planes =
+            n >= kPlaneMinTokens && s->kv_planes && th::attention_planes_supported(aa, n, hd);
         bool planes_written = false;
         // Residual add of the previous layer's MLP output, then the attention norm.
         if (hl) {
@@ -658,7 +680,7 @@ int enqueue_fused(th_state *s, const uint32_t *tokens, size_t n, size_t pos, con
         } else {
             TH_HIP(th::launch_add_rmsnorm_parts(st, s->fx, res, nres, res_stride, s->fxb, nullptr, nullptr, n,
                                                 L.attn_norm->ptr, H, eps));
-            if (use_gemm(H) && th::gemm_supported(qd, H) && th::gemm_supported(nkv * hd, H)) {
+            if (!few_path && use_gemm(H) && th::gemm_supported(qd, H) && th::gemm_supported(nkv * hd, H)) {
                 const th::GemmOut o[3] = {
                     {L.q->ptr, qd, s->fq}, {L.k->ptr, nkv * hd, s->fk}, {L.v->ptr, nkv * hd, s->fv}};
                 TH_HIP(th::launch_gemm_multi(st, s->fxb, n, H, o, 3, s->fsplit, s->fsplit_bytes));
@@ -698,7 +720,7 @@ int enqueue_fused(th_state *s, const uint32_t *tokens, size_t n, size_t pos, con
             }
             continue;
         }
-        if (use_gemm(qd) && th::gemm_supported(H, qd)) {
+        if (!few_path && use_gemm(qd) && th::gemm_supported(H, qd)) {
             const th::GemmOut o{L.o->ptr, H, s->fy};
             TH_HIP(th::launch_gemm_multi(st, s->fatt, n, qd, &o, 1, s->fsplit, s->fsplit_bytes));
             one_residual();
@@ -707,7 +729,7 @@ int enqueue_fused(th_state *s, const uint32_t *tokens, size_t n, size_t pos, con
         }
         TH_HIP(th::launch_add_rmsnorm_parts(st, s->fx, res, nres, res_stride, s->fxb, nullptr, nullptr, n,
                                             L.mlp_norm->ptr, H, eps));
-        if (use_gemm(H) && th::gemm_supported(I, H)) {
+        if (!few_path && use_gemm(H) && th::gemm_supported(I, H)) {
             const th::GemmOut o[2] = {{L.gate->ptr, I, s->fgate}, {L.up->ptr, I, s->fup}};
             TH_HIP(th::launch_gemm_multi(st, s->fxb, n, H, o, 2, s->fsplit, s->fsplit_bytes));
             TH_HIP(th::launch_silu_mul(st, s->fgate, s->fup, n * I));
@@ -718,7 +740,7 @@ int enqueue_fused(th_state *s, const uint32_t *tokens, size_t n, size_t pos, con
             TH_HIP(th::launch_matmul(st, s->fup, L.up->ptr, I, H, s->fxb, n));
             TH_HIP(th::launch_silu_mul(st, s->fgate, s->fup, n * I));
         }
-        if (use_gemm(I) && th::gemm_supported(H, I)) {
+        if (!few_path && use_gemm(I) && th::gemm_supported(H, I)) {
             const th::GemmOut o{L.down->ptr, H, s->fy};
             TH_HIP(th::launch_gemm_multi(st, s->fgate, n, I, &o, 1, s->fsplit, s->fsplit_bytes));
             one_residual();
