@@ -324,6 +324,7 @@ def test_step_attention_split(hip, tlib, nh, nkv, ctx, max_len, kv_bf16):
 
 
 @pytest.mark.parametrize("shape,n,pos", [("0.6b", 100, 0), ("0.6b", 512, 37), ("0.6b", 512, 64), ("4b", 100, 20),
+                                         ("0.6b", 1000, 5), ("0.6b", 970, 32), ("4b", 512, 32), ("4b", 450, 7),
                                          ("narrow", 12288, 0), ("narrow", 12200, 96)])
 def test_gemm_qkv(hip, tlib, shape, n, pos):
     """The head tile (32 tokens x one head) and, for the narrow shape, the
@@ -397,7 +398,8 @@ def _check_planes(got, dk, dv, pos, n, nkv, L):
         assert bad.size == 0, f"{name}: {bad.size} entries differ, first at {bad[:4]}"
 
 
-@pytest.mark.parametrize("H,I,n", [(1024, 3072, 100), (1024, 3072, 512), (2560, 9728, 100), (256, 3072, 8000)])
+@pytest.mark.parametrize("H,I,n", [(1024, 3072, 100), (1024, 3072, 512), (2560, 9728, 100), (256, 3072, 8000),
+                                   (1024, 3072, 250), (1024, 3072, 1000), (2560, 9728, 256), (512, 3200, 300)])
 def test_gemm_silu(hip, tlib, H, I, n):
     """The 0.6B and 4B shapes take the 64 x 64 and 128 x 128 tiles; 8000
     tokens x 2 x 3072 rows, 768 tiles of 256 x 256, the largest tile with its

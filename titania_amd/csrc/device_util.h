@@ -164,6 +164,22 @@ __device__ __forceinline__ float rows_sum(float v) {
     return __uint_as_float(q[0]) + __uint_as_float(q[1]);
 }
 
+// wave_sum's value, bit for bit, without its six LDS round trips: the same
+// butterfly, lanes 32 and 16 apart by permlane swaps, 8 and 4 by rotations of
+// a 16-lane row (4 apart, a rotation brings the other lane or the one 8 from
+// it, which holds the same sum by then), 2 and 1 within quads.
+__device__ __forceinline__ float wave_sum_swap(float v) {
+    auto q = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(q[0]) + __uint_as_float(q[1]);
+    auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+    v += dpp_get<0x128>(v, 0.f);  // row_ror:8
+    v += dpp_get<0x124>(v, 0.f);  // row_ror:4
+    v += dpp_get<0x4E>(v, 0.f);   // quad_perm [2,3,0,1]
+    v += dpp_get<0xB1>(v, 0.f);   // quad_perm [1,0,3,2]
+    return v;
+}
+
 // Sum over aligned groups of `width` lanes (width a power of two <= 64).
 template <int WIDTH>
 __device__ __forceinline__ float group_sum(float v) {

@@ -159,7 +159,7 @@ __device__ __forceinline__ void norm_rope_pairs(float av[4], float bv[4], int la
 #pragma unroll
     for (int k = 0; k < 4; ++k) ss += av[k] * av[k] + bv[k] * bv[k];
     if (gain) {
-        ss = wave_sum(ss);
+        ss = wave_sum_swap(ss);
         const float scale = 1.0f / sqrtf(ss / (float)hd + eps);
 #pragma unroll
         for (int k = 0; k < 4; ++k) {

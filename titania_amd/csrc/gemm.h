@@ -69,7 +69,7 @@ hipError_t launch_gemm_silu(hipStream_t s, const uint16_t *hi, const uint16_t *l
                             const uint16_t *gate, const uint16_t *up, size_t inter, uint16_t *h_hi, uint16_t *h_lo);
 
 // Whether the q/k/v GEMM of n tokens takes launch_gemm_qkv: head_dim 128 and
-// a launch the large tile would not take.
+// a launch the 256 x 256 tile would not take.
 bool gemm_qkv_fused(size_t n, size_t q_rows, size_t kv_rows, size_t cols, size_t head_dim);
 
 // The q, k and v GEMMs on split activations hi/lo [a.n][cols] (weights

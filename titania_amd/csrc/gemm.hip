@@ -65,6 +65,14 @@ using Small = Tile<64, 64, 64, 3>;    // 24 KB a stage: two blocks a CU
 using Small2 = Tile<64, 64, 64, 2>;
 using Large = Tile<128, 128, 64, 3, 4, 2>;  // 48 KB a stage: one block a CU, eight waves of 32 x 64
 using Head = Tile<32, 128, 64, 3>;          // one attention head's 128 rows: 24 KB a stage, two blocks a CU
+// One block a CU for launches of about one or two tiles a CU, where the small
+// tiles are bound by the operands' bytes through L2 (each block stages 24 KB
+// for 64 x 64 products): eight waves, 32 KB a stage for twice the products, 40
+// KB for three times (the GEMM alone, 512 tokens x 4096 x 1024, 256 blocks:
+// 12.8 us against 15.4 with the head tile; x 6144 x 1024, 256 blocks: 16.4
+// against 21.4 with Small2; x 6144 x 2560 35.3 against 48.3).
+using Mid = Tile<64, 128, 64, 4, 2, 4>;
+using Wide = Tile<64, 192, 64, 3, 2, 4>;
 // 48 KB a stage of 32 K columns: one block a CU, eight waves of 64 x 128. A
 // wave reads 16 fragments from LDS per 64 products, against 8 per 16 in the
 // 32 x 64 waves of the large tile.
@@ -446,6 +454,26 @@ __device__ __forceinline__ void gemm_tile(int ty, SegTile sg, const uint16_t *__
         static_assert(T::BN == 128, "one head of 128 dimensions a tile");
         static_assert(sizeof(ring) >= sizeof(float) * T::BM * EPS, "the epilogue tile fits the ring");
         float *ep = reinterpret_cast<float *>(ring);
+        const QkvPostArgs &a = *ht.a;
+        const long long pos0 = a.pos_dev ? *a.pos_dev : a.pos;
+        // The gains and angles of this wave's tokens, requested before the
+        // tile goes to LDS (read token by token, each was one more memory
+        // round trip: 512 tokens x 4096 x 1024 with this epilogue 20.2 -> 19.0 us).
+        constexpr int NWAVES = T::NT / 64, TPW = T::BM / NWAVES;
+        const uint16_t *gain = ht.role == 0 ? a.q_norm : ht.role == 1 ? a.k_norm : nullptr;
+        float g0 = 1.f, g1 = 1.f;
+        float2 cs[TPW];
+        if (ht.role < 2) {
+            if (gain) {
+                g0 = bf16_to_f32(gain[lane]);
+                g1 = bf16_to_f32(gain[lane + 64]);
+            }
+#pragma unroll
+            for (int k = 0; k < TPW; ++k) {
+                const long long t = min(t0 + wave + k * NWAVES, n - 1);
+                cs[k] = reinterpret_cast<const float2 *>(a.rope + (pos0 + t) * 128)[lane];
+            }
+        }
         __syncthreads();
 #pragma unroll
         for (int m = 0; m < FM; ++m)
@@ -454,20 +482,20 @@ __device__ __forceinline__ void gemm_tile(int ty, SegTile sg, const uint16_t *__
 #pragma unroll
                 for (int i = 0; i < 4; ++i) ep[(wm + m * 16 + fq * 4 + i) * EPS + wn + q * 16 + fr] = acc[m][q][i];
         __syncthreads();
-        const QkvPostArgs &a = *ht.a;
-        const long long pos0 = a.pos_dev ? *a.pos_dev : a.pos;
-        // A v head's V^T planes: a whole tile of 32 tokens that starts a
-        // 32-key slice writes its slice from LDS, 16 bytes a store; other
-        // tiles write each element at its column.
-        const bool vt_tile = ht.role == 2 && a.vh && ((pos0 + t0) & 31) == 0 && t0 + T::BM <= n;
-        if (vt_tile) {
-            static_assert(T::BM == 32, "a tile of one 32-key slice");
-            const long long c0 = pos0 + t0;
-            for (int e = tid; e < 128 * 4; e += T::NT) {
-                const int d = e >> 2, g = e & 3;
+        // A v head's V^T planes: 32 tokens of the tile that make a whole
+        // 32-key slice are written from LDS, 16 bytes a store; others write
+        // each element at its column.
+        static_assert(T::BM % 32 == 0, "tiles of whole 32-key slices");
+        const bool aligned = ht.role == 2 && a.vh && ((pos0 + t0) & 31) == 0;
+        auto vt_slice = [&](int tl) { return aligned && t0 + (tl & ~31) + 32 <= n; };
+        if (aligned) {
+            for (int e = tid; e < T::BM * 16; e += T::NT) {
+                const int s0 = e / 512 * 32, d = (e >> 2) & 127, g = e & 3;
+                if (!vt_slice(s0)) continue;
+                const long long c0 = pos0 + t0 + s0;
                 float f[8];
 #pragma unroll
-                for (int i = 0; i < 8; ++i) f[i] = ep[(i < 4 ? 4 * g + i : 16 + 4 * g + i - 4) * EPS + d];
+                for (int i = 0; i < 8; ++i) f[i] = ep[(s0 + (i < 4 ? 4 * g + i : 16 + 4 * g + i - 4)) * EPS + d];
                 uint2 h0, l0, h1, l1;
                 split_bf16x4(make_float4(f[0], f[1], f[2], f[3]), h0, l0);
                 split_bf16x4(make_float4(f[4], f[5], f[6], f[7]), h1, l1);
@@ -476,39 +504,49 @@ __device__ __forceinline__ void gemm_tile(int ty, SegTile sg, const uint16_t *__
                 *reinterpret_cast<uint4 *>(a.vl + o) = make_uint4(l0.x, l0.y, l1.x, l1.y);
             }
         }
-        for (int tl = wave; tl < T::BM; tl += T::NT / 64) {
+#pragma unroll
+        for (int k = 0; k < TPW; ++k) {
+            const int tl = wave + k * NWAVES;
             const long long t = t0 + tl;
             if (t >= n) break;
-            float av[4] = {ep[tl * EPS + lane], 0.f, 0.f, 0.f}, bv[4] = {ep[tl * EPS + 64 + lane], 0.f, 0.f, 0.f};
+            float av = ep[tl * EPS + lane], bv = ep[tl * EPS + 64 + lane];
             const long long pos = pos0 + t;
             if (ht.role == 2) {
                 KV *vc = reinterpret_cast<KV *>(a.v_cache) + (long long)ht.head * a.head_stride + pos * a.pos_stride;
-                store_kv(vc + lane, av[0]);
-                store_kv(vc + lane + 64, bv[0]);
-                if (a.vh && !vt_tile) {
+                store_kv(vc + lane, av);
+                store_kv(vc + lane + 64, bv);
+                if (a.vh && !vt_slice(tl)) {
                     // V^T planes: dimension-major rows, the key's column in its slice.
                     const long long col = (pos & ~31LL) + vt_column((int)(pos & 31));
                     const long long o0 = ((long long)ht.head * 128 + lane) * a.plane_len + col;
                     const long long o1 = o0 + 64 * a.plane_len;
-                    split_bf16(av[0], a.vh[o0], a.vl[o0]);
-                    split_bf16(bv[0], a.vh[o1], a.vl[o1]);
+                    split_bf16(av, a.vh[o0], a.vl[o0]);
+                    split_bf16(bv, a.vh[o1], a.vl[o1]);
                 }
                 continue;
             }
-            norm_rope_pairs(av, bv, lane, 128, ht.role == 0 ? a.q_norm : a.k_norm, a.eps, a.rope + pos * 128);
+            // norm_rope_pairs' operations, in its order.
+            if (gain) {
+                const float scale = 1.0f / sqrtf(wave_sum_swap(av * av + bv * bv) / 128.f + a.eps);
+                av = av * (scale * g0);
+                bv = bv * (scale * g1);
+            }
+            const float x0 = av * cs[k].x - bv * cs[k].y, x1 = bv * cs[k].x + av * cs[k].y;
+            av = x0;
+            bv = x1;
             if (ht.role == 0) {
                 float *dst = a.q + (t * a.n_heads + ht.head) * 128;
-                dst[lane] = av[0];
-                dst[lane + 64] = bv[0];
+                dst[lane] = av;
+                dst[lane + 64] = bv;
             } else {
                 KV *kc = reinterpret_cast<KV *>(a.k_cache) + (long long)ht.head * a.head_stride + pos * a.pos_stride;
-                store_kv(kc + lane, av[0]);
-                store_kv(kc + lane + 64, bv[0]);
+                store_kv(kc + lane, av);
+                store_kv(kc + lane + 64, bv);
                 if (a.kh) {
                     // K planes: row-major, the key's row at its position.
                     const long long o = ((long long)ht.head * a.plane_len + pos) * 128 + lane;
-                    split_bf16(av[0], a.kh[o], a.kl[o]);
-                    split_bf16(bv[0], a.kh[o + 64], a.kl[o + 64]);
+                    split_bf16(av, a.kh[o], a.kl[o]);
+                    split_bf16(bv, a.kh[o + 64], a.kl[o + 64]);
                 }
             }
         }
@@ -562,16 +600,16 @@ __global__ __launch_bounds__(T::NT, T::NT == 256 ? (T::kStages == 2 ? 3 : 2) : 1
     const uint16_t *__restrict__ lo, int n, int cols, int inter, int gx, int gy, uint16_t *__restrict__ h_hi,
     uint16_t *__restrict__ h_lo) {
     int tx, ty;
-    tile_of_block<T::NT == 256 ? 8 : T::BM == 256 ? 2 : 4>(tx, ty, gx, gy);
+    tile_of_block<T::BM == 64 ? 8 : T::BM == 256 ? 2 : 4>(tx, ty, gx, gy);
     const PairTile pt{gate, up, h_hi, h_lo, inter, tx * (T::BN / 2)};
     gemm_tile<T, kSiluPairs>(ty, SegTile{}, hi, lo, n, cols, nullptr, 1, pt);
 }
 
 // q, k and v in one launch, block x taking attention head x of the
-// concatenation (q heads, then k, then v) for 32 tokens, with the q/k/v
+// concatenation (q heads, then k, then v) for T::BM tokens, with the q/k/v
 // post-processing epilogue (the work of qk_norm_rope_append).
-template <typename KV>
-__global__ __launch_bounds__(Head::NT, 2) void gemm_qkv_kernel(const uint16_t *__restrict__ wq,
+template <class T, typename KV>
+__global__ __launch_bounds__(T::NT, T::NT == 256 ? 2 : 1) void gemm_qkv_kernel(const uint16_t *__restrict__ wq,
                                                                const uint16_t *__restrict__ wk,
                                                                const uint16_t *__restrict__ wv,
                                                                const uint16_t *__restrict__ hi,
@@ -581,12 +619,12 @@ __global__ __launch_bounds__(Head::NT, 2) void gemm_qkv_kernel(const uint16_t *_
     // that every field the first loads need fits the 14 preloaded dwords.
     const int nq = nqkv & 0xffff, nkv = nqkv >> 16;
     int h, ty;
-    tile_of_block<8>(h, ty, gxy & 0xffff, gxy >> 16);
+    tile_of_block<T::BM <= 64 ? 8 : 4>(h, ty, gxy & 0xffff, gxy >> 16);
     const int role = h < nq ? 0 : h < nq + nkv ? 1 : 2;
     const int head = role == 0 ? h : role == 1 ? h - nq : h - nq - nkv;
     const uint16_t *w = (role == 0 ? wq : role == 1 ? wk : wv) + (size_t)head * 128 * cols;
     SegTile sg{w, nullptr, 128, 0};
-    gemm_tile<Head, kQkvHead, KV>(ty, sg, hi, lo, n, cols, nullptr, 1, PairTile{}, HeadTile{&a, role, head});
+    gemm_tile<T, kQkvHead, KV>(ty, sg, hi, lo, n, cols, nullptr, 1, PairTile{}, HeadTile{&a, role, head});
 }
 
 // q, k and v in one launch on the 256 x 256 tile, block x taking rows
@@ -789,6 +827,24 @@ Plan gemm_plan(size_t n, size_t rows, size_t cols, int n_outs, bool rows_large, 
     return {false, false, (int)std::max<size_t>(std::min(fill, most), 1)};
 }
 
+// What a launch of a tile costs, in the time of one K step of one product
+// block: rounds of blocks on the chip's 256 CUs, each of the tile's products,
+// times what such a round took for each product, relative (the GEMM alone,
+// 1024 columns: 256 blocks of Wide 16.4 us, 256 of Mid 12.8 and 192 12.4, 192
+// of Large 18.6, 512 of Small and Head 15.5 and 256 10.1 to 10.6, 768 of
+// Small2 21.4).
+double tile_cost(size_t blocks, size_t products, size_t per_cu, double per_product) {
+    return (double)((blocks + 256 * per_cu - 1) / (256 * per_cu)) * (double)(per_cu * products) * per_product;
+}
+size_t tiles_of(size_t n, size_t per) { return (n + per - 1) / per; }
+// The small tiles' rounds: half empty ones still take most of their time.
+double small_cost(size_t blocks) {
+    return blocks <= 256 ? tile_cost(blocks, 64 * 64, 1, 2.6) : tile_cost(blocks, 64 * 64, 2, 1.9);
+}
+double mid_cost(size_t blocks) { return tile_cost(blocks, 64 * 128, 1, 1.5); }
+double wide_cost(size_t blocks) { return tile_cost(blocks, 64 * 192, 1, 1.3); }
+double large_cost(size_t blocks) { return tile_cost(blocks, 128 * 128, 1, 1.1); }
+
 // Whether the plan for these matrices is the small tile.
 bool small_plan(size_t n, size_t cols, const GemmOut *outs, int n_outs, int *ksplit) {
     size_t total = 0;
@@ -890,6 +946,21 @@ hipError_t launch_gemm_silu(hipStream_t s, const uint16_t *hi, const uint16_t *l
         gemm_silu_kernel<Large><<<grid, Large::NT, 0, s>>>(gate, up, hi, lo, (int)n, (int)cols, (int)inter,
                                                            (int)grid.x, (int)grid.y, h_hi, h_lo);
     } else {
+        // Fewer large tiles than two a CU: the tile whose rounds cost least.
+        const size_t small = tiles_of(n, 64) * (inter / (Small::BN / 2)), mid = tiles_of(n, 64) * (inter / (Mid::BN / 2));
+        const double cs = small > kSmall2MinTiles ? tile_cost(small, 64 * 64, 3, 1.74) : small_cost(small);
+        const double cm = mid_cost(mid), cl = large_cost(tiles_of(n, 128) * (inter / (Large::BN / 2)));
+        const double cw = inter % (Wide::BN / 2) ? 1e30 : wide_cost(tiles_of(n, 64) * (inter / (Wide::BN / 2)));
+        auto launch = [&](auto tile) {
+            using T = decltype(tile);
+            const dim3 grid((unsigned)(inter / (T::BN / 2)), (unsigned)tiles_of(n, T::BM));
+            gemm_silu_kernel<T><<<grid, T::NT, 0, s>>>(gate, up, hi, lo, (int)n, (int)cols, (int)inter, (int)grid.x,
+                                                       (int)grid.y, h_hi, h_lo);
+            return hipGetLastError();
+        };
+        if (cw < cs && cw <= cm && cw <= cl) return launch(Wide{});
+        if (cl < cs && cl <= cm) return launch(Large{});
+        if (cm < cs) return launch(Mid{});
         dim3 grid((unsigned)(inter / (Small::BN / 2)), (unsigned)((n + Small::BM - 1) / Small::BM));
         if ((size_t)grid.x * grid.y > kSmall2MinTiles)
             gemm_silu_kernel<Small2><<<grid, Small2::NT, 0, s>>>(gate, up, hi, lo, (int)n, (int)cols, (int)inter,
@@ -926,7 +997,9 @@ hipError_t launch_gemm_qkv_huge(hipStream_t s, const uint16_t *hi, const uint16_
 
 bool gemm_qkv_fused(size_t n, size_t q_rows, size_t kv_rows, size_t cols, size_t head_dim) {
     return head_dim == 128 && q_rows % 128 == 0 && kv_rows % 128 == 0 && cols % BK == 0 &&
-           !gemm_plan(n, q_rows + 2 * kv_rows, cols, 3, true, false).large;
+           !gemm_plan(n, q_rows + 2 * kv_rows, cols, 3, true,
+                      q_rows % Huge::BN == 0 && kv_rows % Huge::BN == 0)
+                .huge;
 }
 
 hipError_t launch_gemm_qkv(hipStream_t s, const uint16_t *hi, const uint16_t *lo, size_t cols, const uint16_t *wq,
@@ -941,13 +1014,24 @@ hipError_t launch_gemm_qkv(hipStream_t s, const uint16_t *hi, const uint16_t *lo
     if (a.kh && (!a.kl || !a.vh || !a.vl || a.kv_bf16 || a.plane_len % 64 ||
                  (!a.pos_dev && (a.pos < 0 || a.pos + a.n > a.plane_len))))
         return hipErrorInvalidValue;
-    dim3 grid((unsigned)(a.n_heads + 2 * a.n_kv_heads), (unsigned)((a.n + Head::BM - 1) / Head::BM));
-    const int gxy = (int)(grid.x | grid.y << 16), nqkv = a.n_heads | a.n_kv_heads << 16;
-    if (a.kv_bf16)
-        gemm_qkv_kernel<uint16_t><<<grid, Head::NT, 0, s>>>(wq, wk, wv, hi, lo, a.n, (int)cols, gxy, nqkv, a);
-    else
-        gemm_qkv_kernel<float><<<grid, Head::NT, 0, s>>>(wq, wk, wv, hi, lo, a.n, (int)cols, gxy, nqkv, a);
-    return hipGetLastError();
+    const size_t heads = (size_t)a.n_heads + 2 * (size_t)a.n_kv_heads, n = (size_t)a.n;
+    const int nqkv = a.n_heads | a.n_kv_heads << 16;
+    auto launch = [&](auto tile) {
+        using T = decltype(tile);
+        const dim3 grid((unsigned)heads, (unsigned)tiles_of(n, T::BM));
+        const int gxy = (int)(grid.x | grid.y << 16);
+        if (a.kv_bf16)
+            gemm_qkv_kernel<T, uint16_t><<<grid, T::NT, 0, s>>>(wq, wk, wv, hi, lo, a.n, (int)cols, gxy, nqkv, a);
+        else
+            gemm_qkv_kernel<T, float><<<grid, T::NT, 0, s>>>(wq, wk, wv, hi, lo, a.n, (int)cols, gxy, nqkv, a);
+        return hipGetLastError();
+    };
+    // The tile whose rounds cost least.
+    const double ch = small_cost(tiles_of(n, 32) * heads), cm = mid_cost(tiles_of(n, 64) * heads),
+                 cl = large_cost(tiles_of(n, 128) * heads);
+    if (cl < ch && cl <= cm) return launch(Large{});
+    if (cm < ch) return launch(Mid{});
+    return launch(Head{});
 }
 
 hipError_t launch_splitk_sum(hipStream_t s, const float *part, float *out, size_t m, int ksplit) {
