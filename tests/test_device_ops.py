@@ -249,6 +249,14 @@ def test_qwen4b_prefill_gemm(hip, name, n):
     assert np.all(np.abs(got.astype(np.float64) - expected) <= 3e-5 * bound + 1e-6)
 
 
+@pytest.mark.parametrize("rows,cols,n", [(2560, 9728, 500), (9728, 2560, 129), (2560, 4160, 700), (1152, 6208, 1900)])
+def test_large_tile_split_k(hip, rows, cols, n):
+    """Matrices whose large-tile launch takes K in 3 or more parts (two for the
+    last), uneven ones and tokens past a tile's edge; the bound of
+    test_split_k_matmul."""
+    test_split_k_matmul(hip, rows, cols, n)
+
+
 @pytest.mark.parametrize("n", [16, 33, 64, 65, 130])
 @pytest.mark.parametrize("rows,cols", [(64, 64), (64, 1088), (192, 1280), (1088, 2048), (2560, 1152), (64, 4160)])
 def test_split_k_matmul(hip, rows, cols, n):

@@ -801,7 +801,30 @@ constexpr size_t kHugeSplitMinTiles = 256;
 struct Plan {
     bool large, huge;
     int ksplit;
+    double gain = 1e30;  // us that the large tile is ahead of the small one, where both were considered
 };
+
+// Floats of partials that more than two parts of a large tile's K may take.
+constexpr size_t kSplitFloats = (size_t)1 << 23;
+// us by which the large tile has to be ahead where the activations are f32 and
+// must be split first: two launches and an allocation (256 tokens x 9728 x
+// 2560 57.4 us with the small tile, 36.8 + 2.8 + 5 with the large; 512 x 4096 x
+// 2560 34.1, and 25.6 + 3.2 + 2.9).
+constexpr double kSplitLaunchUs = 10;
+
+// Parts of K that a single matrix takes in small tiles, so that the launch
+// fills the chip in whole rounds (up to 64 tiles: a block a CU; past them two)
+// with at least 4 K steps a part. The GEMM alone in 1 / 2 / 4 / 6 / 8 / 12 / 16
+// parts: 64 tokens x 1024 x 3072 (16 tiles) 25.4 / 14.3 / 8.8 / 6.9 / 6.1 / 5.3
+// / 5.1 us, x 2560 x 9728 (40 tiles) 75.0 / 39.8 / 22.9 / 17.4 / 21.9 / 17.6 /
+// 19.9; 128 tokens x 2560 x 9728 in 4 / 6 / 8: 36.6 / 27.4 / 30.3; 512 x 1024 x
+// 3072 in 2 / 4 / 6: 15.0 / 13.8 / 16.2.
+size_t most_parts(size_t cols) { return std::min<size_t>(kGemmMaxSplitK, std::max<size_t>(cols / BK / 4, 1)); }
+int small_ksplit(size_t n, size_t rows, size_t cols) {
+    const size_t tiles = (rows / Small::BN) * ((n + Small::BM - 1) / Small::BM);
+    const size_t fill = (tiles <= 64 ? 256 : 512) / std::max<size_t>(tiles, 1);
+    return (int)std::max<size_t>(std::min(fill, most_parts(cols)), 1);
+}
 
 // rows_large / rows_huge: every matrix's rows are whole large / huge tiles.
 Plan gemm_plan(size_t n, size_t rows, size_t cols, int n_outs, bool rows_large, bool rows_huge) {
@@ -813,18 +836,34 @@ Plan gemm_plan(size_t n, size_t rows, size_t cols, int n_outs, bool rows_large, 
     if (lt >= kLargeMinTiles) return {true, false, 1};
     if (n_outs == 1 && lt >= kLargeSplitMinTiles && nk >= 96) return {true, false, 2};
     if (n_outs != 1) return {false, false, 1};
-    // Small tiles: a single matrix with few row tiles (o, down) splits K so
-    // that the launch fills the chip in whole rounds (up to 64 tiles: a block
-    // a CU; past them two), keeping at least 4 K steps a split. The GEMM alone
-    // in 1 / 2 / 4 / 6 / 8 / 12 / 16 parts: 64 tokens x 1024 x 3072 (16 tiles)
-    // 25.4 / 14.3 / 8.8 / 6.9 / 6.1 / 5.3 / 5.1 us, x 2560 x 9728 (40 tiles)
-    // 75.0 / 39.8 / 22.9 / 17.4 / 21.9 / 17.6 / 19.9; 128 tokens x 2560 x 9728
-    // in 4 / 6 / 8: 36.6 / 27.4 / 30.3; 512 x 1024 x 3072 in 2 / 4 / 6: 15.0 /
-    // 13.8 / 16.2.
     const size_t tiles = (rows / Small::BN) * ((n + Small::BM - 1) / Small::BM);
-    const size_t most = std::min<size_t>(kGemmMaxSplitK, std::max<size_t>(nk / 4, 1));
-    const size_t fill = (tiles <= 64 ? 256 : 512) / std::max<size_t>(tiles, 1);
-    return {false, false, (int)std::max<size_t>(std::min(fill, most), 1)};
+    const size_t small_ks = (size_t)small_ksplit(n, rows, cols);
+    if (lt == 0) return {false, false, (int)small_ks};
+    // Or large tiles, K in as many parts as make whole rounds of one block a
+    // CU: a CU's two small tiles stage as many bytes for half the products,
+    // and at a few hundred tokens of wide rows they fill no second round
+    // (small tiles against large ones in three parts: 512 tokens x 2560 x 9728
+    // 115.7 and 51.7 us, x 2560 x 4096 47.7 and 26.9; 1024 tokens 169 and 99,
+    // 77 and 48; 512 x 1024 x 3072, 13.3 and 13.3 to 15.5, stays; a 512-token
+    // prompt on four Qwen3-4B layers 1.56 -> 1.22 ms). Times in us
+    // as measured: ns a column and round, what a launch takes besides, and the
+    // partials that the consumer reads at 5 TB/s; large tiles from 15% less,
+    // what the estimate may be off.
+    auto partials = [&](size_t ks) { return ks > 1 ? (double)(ks * n * rows) * 4 / 5e6 : 0.; };
+    const size_t sb = tiles * small_ks;
+    const double small_us = (sb <= 256 ? 7.8e-3 : 13.5e-3 * (double)((sb + 511) / 512)) * (double)(cols / small_ks) + 3.4 +
+                            partials(small_ks);
+    double large_us = 1e30;
+    size_t large_ks = 1;
+    for (size_t ks = 1; ks <= most_parts(cols) && (ks <= 2 || ks * n * rows <= kSplitFloats); ++ks) {
+        const double us = 13.2e-3 * (double)((lt * ks + 255) / 256) * (double)(cols / ks) + 8.9 + partials(ks);
+        if (us < large_us) {
+            large_us = us;
+            large_ks = ks;
+        }
+    }
+    if (large_us < 0.85 * small_us) return {true, false, (int)large_ks, small_us - large_us};
+    return {false, false, (int)small_ks};
 }
 
 // What a launch of a tile costs, in the time of one K step of one product
@@ -856,16 +895,20 @@ bool small_plan(size_t n, size_t cols, const GemmOut *outs, int n_outs, int *ksp
     }
     const Plan plan = gemm_plan(n, total, cols, n_outs, rows_large, rows_huge);
     *ksplit = plan.ksplit;
-    return !plan.large && !plan.huge && total / Small::BN <= 0xffff && (n + Small::BM - 1) / Small::BM <= 0xffff &&
+    if (plan.large && !plan.huge && plan.gain <= kSplitLaunchUs) *ksplit = small_ksplit(n, total, cols);
+    else if (plan.large || plan.huge) return false;
+    return total / Small::BN <= 0xffff && (n + Small::BM - 1) / Small::BM <= 0xffff &&
            n <= ((size_t)1 << 24);
 }
 
 }  // namespace
 
 size_t gemm_scratch_bytes(size_t n, size_t cols, size_t rows) {
-    // The larger tiles split K in two at most, the small one into at most 512
-    // tiles in all.
-    return n * cols * 2 * sizeof(uint16_t) + std::max(2 * n * rows, kPartFloats) * sizeof(float);
+    // K in two parts at any size, in more within kSplitFloats (the large tile)
+    // or kPartFloats (the small one's at most 512 tiles in all).
+    static_assert(kPartFloats <= kSplitFloats, "the small tile's partials fit");
+    const size_t part = std::max(2 * n * rows, std::min((size_t)kGemmMaxSplitK * n * rows, kSplitFloats));
+    return n * cols * 2 * sizeof(uint16_t) + part * sizeof(float);
 }
 
 hipError_t launch_gemm_split(hipStream_t s, const float *x, size_t n, size_t cols, uint16_t *hi, uint16_t *lo) {
@@ -1089,10 +1132,9 @@ hipError_t launch_gemm_outs(hipStream_t s, const float *x, size_t n, size_t cols
                             float *part) {
     if (n == 0) return hipSuccess;
     if (n_outs < 1 || n_outs > 3 || (uintptr_t)x % 16) return hipErrorInvalidValue;
-    size_t most = 0, total = 0;
+    size_t total = 0;
     for (int i = 0; i < n_outs; ++i) {
         if (!gemm_supported(outs[i].rows, cols)) return hipErrorInvalidValue;
-        most = std::max(most, outs[i].rows);
         total += outs[i].rows;
     }
     // Small tiles take the f32 activations as they are, with partials in the
@@ -1107,7 +1149,8 @@ hipError_t launch_gemm_outs(hipStream_t s, const float *x, size_t n, size_t cols
         return e != hipSuccess || ksplit == 1 ? e : launch_splitk_sum(s, part, outs[0].out, n * total, ksplit);
     }
     void *scratch = nullptr;
-    const size_t bytes = gemm_scratch_bytes(n, cols, most);
+    const size_t bytes = n * cols * 2 * sizeof(uint16_t) +
+                         (size_t)gemm_ksplit(n, total, cols, n_outs) * n * total * sizeof(float);
     hipError_t e = hipMallocAsync(&scratch, bytes, s);
     if (e != hipSuccess) return e;
     e = launch_gemm_multi(s, x, n, cols, outs, n_outs, scratch, bytes);
