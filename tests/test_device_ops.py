@@ -457,6 +457,16 @@ def test_prefill_attention_tiles(hip, n, pos, H, KVH):
     assert_close(got, expected, rel=1e-4, abs_=1e-5, what=f"prefill attention n={n} pos={pos}")
 
 
+@pytest.mark.parametrize("n,pos,H,KVH", [(8, 8, 16, 8), (11, 150, 16, 8), (11, 700, 32, 8), (40, 1500, 16, 8),
+                                         (64, 1000, 32, 8), (17, 3000, 8, 1), (200, 700, 32, 8), (129, 129, 4, 4)])
+def test_attention_after_context(hip, n, pos, H, KVH):
+    """Several tokens after a longer context: one key tile, three, a split a
+    tile, splits of uneven tiles, both combine kernels, one KV head, several
+    token tiles, and the shortest context that counts as longer. The bounds of
+    test_prefill_attention_tiles (the same products and partial sums)."""
+    test_prefill_attention_tiles(hip, n, pos, H, KVH)
+
+
 # ---- fused extensions ----
 
 def test_add_rmsnorm(hip):

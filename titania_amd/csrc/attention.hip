@@ -579,6 +579,10 @@ __global__ __launch_bounds__(64) void attn_combine_lanes_kernel(float *__restric
     }
 }
 
+// attention_splits_at: most splits, and most blocks (of kGqaRows rows and a
+// split each) where that is more than one.
+constexpr size_t kMaxRoundSplits = 64, kMaxRoundBlocks = 1024;
+
 int attention_splits(size_t n, size_t n_heads, size_t n_kv_heads, size_t max_len, size_t head_dim) {
     // Several tokens on the matrix cores: split the keys until the launch has
     // about 512 blocks (two a CU), keeping at least two 64-key tiles a split,
@@ -586,6 +590,7 @@ int attention_splits(size_t n, size_t n_heads, size_t n_kv_heads, size_t max_len
     // one split needs no combine launch at all). Splitting on to about 1024
     // blocks was slower: 9.71 against 9.26 ms for a 2048-token Qwen3-0.6B
     // prefill, 205.7 against 202.5 ms for 8192 tokens of the Qwen3-4B shape.
+    // Tokens after a context at least as long take attention_splits_at.
     if (head_dim == 128 && n >= kAttnTileMin) {
         const size_t group = n_kv_heads ? n_heads / n_kv_heads : 0;
         const bool gqa = group >= 1 && group <= 8 && 8 % group == 0 && group * n_kv_heads == n_heads;
@@ -610,6 +615,37 @@ int attention_splits(size_t n, size_t n_heads, size_t n_kv_heads, size_t max_len
     size_t cap = (max_len + 63) / 64;
     size_t s = std::min(want, cap);
     return (int)std::max<size_t>(1, std::min<size_t>(s, 256));
+}
+
+size_t attention_splits_scratch(size_t n, size_t n_heads, size_t max_len, size_t head_dim) {
+    const size_t ns = std::min<size_t>(kMaxRoundSplits, (max_len + kGqaKeys - 1) / kGqaKeys);
+    return std::min(n * n_heads * ns, kMaxRoundBlocks * kGqaRows) * (head_dim + 2);
+}
+
+int attention_splits_at(size_t n, size_t n_heads, size_t n_kv_heads, size_t pos, size_t head_dim, size_t floats) {
+    const int least = attention_splits(n, n_heads, n_kv_heads, pos + n, head_dim);
+    const size_t group = n_kv_heads ? n_heads / n_kv_heads : 0;
+    if (head_dim != 128 || n < kAttnTileMin || pos < n || group < 1 || group > 8 || 8 % group ||
+        group * n_kv_heads != n_heads)
+        return least;
+    const size_t qt = kGqaRows / group, blocks = (n + qt - 1) / qt * n_kv_heads;
+    // Past 96 blocks a launch takes several rounds anyway, which the order of
+    // its blocks fills better than the estimate knows (Qwen3-0.6B, 2000 tokens
+    // at 2500, 256 blocks: 4.78 ms in two splits, 4.99 in one).
+    if (blocks > 96) return least;
+    const size_t tiles = (pos + n + kGqaKeys - 1) / kGqaKeys;
+    double best = 1e30;
+    size_t ns = 1;
+    for (size_t k = 1; k <= std::min(tiles, kMaxRoundSplits) && (k == 1 || blocks * k <= kMaxRoundBlocks); ++k) {
+        const double rounds = (double)((blocks * k + 255) / 256);
+        const double cost = rounds * (double)((tiles + k - 1) / k + 2) +
+                            (k > 1 ? 1.4 + (double)(n * n_heads * k) * 5.2e-5 : 0.);
+        if (cost < best) {
+            best = cost;
+            ns = k;
+        }
+    }
+    return attention_scratch(n, n_heads, head_dim, (int)ns) <= floats ? (int)ns : least;
 }
 
 size_t attention_scratch(size_t n, size_t n_heads, size_t head_dim, int nsplit) {

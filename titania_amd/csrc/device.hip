@@ -444,8 +444,14 @@ int attention(th_device *dev, th_buffer *out, const th_buffer *q, const th_buffe
     TH_REQUIRE(k_cache->len >= (pos + n) * kv_dim && v_cache->len >= (pos + n) * kv_dim,
                "the caches do not hold position %zu", pos + n - 1);
     TH_REQUIRE(out->ptr != q->ptr, "attention cannot write its queries");
+    // Calls that cannot grow their scratch are refused by what
+    // attention_splits needs, and split further only within what there is.
+    const size_t room = fixed ? th::noalloc_scratch_bytes() / sizeof(float)
+                        : dev->capturing ? dev->scratch_bytes / sizeof(float) : SIZE_MAX;
     int nsplit = th::attention_splits(n, n_heads, n_kv_heads, pos + n, head_dim);
-    size_t floats = th::attention_scratch(n, n_heads, head_dim, nsplit);
+    if (th::attention_scratch(n, n_heads, head_dim, nsplit) <= room)
+        nsplit = th::attention_splits_at(n, n_heads, n_kv_heads, pos, head_dim, room);
+    const size_t floats = th::attention_scratch(n, n_heads, head_dim, nsplit);
     float *scr = nullptr;
     if (floats && fixed) {
         TH_REQUIRE(floats * sizeof(float) <= th::noalloc_scratch_bytes(),

@@ -324,6 +324,10 @@ int ensure_fused_state(th_state *s) {
         s->attn_part_floats =
             std::max(s->attn_part_floats, th::attention_scratch(n, (size_t)c.num_attention_heads, hd, ns));
     }
+    if (hd == 128)
+        s->attn_part_floats =
+            std::max(s->attn_part_floats,
+                     th::attention_splits_scratch(s->fb, (size_t)c.num_attention_heads, s->max_len, hd));
     if (s->attn_part_floats) TH_HIP(hipMalloc(&s->attn_part, s->attn_part_floats * sizeof(float)));
     if (s->kv_dtype == TH_KV_F32 && s->fb >= th::kGemmMinTokens && hd == 128) {
         s->kv_planes_bytes = th::attention_planes_bytes(s->max_len, (size_t)c.num_key_value_heads);
@@ -528,7 +532,8 @@ int enqueue_fused(th_state *s, const uint32_t *tokens, size_t n, size_t pos, con
     const size_t qd = nh * hd;
     const int kv_bf16 = s->kv_dtype == TH_KV_BF16;
     const size_t max_ctx = pos_dev ? s->max_len : pos + n;
-    const int nsplit = th::attention_splits(n, nh, nkv, max_ctx, hd);
+    const int nsplit = pos_dev ? th::attention_splits(n, nh, nkv, max_ctx, hd)
+                               : th::attention_splits_at(n, nh, nkv, pos, hd, s->attn_part_floats);
     if (th::attention_scratch(n, nh, hd, nsplit) > s->attn_part_floats)
         return fail(TH_ERR_INVALID, "attention partials exceed the state's scratch");
     // Chunks of kGemmMinTokens or more go through the MFMA GEMM (activations
