@@ -327,6 +327,26 @@ def test_few_token_matmul(hip, rows, cols, n):
     assert np.all(np.abs(got[fine] - exp[fine]) <= bound[fine])
 
 
+@pytest.mark.parametrize("n", [33, 64, 65, 130, 300])
+@pytest.mark.parametrize("rows,cols", [(1, 8), (63, 64), (65, 72), (100, 1096), (40, 3000), (1003, 520), (300, 4088)])
+def test_ragged_matmul(hip, rows, cols, n):
+    """More than a few tokens of matrices that are not whole tiles: rows and
+    columns past a tile's edge by one row or chunk, K split or not, tokens
+    past a tile. Three bf16 terms are x exactly; the f32 sums add cols * 2^-24
+    of sum |w x| at most. Rows past the output stay as they were."""
+    rng = np.random.default_rng(rows + cols + n)
+    w = normal_bf16(rows * cols, 5, "ragged", 0.05)
+    x = rng.standard_normal((n, cols)).astype(np.float32)
+    wf = bf16_to_f32(w).astype(np.float64).reshape(rows, cols)
+    exp, size = x.astype(np.float64) @ wf.T, np.abs(x).astype(np.float64) @ np.abs(wf).T
+    bx, out = hip.alloc(x.size), hip.alloc(n * rows)
+    hip.write(bx, x)
+    hip.write(out, np.full(n * rows, np.nan, np.float32))
+    hip.matmul(out, hip.upload(Tensor((rows, cols), w)), bx)
+    got = hip.read(out).reshape(n, rows)
+    assert np.all(np.abs(got - exp) <= cols * 2.0**-24 * size)
+
+
 @pytest.mark.parametrize("rows,cols,n", [(6144, 1024, 2000), (4096, 6144, 1024), (6144, 512, 8000),
                                          (2560, 1024, 8000)])
 def test_large_tile_gemm(hip, rows, cols, n):

@@ -164,6 +164,44 @@ __device__ __forceinline__ float rows_sum(float v) {
     return __uint_as_float(q[0]) + __uint_as_float(q[1]);
 }
 
+typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16_term8;
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32_acc4;
+
+// Eight f32 as three bf16 terms. Cutting bits off, where rounding would carry,
+// leaves a remainder of at most 16 bits, exactly. An infinity is its own first
+// term, with nothing left over; a NaN's first term is one.
+__device__ __forceinline__ void split3(const uint4 &a, const uint4 &b, bf16_term8 (&t)[3]) {
+    const uint32_t u[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    uint32_t w[3][8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const float f = __uint_as_float(u[i]), h = __uint_as_float(u[i] & 0xffff0000u);
+        const float r = h == f ? 0.f : f - h;
+        const float m = __uint_as_float(__float_as_uint(r) & 0xffff0000u);
+        w[0][i] = u[i];
+        w[1][i] = __float_as_uint(r);
+        w[2][i] = __float_as_uint(r - m);
+    }
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        uint4 p;  // the upper halves of two words each
+        p.x = __builtin_amdgcn_perm(w[k][1], w[k][0], 0x07060302u);
+        p.y = __builtin_amdgcn_perm(w[k][3], w[k][2], 0x07060302u);
+        p.z = __builtin_amdgcn_perm(w[k][5], w[k][4], 0x07060302u);
+        p.w = __builtin_amdgcn_perm(w[k][7], w[k][6], 0x07060302u);
+        t[k] = __builtin_bit_cast(bf16_term8, p);
+    }
+}
+
+// Columns [c0, c1) of w . x one by one: for a sum of split3 terms' products
+// that is NaN, as a later term of zero times an infinite weight is where x w
+// is infinite.
+__device__ __forceinline__ float plain_dot(const uint16_t *w, const float *x, int c0, int c1) {
+    float s = 0.f;
+    for (int c = c0; c < c1; ++c) s = fmaf(bf16_to_f32(w[c]), x[c], s);
+    return s;
+}
+
 // wave_sum's value, bit for bit, without its six LDS round trips: the same
 // butterfly, lanes 32 and 16 apart by permlane swaps, 8 and 4 by rotations of
 // a 16-lane row (4 apart, a rotation brings the other lane or the one 8 from

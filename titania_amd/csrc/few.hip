@@ -26,8 +26,8 @@
 namespace th {
 namespace {
 
-typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
-typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4;
+typedef bf16_term8 bf16x8;
+typedef f32_acc4 f32x4;
 
 constexpr int kTokens = 16, kTerms = 3;
 constexpr unsigned kPastEnd = 0xfffffff0u;  // an offset no descriptor reaches: the load gives zero
@@ -50,32 +50,6 @@ __device__ __forceinline__ uint4 load16(__amdgpu_buffer_rsrc_t r, unsigned off) 
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t records(const void *p, unsigned bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, (int)bytes, kBufferRsrcWord3);
-}
-
-// Eight f32 as three bf16 terms. Cutting bits off, where rounding would carry,
-// leaves a remainder of at most 16 bits, exactly; an infinity is its own
-// first term, with nothing left over, and a NaN stays in the remainder.
-__device__ __forceinline__ void split8(const uint4 &a, const uint4 &b, bf16x8 (&t)[kTerms]) {
-    const uint32_t u[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-    uint32_t w[kTerms][8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const float f = __uint_as_float(u[i]), h = __uint_as_float(u[i] & 0xffff0000u);
-        const float r = h == f ? 0.f : f - h;
-        const float m = __uint_as_float(__float_as_uint(r) & 0xffff0000u);
-        w[0][i] = u[i];
-        w[1][i] = __float_as_uint(r);
-        w[2][i] = __float_as_uint(r - m);
-    }
-#pragma unroll
-    for (int k = 0; k < kTerms; ++k) {
-        uint4 p;  // the upper halves of two words each
-        p.x = __builtin_amdgcn_perm(w[k][1], w[k][0], 0x07060302u);
-        p.y = __builtin_amdgcn_perm(w[k][3], w[k][2], 0x07060302u);
-        p.z = __builtin_amdgcn_perm(w[k][5], w[k][4], 0x07060302u);
-        p.w = __builtin_amdgcn_perm(w[k][7], w[k][6], 0x07060302u);
-        t[k] = __builtin_bit_cast(bf16x8, p);
-    }
 }
 
 enum Epi { kRows, kSilu };
@@ -118,7 +92,7 @@ __global__ __launch_bounds__(64 * WK) void few_kernel(Args a) {
         }
         return [=](bf16x8(&xs)[NKS][kTerms]) {
 #pragma unroll
-            for (int k = 0; k < NKS; ++k) split8(v[k][0], v[k][1], xs[k]);
+            for (int k = 0; k < NKS; ++k) split3(v[k][0], v[k][1], xs[k]);
         };
     };
     // The weights of (tile, chunk), `second`: of up. Past the last tile, no
@@ -280,6 +254,14 @@ bool few_preferred(size_t n, size_t rows, size_t cols, int n_outs) {
     // x 9728, 32 tokens, 22.8 against 17, and x 19456 x 2560, 64 tokens, 53
     // against 45.
     return n_outs == 1 ? cols <= 1024 : rows * cols <= ((size_t)32 << 20) || n <= 32;
+}
+
+double few_us(size_t n, size_t rows, size_t cols) {
+    // Rounds of row tiles, past the chunks that the registers hold three times
+    // as long a column; besides, the launch and the first read of x.
+    const size_t y = (n + kTokens - 1) / kTokens, slots = std::max<size_t>(1, 256 / y);
+    const double rounds = (double)(((rows + 15) / 16 + slots - 1) / slots), c = 1e-3 * (double)cols;
+    return cols > 2560 ? 4 + 3 * rounds * c : 4 + 2 * c + rounds * std::max(0.9 * c, 0.5);
 }
 
 hipError_t launch_few(hipStream_t s, const float *x, size_t n, size_t cols, const GemmOut *outs, int n_outs,

@@ -44,6 +44,16 @@ hipError_t launch_gemm_f32(hipStream_t s, const float *x, size_t n, size_t cols,
 hipError_t launch_gemm_outs(hipStream_t s, const float *x, size_t n, size_t cols, const GemmOut *outs, int n_outs,
                             float *part);
 
+// The GEMM on f32 activations for a matrix of any number of rows, of columns
+// in whole 16-byte chunks: x enters as three bf16 terms, exactly. K in ksplit
+// parts as launch_gemm_f32 (gemm_ragged_ksplit: those that fill the chip).
+bool gemm_ragged_supported(size_t n, size_t rows, size_t cols);
+int gemm_ragged_ksplit(size_t n, size_t rows, size_t cols);
+// About how long launch_gemm_ragged and the sum of its parts take.
+double gemm_ragged_us(size_t n, size_t rows, size_t cols, int ksplit);
+hipError_t launch_gemm_ragged(hipStream_t s, const float *x, size_t n, size_t cols, const uint16_t *w, size_t rows,
+                              float *out, float *part, int ksplit);
+
 // Most ways a single-matrix GEMM splits its K range (into partial tiles that a
 // second kernel sums in a fixed order).
 constexpr int kGemmMaxSplitK = 16;

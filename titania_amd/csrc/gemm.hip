@@ -662,12 +662,18 @@ struct alignas(16) F32Stage {
 // waves a SIMD, one of which splits while the other multiplies. 64 tokens x
 // 2560 x 9728 with the sum of its parts, from HBM: 23.7 us; four waves of 16 x
 // 64 33.4, of 32 x 32 (each fragment split twice) 34.1.
+// TERMS 2: shapes of whole tiles, hi and lo terms. TERMS 3: one matrix of any
+// rows and of columns in whole 16-byte chunks, and the exact three terms of
+// few.hip's kernel, which otherwise takes these shapes and reads the weights
+// again for every 16 tokens.
 constexpr int kF32Threads = 512;
+template <int TERMS>
 __global__ __launch_bounds__(kF32Threads, 2) void gemm_f32_kernel(int gxy, int rows0, const uint16_t *__restrict__ w0,
                                                                   float *__restrict__ out0,
                                                                   const float *__restrict__ x, int n, int cols,
                                                                   int ksplit, float *__restrict__ part, Segs segs) {
     using T = Small;
+    constexpr bool RAGGED = TERMS == 3;
     constexpr int FN = T::BN / 16, kStages = T::kStages;
     static_assert(kF32Threads == 64 * 2 * (T::BM / 16) && T::BK == 64, "a wave for 16 tokens and half a stage");
     constexpr int XI = T::BM * 16 / kF32Threads, WI = T::TB / kF32Threads;  // loads a lane, of each
@@ -678,26 +684,32 @@ __global__ __launch_bounds__(kF32Threads, 2) void gemm_f32_kernel(int gxy, int r
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, t0 = ty * T::BM;
     const int wm = (wave & 3) * 16, half = wave >> 2;
     const int fr = lane & 15, fq = lane >> 4;
-    const int nk_all = cols / T::BK, z = blockIdx.z;
+    const int nk_all = RAGGED ? (cols + T::BK - 1) / T::BK : cols / T::BK, z = blockIdx.z;
     const int kb = (int)((long long)z * nk_all / ksplit), nk = (int)((long long)(z + 1) * nk_all / ksplit) - kb;
     const uint16_t *w = sg.w + (size_t)sg.local * cols + (size_t)kb * T::BK;
     const float *xk = x + (size_t)kb * T::BK;
-    // Token rows past n read row n - 1 (their results are never stored).
+    // Token rows past n read row n - 1 (their results are never stored); with
+    // RAGGED, weight rows past the last likewise, and columns past a row's end
+    // its last chunk (zeroed where they are read).
+    auto chunk = [&](int k0, int c, int width) { return RAGGED ? min(k0 + c, cols - kb * T::BK - width) : k0 + c; };
     auto issue = [&](F32Stage &st, int k0) {
 #pragma unroll
         for (int i = 0; i < XI; ++i) {
             const int span = wave * XI + i, p = span * 64 + lane, row = p / 16, pc = p % 16;
-            dma16(xk + (size_t)min(t0 + row, n - 1) * cols + k0 + (pc ^ (row & 15)) * 4, st.x + span * 64);
+            dma16(xk + (size_t)min(t0 + row, n - 1) * cols + chunk(k0, (pc ^ (row & 15)) * 4, 4), st.x + span * 64);
         }
 #pragma unroll
         for (int i = 0; i < WI; ++i) {
             const int span = wave * WI + i, p = span * 64 + lane, row = p / T::CH, pc = p % T::CH;
-            dma16(w + (size_t)row * cols + k0 + (pc ^ swz<T::CH>(row)) * 8, st.w + span * 64);
+            const int wr = RAGGED ? min(row, sg.rows - 1 - sg.local) : row;
+            dma16(w + (size_t)wr * cols + chunk(k0, (pc ^ swz<T::CH>(row)) * 8, 8), st.w + span * 64);
         }
     };
-    f32x4 acc[FN];
+    f32x4 acc[FN], rest[RAGGED ? FN : 1];  // RAGGED: the later terms' sums apart
 #pragma unroll
     for (int q = 0; q < FN; ++q) acc[q] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int q = 0; q < (RAGGED ? FN : 1); ++q) rest[q] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int s = 0; s < kStages - 1; ++s)
         if (s < nk) issue(ring[s], s * T::BK);
@@ -707,21 +719,41 @@ __global__ __launch_bounds__(kF32Threads, 2) void gemm_f32_kernel(int gxy, int r
         else wait_vm<0>();
         stage_barrier();
         const F32Stage &st = ring[k % kStages];
-        const uint4 x0 = st.x[row * 16 + ((2 * lc) ^ (row & 15))], x1 = st.x[row * 16 + ((2 * lc + 1) ^ (row & 15))];
+        uint4 x0 = st.x[row * 16 + ((2 * lc) ^ (row & 15))], x1 = st.x[row * 16 + ((2 * lc + 1) ^ (row & 15))];
         bf16x8 b[FN];
 #pragma unroll
         for (int q = 0; q < FN; ++q) b[q] = frag<T::CH>(st.w, q * 16 + fr, lc);
         if (k + kStages - 1 < nk) issue(ring[(k + kStages - 1) % kStages], (k + kStages - 1) * T::BK);
-        uint2 h0, l0, h1, l1;
-        split_bf16x4(__builtin_bit_cast(float4, x0), h0, l0);
-        split_bf16x4(__builtin_bit_cast(float4, x1), h1, l1);
-        const bf16x8 ah = __builtin_bit_cast(bf16x8, make_uint4(h0.x, h0.y, h1.x, h1.y));
-        const bf16x8 al = __builtin_bit_cast(bf16x8, make_uint4(l0.x, l0.y, l1.x, l1.y));
+        if constexpr (RAGGED) {
+            if ((kb + k + 1) * T::BK > cols && (kb + k) * T::BK + 8 * lc >= cols) {
+                x0 = x1 = make_uint4(0u, 0u, 0u, 0u);
 #pragma unroll
-        for (int q = 0; q < FN; ++q) acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, b[q], acc[q], 0, 0, 0);
+                for (int q = 0; q < FN; ++q) b[q] = __builtin_bit_cast(bf16x8, x0);
+            }
+            bf16x8 t[3];
+            split3(x0, x1, t);
 #pragma unroll
-        for (int q = 0; q < FN; ++q) acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, b[q], acc[q], 0, 0, 0);
+            for (int q = 0; q < FN; ++q) acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(t[0], b[q], acc[q], 0, 0, 0);
+#pragma unroll
+            for (int i = 1; i < 3; ++i)
+#pragma unroll
+                for (int q = 0; q < FN; ++q)
+                    rest[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(t[i], b[q], rest[q], 0, 0, 0);
+        } else {
+            uint2 h0, l0, h1, l1;
+            split_bf16x4(__builtin_bit_cast(float4, x0), h0, l0);
+            split_bf16x4(__builtin_bit_cast(float4, x1), h1, l1);
+            const bf16x8 ah = __builtin_bit_cast(bf16x8, make_uint4(h0.x, h0.y, h1.x, h1.y));
+            const bf16x8 al = __builtin_bit_cast(bf16x8, make_uint4(l0.x, l0.y, l1.x, l1.y));
+#pragma unroll
+            for (int q = 0; q < FN; ++q) acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, b[q], acc[q], 0, 0, 0);
+#pragma unroll
+            for (int q = 0; q < FN; ++q) acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, b[q], acc[q], 0, 0, 0);
+        }
     }
+    if constexpr (RAGGED)
+#pragma unroll
+        for (int q = 0; q < FN; ++q) acc[q] += rest[q];
     // The second half's sums, through the ring (free once every wave is here).
     f32x4(*ep)[FN][64] = reinterpret_cast<f32x4(*)[FN][64]>(&ring[0]);
     static_assert(sizeof(ring) >= sizeof(f32x4) * (T::BM / 16) * FN * 64, "the sums fit the ring");
@@ -738,8 +770,12 @@ __global__ __launch_bounds__(kF32Threads, 2) void gemm_f32_kernel(int gxy, int r
         const f32x4 s = acc[q] + ep[wave][q][lane];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const int t = t0 + wm + fq * 4 + i;
-            if (t < n) out[(size_t)t * rows + sg.local + q * 16 + fr] = s[i];
+            const int t = t0 + wm + fq * 4 + i, r = q * 16 + fr;
+            if (t >= n || (RAGGED && sg.local + r >= rows)) continue;
+            float v = s[i];
+            if (RAGGED && __builtin_expect(v != v, 0))
+                v = plain_dot(w + (size_t)r * cols, xk + (size_t)t * cols, 0, min(nk * T::BK, cols - kb * T::BK));
+            out[(size_t)t * rows + sg.local + r] = v;
         }
     }
 }
@@ -1123,8 +1159,42 @@ hipError_t launch_gemm_f32(hipStream_t s, const float *x, size_t n, size_t cols,
     const size_t tx = total / Small::BN, ty = (n + Small::BM - 1) / Small::BM;
     if (tx > 0xffff || ty > 0xffff || n > ((size_t)1 << 24)) return hipErrorInvalidValue;
     const dim3 grid((unsigned)tx, (unsigned)ty, (unsigned)ksplit);
-    gemm_f32_kernel<<<grid, kF32Threads, 0, s>>>((int)(tx | ty << 16), sg.rows[0], sg.w[0], sg.out[0], x, (int)n,
+    gemm_f32_kernel<2><<<grid, kF32Threads, 0, s>>>((int)(tx | ty << 16), sg.rows[0], sg.w[0], sg.out[0], x, (int)n,
                                                (int)cols, ksplit, part, sg);
+    return hipGetLastError();
+}
+
+bool gemm_ragged_supported(size_t n, size_t rows, size_t cols) {
+    return rows >= 1 && cols >= 8 && cols % 8 == 0 && cols < ((size_t)1 << 24) && n <= ((size_t)1 << 20) &&
+           (rows + Small::BN - 1) / Small::BN <= 0xffff;
+}
+
+int gemm_ragged_ksplit(size_t n, size_t rows, size_t cols) {
+    const size_t up = (rows + Small::BN - 1) / Small::BN * Small::BN, steps = (cols + BK - 1) / BK * BK;
+    return small_ksplit(n, up, steps);
+}
+
+double gemm_ragged_us(size_t n, size_t rows, size_t cols, int ksplit) {
+    // Rounds of two blocks a CU (or one) times their K steps, as measured.
+    const size_t blocks = tiles_of(rows, Small::BN) * tiles_of(n, Small::BM) * (size_t)ksplit;
+    const double step = blocks <= 256 ? 0.6 : (double)((blocks + 511) / 512);
+    return 3 + step * (double)tiles_of(cols, BK * (size_t)ksplit) + (ksplit > 1 ? 3.5 : 0);
+}
+
+hipError_t launch_gemm_ragged(hipStream_t s, const float *x, size_t n, size_t cols, const uint16_t *w, size_t rows,
+                              float *out, float *part, int ksplit) {
+    if (n == 0) return hipSuccess;
+    if (!gemm_ragged_supported(n, rows, cols) || ((uintptr_t)x | (uintptr_t)w) % 16 || ksplit < 1 ||
+        (ksplit > 1 && !part) || (size_t)ksplit > (cols + BK - 1) / BK)
+        return hipErrorInvalidValue;
+    Segs sg{};
+    sg.n = 1;
+    sg.w[0] = w;
+    sg.out[0] = out;
+    sg.rows[0] = (int)rows;
+    const unsigned tx = (unsigned)((rows + Small::BN - 1) / Small::BN), ty = (unsigned)((n + Small::BM - 1) / Small::BM);
+    gemm_f32_kernel<3><<<dim3(tx, ty, (unsigned)ksplit), kF32Threads, 0, s>>>((int)(tx | ty << 16), (int)rows, w, out, x,
+                                                                             (int)n, (int)cols, ksplit, part, sg);
     return hipGetLastError();
 }
 

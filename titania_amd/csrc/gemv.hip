@@ -121,10 +121,20 @@ hipError_t launch_matmul(hipStream_t s, float *out, const uint16_t *w, size_t ro
         }
         return hipSuccess;
     }
+    // The partials' room and their sum's 16-byte chunks.
+    auto fits = [&](int k) { return part && n * rows % 4 == 0 && (size_t)k * n * rows <= kPartFloats; };
     int ksplit = n < kGemmMinTokens ? few_ksplit(n, rows, cols) : 1;
-    if (!part || n * rows % 4 || (size_t)ksplit * n * rows > kPartFloats) ksplit = 1;
+    if (!fits(ksplit)) ksplit = 1;
+    bool ragged = false;
+    if (n > 16 && gemm_ragged_supported(n, rows, cols) && !gemm_supported(rows, cols)) {
+        int k = gemm_ragged_ksplit(n, rows, cols);
+        if (!fits(k)) k = 1;
+        ragged = gemm_ragged_us(n, rows, cols, k) + 2 < few_us(n, rows, cols);
+        if (ragged) ksplit = k;
+    }
     const GemmOut o{w, rows, out};
-    const hipError_t e = launch_few(s, x, n, cols, &o, 1, part, ksplit);
+    const hipError_t e = ragged ? launch_gemm_ragged(s, x, n, cols, w, rows, out, part, ksplit)
+                                : launch_few(s, x, n, cols, &o, 1, part, ksplit);
     if (e != hipSuccess || ksplit == 1) return e;
     return launch_splitk_sum(s, part, out, n * rows, ksplit);
 }
