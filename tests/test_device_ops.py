@@ -347,6 +347,27 @@ def test_ragged_matmul(hip, rows, cols, n):
     assert np.all(np.abs(got - exp) <= cols * 2.0**-24 * size)
 
 
+@pytest.mark.parametrize("n", [4, 15, 50, 70])
+def test_few_token_matmul_not_finite(hip, n):
+    """Infinite and NaN weights and activations give what their products and
+    sums in f32 give."""
+    rows, cols = 100, 1096
+    rng = np.random.default_rng(n)
+    wf = bf16_to_f32(normal_bf16(rows * cols, 6, "inf", 0.05)).reshape(rows, cols).copy()
+    x = np.round(rng.standard_normal((n, cols)).astype(np.float32) * 4) / 4 + np.float32(0.125)  # no zero; bf16 exactly
+    wf[3, 700], wf[5, 10], wf[7, 900], wf[7, 30] = np.inf, -np.inf, np.inf, np.nan
+    x[1, 200], x[2, 1095] = np.inf, np.uint32(0x7f800001).view(np.float32)  # a NaN of low bits only
+    with np.errstate(invalid="ignore"):
+        exp = (wf[None].astype(np.float64) * x[:, None].astype(np.float64)).sum(-1)
+    bx, out = hip.alloc(x.size), hip.alloc(n * rows)
+    hip.write(bx, x)
+    hip.matmul(out, hip.upload(Tensor((rows, cols), f32_to_bf16(wf.reshape(-1)))), bx)
+    got = hip.read(out).reshape(n, rows).astype(np.float64)
+    assert np.array_equal(np.isnan(got), np.isnan(exp))
+    infinite = np.isinf(exp)
+    assert np.array_equal(got[infinite], exp[infinite]) and np.all(np.isfinite(got[np.isfinite(exp)]))
+
+
 @pytest.mark.parametrize("rows,cols,n", [(6144, 1024, 2000), (4096, 6144, 1024), (6144, 512, 8000),
                                          (2560, 1024, 8000)])
 def test_large_tile_gemm(hip, rows, cols, n):
