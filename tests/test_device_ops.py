@@ -333,7 +333,7 @@ def test_ragged_matmul(hip, rows, cols, n):
     """More than a few tokens of matrices that are not whole tiles: rows and
     columns past a tile's edge by one row or chunk, K split or not, tokens
     past a tile. Three bf16 terms are x exactly; the f32 sums add cols * 2^-24
-    of sum |w x| at most. Rows past the output stay as they were."""
+    of sum |w x| at most."""
     rng = np.random.default_rng(rows + cols + n)
     w = normal_bf16(rows * cols, 5, "ragged", 0.05)
     x = rng.standard_normal((n, cols)).astype(np.float32)
