@@ -292,9 +292,14 @@ def test_tiny8_decode_crossing(tiny8, decode_mode, n, steps, max_len, kv):
                                                 (2043, 8, 2070, TH_KV_BF16)])
 def test_tiny8_forward_one_token(tiny8, monkeypatch, n, steps, max_len, kv):
     """A forward of one token runs a decode step's kernels: fed the tokens of a
-    decode, it returns the decode's logits bit for bit, through the chunked
-    launch, the streaming one and the step between them, with a decode call in
-    the middle and one that follows picking from the logits it left."""
+    decode, it returns the decode's logits (over f32 caches bit for bit; over
+    bf16 ones a decode step attends to its new key and value in f32, a forward
+    to what the caches hold), through the chunked launch, the streaming one
+    and the step between them, with a decode call in the middle and one that
+    follows picking from the logits it left."""
+    def agree(x, y):
+        return np.array_equal(x, y) if kv == TH_KV_F32 else float(np.max(np.abs(x - y))) <= LOGIT_TOL
+
     monkeypatch.setenv("TITANIA_DECODE", "eager")  # chooses the launch step by step, as the forward does
     m, _ = tiny8
     prompt = synth.prompt(n, QWEN3_TINY8.vocab_size, seed=n)
@@ -303,11 +308,31 @@ def test_tiny8_forward_one_token(tiny8, monkeypatch, n, steps, max_len, kv):
     m.forward(b, prompt, 0, TH_PATH_FUSED, want_logits=False)
     toks, logits = m.decode(a, n, steps, keep_logits=True)
     for i in range(steps - 2):
-        assert np.array_equal(m.forward(b, [int(toks[i])], n + i, TH_PATH_FUSED), logits[i]), f"step {i}"
+        assert agree(m.forward(b, [int(toks[i])], n + i, TH_PATH_FUSED), logits[i]), f"step {i}"
     assert list(m.decode(b, n + steps - 2, 1)) == [toks[steps - 2]]
-    assert np.array_equal(m.forward(b, [int(toks[-1])], n + steps - 1, TH_PATH_FUSED), logits[-1])
+    assert agree(m.forward(b, [int(toks[-1])], n + steps - 1, TH_PATH_FUSED), logits[-1])
     with pytest.raises(InvalidArgument, match="vocabulary"):
         m.forward(b, [QWEN3_TINY8.vocab_size], 0, TH_PATH_FUSED)
+    a.close()
+    b.close()
+
+
+@pytest.mark.parametrize("n,max_len", [(0, 16), (1, 16), (0, 9000)])
+def test_tiny8_forward_one_token_bf16(tiny8, n, max_len):
+    """A forward of one token attends to its new key and value as a bf16 cache
+    holds them, as a forward of several does, in states of one chunk and of
+    many. Where every token is the same, so is every value, and
+    the attention's result at any position is that value: the logits equal
+    those of two tokens. A value taken in f32 differs by up to 2^-9 in every
+    element, one rounded the other way by 2^-8 in one of 1024 (1.2e-4 of the
+    result, and less of the logits)."""
+    m, _ = tiny8
+    a, b = State(m, max_len, TH_KV_BF16), State(m, max_len, TH_KV_BF16)
+    want = m.forward(a, [7, 7], 0, TH_PATH_FUSED)
+    if n:
+        m.forward(b, [7] * n, 0, TH_PATH_FUSED, want_logits=False)
+    got = m.forward(b, [7], n, TH_PATH_FUSED)
+    assert float(np.linalg.norm(got - want)) <= 1e-4 * float(np.linalg.norm(want))
     a.close()
     b.close()
 

@@ -403,8 +403,9 @@ bool step_dual(const th_state *s) {
 // Queues one decode step with the fused step kernels: the token and position
 // come from s->step, the picked token goes back there. `chunked`: the q/k/v +
 // attention take the chunked launch, where the state allows it (step_chunked
-// for a short context), or else the streaming one. Without `pick` it ends
-// with the logits.
+// for a short context), or else the streaming one. Without `pick`, a
+// forward's step: it ends with the logits, and takes the new keys and values
+// as the caches hold them.
 int enqueue_step(th_state *s, bool chunked, bool pick = true) {
     th_model *m = s->m;
     hipStream_t st = m->dev->stream;
@@ -465,6 +466,7 @@ int enqueue_step(th_state *s, bool chunked, bool pick = true) {
         a.n_kv_heads = nkv;
         a.nsplit = fuse_attn ? 1 : nsplit;
         a.kv_bf16 = s->kv_dtype == TH_KV_BF16;
+        a.round_new = !pick;
         a.eps = eps;
         a.out = s->s_att;
         a.part_acc = s->attn_part;

@@ -64,6 +64,9 @@ struct StepAttnArgs {
     int n_heads, n_kv_heads;
     int nsplit;
     int kv_bf16;
+    // bf16 caches: attend to the new key and value as the caches will hold
+    // them, as a forward does (a decode step takes them in f32).
+    int round_new;
     float eps;
     float *out;       // [n_heads][head_dim] when nsplit == 1
     float *part_acc;  // [n_heads][nsplit][head_dim] otherwise

@@ -17,6 +17,14 @@ namespace th {
 
 namespace {
 
+// A new key's or value's element as the step attends to it: as a bf16 cache
+// will hold it (StepAttnArgs::round_new), or in f32.
+template <typename KV>
+__device__ __forceinline__ float as_kept(float v, int round) {
+    if constexpr (sizeof(KV) == 2) return round ? bf16_to_f32(f32_to_bf16(v)) : v;
+    return v;
+}
+
 constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / 64;
 
@@ -499,7 +507,7 @@ __device__ __forceinline__ void attend_stream(const StepAttnArgs &a, int g, int 
             }
         }
     }
-    if (tid < HD) hv[tid] = vnew;
+    if (tid < HD) hv[tid] = as_kept<KV>(vnew, a.round_new);
     // RMSNorm (model.rs:111-116) + RoPE (model.rs:117-118), one head a wave.
 #pragma unroll
     for (int hh = 0; hh < HPW; ++hh) {
@@ -513,8 +521,9 @@ __device__ __forceinline__ void attend_stream(const StepAttnArgs &a, int g, int 
             x1 = x1 * (sc * bf16_to_f32(EARLY ? g16b[hh] : (uint16_t)grb[hh]));
         }
         float *x = h < G ? hq + h * HD : hk;
-        x[lane] = x0 * cs.x - x1 * cs.y;
-        x[lane + HALF] = x1 * cs.x + x0 * cs.y;
+        const int round = h < G ? 0 : a.round_new;
+        x[lane] = as_kept<KV>(x0 * cs.x - x1 * cs.y, round);
+        x[lane + HALF] = as_kept<KV>(x1 * cs.x + x0 * cs.y, round);
     }
     __syncthreads();
     // The lane's dims of q, scaled into the base-2 domain: scores come out as
@@ -784,11 +793,12 @@ __device__ __forceinline__ void attend_wave4(const StepAttnArgs &a, int g, int h
                 x0 = x0 * (sc * (wave == 0 ? gq0 : gk0));
                 x1 = x1 * (sc * (wave == 0 ? gq1 : gk1));
             }
-            dst[lane] = x0 * cs.x - x1 * cs.y;
-            dst[lane + HALF] = x1 * cs.x + x0 * cs.y;
+            const int round = wave == 0 ? 0 : a.round_new;
+            dst[lane] = as_kept<KV>(x0 * cs.x - x1 * cs.y, round);
+            dst[lane + HALF] = as_kept<KV>(x1 * cs.x + x0 * cs.y, round);
         } else {
-            dst[lane] = x0;
-            dst[lane + HALF] = x1;
+            dst[lane] = as_kept<KV>(x0, a.round_new);
+            dst[lane + HALF] = as_kept<KV>(x1, a.round_new);
         }
     }
     __syncthreads();
