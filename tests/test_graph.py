@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 
 from oracle import ref
-from titania_amd import Tensor
+from titania_amd import Hip, Sampler, Tensor
 from titania_amd.synth import bf16_to_f32, normal_bf16
 
 pytestmark = pytest.mark.gpu
@@ -103,3 +103,40 @@ def test_capture_refuses_host_and_allocating_calls(hip):
     assert np.array_equal(hip.read(b), np.arange(16, dtype=np.float32))
     graph.free()
     b.free()
+
+
+def test_graph_survives_scratch_growth():
+    """A replay writes its attention partials where it did when it was
+    captured (one token of 16 heads at position 500: 16640 floats), so that
+    memory stays the device's own when a later call needs more scratch (a
+    sample over 151936 values: 76 KB): replays give the eager result, and
+    leave alone buffers allocated since, which would take a freed block's
+    place."""
+    pos, vocab, part = 500, 151936, 16 * 8 * 130
+    data = _inputs()
+    dev = Hip(0)
+    k, v = (dev.alloc((pos + 1) * KVH * HD) for _ in range(2))
+    q, out, logits = dev.alloc(H * HD), dev.alloc(H * HD), dev.alloc(vocab)
+    dev.write(q, data["q"])
+    dev.write(k, data["k"][:(pos + 1) * KVH * HD])
+    dev.write(v, data["v"][:(pos + 1) * KVH * HD])
+    dev.attention(out, q, k, v, pos, H, HD, KVH)
+    want = dev.read(out)
+    dev.graph_begin()
+    try:
+        dev.attention(out, q, k, v, pos, H, HD, KVH)
+    finally:
+        graph = dev.graph_end()
+    dev.sample(logits, Sampler(0.7, 20, 0.8, 1))
+    others = [dev.alloc(n) for n in (part, part, part + 256, 2 * part, 4 * part)]
+    for replay in range(3):
+        for b in others:
+            dev.write(b, np.full(len(b), 3.0, np.float32))
+        dev.write(out, np.zeros(H * HD, np.float32))
+        graph.launch()
+        assert np.array_equal(dev.read(out), want), f"replay {replay}"
+        assert all(np.all(dev.read(b) == 3.0) for b in others), f"replay {replay}"
+    graph.free()
+    for b in others + [k, v, q, out, logits]:
+        b.free()
+    dev.close()

@@ -21,6 +21,13 @@ struct th_device {
     // demand outside graph capture.
     void *scratch = nullptr;
     size_t scratch_bytes = 0;
+    // Scratch that was outgrown after a capture: graphs hold its address, so it
+    // is kept for the device's life. Each block is at least twice the one
+    // before, so together they are smaller than the current one.
+    void *outgrown[64] = {};
+    int n_outgrown = 0;
+    // A graph has been captured on this device's stream.
+    bool captured = false;
     // The device address of the no-alloc entry points' fixed array (looked up
     // once, at th_device_create, with this device current).
     void *noalloc_scratch = nullptr;

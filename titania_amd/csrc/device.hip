@@ -40,6 +40,14 @@ void *scratch(th_device *dev, size_t bytes) {
     }
     size_t want = std::max(bytes, dev->scratch_bytes * 2);
     want = (want + 255) & ~(size_t)255;
+    if (dev->scratch && dev->captured) {
+        void *block = nullptr;
+        if (hipMalloc(&block, want) != hipSuccess) return nullptr;
+        dev->outgrown[dev->n_outgrown++] = dev->scratch;
+        dev->scratch = block;
+        dev->scratch_bytes = want;
+        return block;
+    }
     if (dev->scratch) {
         if (hipStreamSynchronize(dev->stream) != hipSuccess) return nullptr;
         (void)hipFree(dev->scratch);
@@ -146,6 +154,7 @@ void th_device_destroy(th_device *dev) {
     if (dev->stream) (void)hipStreamSynchronize(dev->stream);
     if (dev->tokens) (void)hipFree(dev->tokens);
     if (dev->scratch) (void)hipFree(dev->scratch);
+    for (int i = 0; i < dev->n_outgrown; ++i) (void)hipFree(dev->outgrown[i]);
     if (dev->token_out) (void)hipFree(dev->token_out);
     if (dev->part) (void)hipFree(dev->part);
     if (dev->pinned) (void)hipHostFree(dev->pinned);
@@ -166,6 +175,7 @@ int th_graph_begin(th_device *dev) {
     TH_HIP(hipSetDevice(dev->ordinal));
     TH_HIP(hipStreamBeginCapture(dev->stream, hipStreamCaptureModeThreadLocal));
     dev->capturing = true;
+    dev->captured = true;
     return TH_OK;
 }
 
