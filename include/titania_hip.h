@@ -89,10 +89,11 @@ TH_API int th_rope(th_device *dev, th_buffer *x, const th_buffer *table, size_t 
 TH_API int th_attention(th_device *dev, th_buffer *out, const th_buffer *q, const th_buffer *k_cache,
                  const th_buffer *v_cache, size_t pos, size_t n_heads, size_t head_dim, size_t n_kv_heads);
 /* th_attention without any allocation: its split partials go to a fixed
- * 16 MiB array that the library holds on each GPU until the process ends, so
- * that callers that cannot allocate (code under HIP graph capture, tight
- * serving loops, harnesses that forbid hipMalloc) can call it. No counterpart
- * in model/device.rs. Same arguments, checks and results as th_attention; a
+ * 16 MiB array that the library holds on each GPU until the process ends (those
+ * of several tokens after a context at least as long to a block that the
+ * device handle holds), so that callers that cannot allocate (code under HIP
+ * graph capture, tight serving loops, harnesses that forbid hipMalloc) can
+ * call it. No counterpart in model/device.rs. Same arguments, checks and results as th_attention; a
  * call whose partials need more than 16 MiB (n * n_heads * splits *
  * (head_dim + 2) floats, at most 256 splits for one token: one token of up to
  * 126 heads of head_dim 128 at any context fits, a 2048-token prompt of 32

@@ -13,7 +13,7 @@ import numpy as np
 import pytest
 
 from oracle import ref
-from titania_amd import InvalidArgument
+from titania_amd import Hip, InvalidArgument
 from titania_amd._lib import check, lib
 from titania_amd.synth import bf16_to_f32, normal_bf16
 from util import rel_error
@@ -64,3 +64,31 @@ def test_noalloc_refuses_oversized_partials(hip):
     k, v, q, out = hip.alloc(ctx * KVH * hd), hip.alloc(ctx * KVH * hd), hip.alloc(n * H * hd), hip.alloc(n * H * hd)
     with pytest.raises(InvalidArgument, match="fixed"):
         hip.attention_noalloc(out, q, k, v, ctx - n, H, hd, KVH)
+
+
+@pytest.mark.parametrize("n,ctx,H,KVH", [(64, 32064, 16, 8), (64, 20000, 32, 8), (12, 600, 16, 8)])
+def test_noalloc_and_captured_splits_are_eager(n, ctx, H, KVH):
+    """Several tokens after a longer context, whose splits need more than the
+    fixed array (the first two) or than the device's scratch: th_attention,
+    th_attention_noalloc and a capture on a device that has grown no scratch
+    for it give the same bits."""
+    dev = Hip(0)
+    rng = np.random.default_rng(n)
+    k, v, q = (dev.alloc(ctx * KVH * 128), dev.alloc(ctx * KVH * 128), dev.alloc(n * H * 128))
+    for b in (k, v, q):
+        dev.write(b, rng.standard_normal(len(b), dtype=np.float32))
+    outs = [dev.alloc(len(q)) for _ in range(3)]
+    dev.attention_noalloc(outs[0], q, k, v, ctx - n, H, 128, KVH)
+    dev.graph_begin()
+    try:
+        dev.attention(outs[1], q, k, v, ctx - n, H, 128, KVH)
+    finally:
+        graph = dev.graph_end()
+    graph.launch()
+    dev.attention(outs[2], q, k, v, ctx - n, H, 128, KVH)
+    got = [dev.read(b).view(np.uint32) for b in outs]
+    assert np.array_equal(got[0], got[2]) and np.array_equal(got[1], got[2])
+    graph.free()
+    for b in outs + [k, v, q]:
+        b.free()
+    dev.close()

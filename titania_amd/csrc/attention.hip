@@ -617,12 +617,8 @@ int attention_splits(size_t n, size_t n_heads, size_t n_kv_heads, size_t max_len
     return (int)std::max<size_t>(1, std::min<size_t>(s, 256));
 }
 
-size_t attention_splits_scratch(size_t n, size_t n_heads, size_t max_len, size_t head_dim) {
-    const size_t ns = std::min<size_t>(kMaxRoundSplits, (max_len + kGqaKeys - 1) / kGqaKeys);
-    return std::min(n * n_heads * ns, kMaxRoundBlocks * kGqaRows) * (head_dim + 2);
-}
-
-int attention_splits_at(size_t n, size_t n_heads, size_t n_kv_heads, size_t pos, size_t head_dim, size_t floats) {
+int attention_splits_at(size_t n, size_t n_heads, size_t n_kv_heads, size_t pos, size_t head_dim, bool *by_rounds) {
+    if (by_rounds) *by_rounds = false;
     const int least = attention_splits(n, n_heads, n_kv_heads, pos + n, head_dim);
     const size_t group = n_kv_heads ? n_heads / n_kv_heads : 0;
     if (head_dim != 128 || n < kAttnTileMin || pos < n || group < 1 || group > 8 || 8 % group ||
@@ -645,7 +641,9 @@ int attention_splits_at(size_t n, size_t n_heads, size_t n_kv_heads, size_t pos,
             ns = k;
         }
     }
-    return attention_scratch(n, n_heads, head_dim, (int)ns) <= floats ? (int)ns : least;
+    static_assert(kMaxRoundBlocks * kGqaRows * (128 + 2) <= kAttnRoundFloats, "the partials fit");
+    if (by_rounds) *by_rounds = true;
+    return (int)ns;
 }
 
 size_t attention_scratch(size_t n, size_t n_heads, size_t head_dim, int nsplit) {

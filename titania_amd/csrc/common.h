@@ -31,9 +31,11 @@ struct th_device {
     // The device address of the no-alloc entry points' fixed array (looked up
     // once, at th_device_create, with this device current).
     void *noalloc_scratch = nullptr;
-    // Split-K partials of a matmul: th::kPartFloats, for the device's life (a
-    // matmul of fewer than 16 tokens allocates nothing, so that it can be
-    // captured, and an allocation costs more than most matmuls).
+    // Split-K partials of a matmul (th::kPartFloats) and partials of an
+    // attention split by rounds (th::kAttnRoundFloats), for the device's life:
+    // calls that allocate nothing (a matmul of fewer than 16 tokens, so that
+    // it can be captured; th_attention_noalloc) then split like any other, and
+    // an allocation costs more than most matmuls.
     float *part = nullptr;
     // One u32 the argmax kernels leave their result in.
     uint32_t *token_out = nullptr;
@@ -173,20 +175,19 @@ struct AttnKernelArgs {
 // Splits of the sequence for n tokens (of head_dim) whose contexts reach at
 // most max_len.
 int attention_splits(size_t n, size_t n_heads, size_t n_kv_heads, size_t max_len, size_t head_dim);
-// Splits for n tokens at position pos, where the partials may take `floats`
-// floats. Several tokens after a context at least as long see about the same
-// number of 64-key tiles each, and a CU holds one block of the matrix-core
-// kernels, so the launch takes its rounds of 256 blocks times the tiles a
-// block walks, and the combine (us with attention_splits -> these: 11 tokens
-// at 700 of 32 / 8 heads 18.7 -> 11.8, at 4000 38.2 -> 20.0; 64 at 30000 of 16
-// / 8 222.7 -> 80.3; 300 at 2000 of 32 / 8 70.7 -> 55.4). The estimate counts
-// tiles of 3.3 us: two more a round to start and end it, 1.4 and the partials'
-// bytes for the combine. Others, and partials that do not fit, as
-// attention_splits.
-int attention_splits_at(size_t n, size_t n_heads, size_t n_kv_heads, size_t pos, size_t head_dim, size_t floats);
-// Scratch floats that attention_splits_at's partials take at most for up to n
-// tokens and contexts up to max_len.
-size_t attention_splits_scratch(size_t n, size_t n_heads, size_t max_len, size_t head_dim);
+// Splits for n tokens at position pos. Several tokens after a context at least
+// as long see about the same number of 64-key tiles each, and a CU holds one
+// block of the matrix-core kernels, so the launch takes its rounds of 256
+// blocks times the tiles a block walks, and the combine (us with
+// attention_splits -> these: 11 tokens at 700 of 32 / 8 heads 18.7 -> 11.8, at
+// 4000 38.2 -> 20.0; 64 at 30000 of 16 / 8 222.7 -> 80.3; 300 at 2000 of 32 / 8
+// 70.7 -> 55.4). The estimate counts tiles of 3.3 us: two more a round to start
+// and end it, 1.4 and the partials' bytes for the combine. Others as
+// attention_splits. *by_rounds, if not null: whether they are such a count,
+// whose partials take at most kAttnRoundFloats.
+int attention_splits_at(size_t n, size_t n_heads, size_t n_kv_heads, size_t pos, size_t head_dim,
+                        bool *by_rounds = nullptr);
+constexpr size_t kAttnRoundFloats = (size_t)1024 * 128 * (128 + 2);  // 1024 blocks of 128 rows, head_dim 128
 // Scratch floats the partials of `nsplit` splits take (0 for one split).
 size_t attention_scratch(size_t n, size_t n_heads, size_t head_dim, int nsplit);
 hipError_t launch_attention(hipStream_t s, const AttnKernelArgs &k, size_t n, size_t head_dim);

@@ -129,7 +129,8 @@ int th_device_create(int ordinal, th_device **out) {
     }
     hipError_t e = hipStreamCreateWithFlags(&dev->stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipMalloc(&dev->token_out, 256);
-    if (e == hipSuccess) e = hipMalloc(&dev->part, th::kPartFloats * sizeof(float));
+    if (e == hipSuccess)
+        e = hipMalloc(&dev->part, std::max(th::kPartFloats, th::kAttnRoundFloats) * sizeof(float));
     if (e == hipSuccess)
         e = hipHostMalloc(reinterpret_cast<void **>(&dev->pinned),
                           th::kPinnedFloats * sizeof(float) + th::kPinnedTokens * sizeof(uint32_t), hipHostMallocDefault);
@@ -454,24 +455,24 @@ int attention(th_device *dev, th_buffer *out, const th_buffer *q, const th_buffe
     TH_REQUIRE(k_cache->len >= (pos + n) * kv_dim && v_cache->len >= (pos + n) * kv_dim,
                "the caches do not hold position %zu", pos + n - 1);
     TH_REQUIRE(out->ptr != q->ptr, "attention cannot write its queries");
-    // Calls that cannot grow their scratch are refused by what
-    // attention_splits needs, and split further only within what there is.
-    const size_t room = fixed ? th::noalloc_scratch_bytes() / sizeof(float)
-                        : dev->capturing ? dev->scratch_bytes / sizeof(float) : SIZE_MAX;
-    int nsplit = th::attention_splits(n, n_heads, n_kv_heads, pos + n, head_dim);
-    if (th::attention_scratch(n, n_heads, head_dim, nsplit) <= room)
-        nsplit = th::attention_splits_at(n, n_heads, n_kv_heads, pos, head_dim, room);
-    const size_t floats = th::attention_scratch(n, n_heads, head_dim, nsplit);
+    // Counts by rounds have their partials in the device's own block, so that
+    // every caller takes the same ones (and gives the same bits). The no-alloc
+    // form is refused by what attention_splits' count needs, whichever is taken.
+    bool by_rounds = false;
+    const int nsplit = th::attention_splits_at(n, n_heads, n_kv_heads, pos, head_dim, &by_rounds);
+    const size_t floats = th::attention_scratch(
+        n, n_heads, head_dim, th::attention_splits(n, n_heads, n_kv_heads, pos + n, head_dim));
     float *scr = nullptr;
     if (floats && fixed) {
         TH_REQUIRE(floats * sizeof(float) <= th::noalloc_scratch_bytes(),
                    "th_attention_noalloc: %zu bytes of split partials exceed its fixed %zu-byte scratch",
                    floats * sizeof(float), th::noalloc_scratch_bytes());
         scr = static_cast<float *>(dev->noalloc_scratch);
-    } else if (floats) {
+    } else if (floats && !by_rounds) {
         scr = static_cast<float *>(th::scratch(dev, floats * sizeof(float)));
         if (!scr) return fail(TH_ERR_NOMEM, "no scratch for attention (%zu floats)", floats);
     }
+    if (by_rounds) scr = dev->part;
     th::AttnKernelArgs a{};
     a.out = out->ptr;
     a.q = q->ptr;

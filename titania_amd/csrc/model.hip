@@ -324,10 +324,6 @@ int ensure_fused_state(th_state *s) {
         s->attn_part_floats =
             std::max(s->attn_part_floats, th::attention_scratch(n, (size_t)c.num_attention_heads, hd, ns));
     }
-    if (hd == 128)
-        s->attn_part_floats =
-            std::max(s->attn_part_floats,
-                     th::attention_splits_scratch(s->fb, (size_t)c.num_attention_heads, s->max_len, hd));
     if (s->attn_part_floats) TH_HIP(hipMalloc(&s->attn_part, s->attn_part_floats * sizeof(float)));
     if (s->kv_dtype == TH_KV_F32 && s->fb >= th::kGemmMinTokens && hd == 128) {
         s->kv_planes_bytes = th::attention_planes_bytes(s->max_len, (size_t)c.num_key_value_heads);
@@ -534,9 +530,11 @@ int enqueue_fused(th_state *s, const uint32_t *tokens, size_t n, size_t pos, con
     const size_t qd = nh * hd;
     const int kv_bf16 = s->kv_dtype == TH_KV_BF16;
     const size_t max_ctx = pos_dev ? s->max_len : pos + n;
+    bool by_rounds = false;
     const int nsplit = pos_dev ? th::attention_splits(n, nh, nkv, max_ctx, hd)
-                               : th::attention_splits_at(n, nh, nkv, pos, hd, s->attn_part_floats);
-    if (th::attention_scratch(n, nh, hd, nsplit) > s->attn_part_floats)
+                               : th::attention_splits_at(n, nh, nkv, pos, hd, &by_rounds);
+    float *attn_part = by_rounds ? d->part : s->attn_part;
+    if (!by_rounds && th::attention_scratch(n, nh, hd, nsplit) > s->attn_part_floats)
         return fail(TH_ERR_INVALID, "attention partials exceed the state's scratch");
     // Chunks of kGemmMinTokens or more go through the MFMA GEMM (activations
     // split once per input into fsplit).
@@ -640,8 +638,8 @@ int enqueue_fused(th_state *s, const uint32_t *tokens, size_t n, size_t pos, con
         aa.nsplit = nsplit;
         aa.kv_bf16 = kv_bf16;
         aa.scale = 1.0f / sqrtf((float)hd);
-        aa.part_acc = s->attn_part;
-        aa.part_ml = s->attn_part ? s->attn_part + n * nh * (size_t)nsplit * hd : nullptr;
+        aa.part_acc = attn_part;
+        aa.part_ml = attn_part ? attn_part + n * nh * (size_t)nsplit * hd : nullptr;
         if (hl) {
             aa.out_hi = hi;
             aa.out_lo = lo;

@@ -379,7 +379,7 @@ int th_test_attention_prefill(th_device *dev, const th_buffer *q, const th_buffe
     a.pos = (long long)pos;
     a.pos_stride = (long long)hd;
     a.head_stride = (long long)(max_len * hd);
-    a.nsplit = th::attention_splits_at(n, n_heads, n_kv_heads, pos, hd, SIZE_MAX);
+    a.nsplit = th::attention_splits_at(n, n_heads, n_kv_heads, pos, hd);
     a.kv_bf16 = 0;
     a.scale = 1.0f / sqrtf((float)hd);
     DevMem part, pl;
