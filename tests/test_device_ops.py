@@ -368,6 +368,36 @@ def test_few_token_matmul_not_finite(hip, n):
     assert np.array_equal(got[infinite], exp[infinite]) and np.all(np.isfinite(got[np.isfinite(exp)]))
 
 
+@pytest.mark.parametrize("n,rows,cols", [(12, 9728, 2560), (40, 5003, 2968)])
+def test_few_token_matmul_not_finite_time(hip, n, rows, cols):
+    """Inputs that make every result NaN take no more than a pass over each
+    tile's weights and each wave's activations again: about 5 times the finite
+    call, where summing each NaN one by one took 40 to 140 times it."""
+    w = hip.upload(Tensor((rows, cols), normal_bf16(rows * cols, 6, "inf", 0.05)))
+    x = np.random.default_rng(n).standard_normal((n, cols)).astype(np.float32)
+    bx, out = hip.alloc(x.size), hip.alloc(n * rows)
+
+    def ms():
+        best = []
+        for _ in range(8):
+            hip.timer_begin()
+            for _ in range(4):
+                hip.matmul(out, w, bx)
+            best.append(hip.timer_end())
+        return min(best)
+
+    hip.write(bx, x)
+    finite = ms()
+    x[:, 7] = np.nan
+    hip.write(bx, x)
+    nan = ms()
+    assert np.all(np.isnan(hip.read(out)))
+    x[:, 7], x[:, 9] = np.inf, -np.inf
+    hip.write(bx, x)
+    inf = ms()
+    assert nan < 15 * finite and inf < 15 * finite
+
+
 @pytest.mark.parametrize("rows,cols,n", [(6144, 1024, 2000), (4096, 6144, 1024), (6144, 512, 8000),
                                          (2560, 1024, 8000)])
 def test_large_tile_gemm(hip, rows, cols, n):

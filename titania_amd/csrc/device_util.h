@@ -193,13 +193,91 @@ __device__ __forceinline__ void split3(const uint4 &a, const uint4 &b, bf16_term
     }
 }
 
-// Columns [c0, c1) of w . x one by one: for a sum of split3 terms' products
-// that is NaN, as a later term of zero times an infinite weight is where x w
-// is infinite.
-__device__ __forceinline__ float plain_dot(const uint16_t *w, const float *x, int c0, int c1) {
-    float s = 0.f;
-    for (int c = c0; c < c1; ++c) s = fmaf(bf16_to_f32(w[c]), x[c], s);
-    return s;
+// Whether one of the word's two bf16 is infinite.
+__device__ __forceinline__ int has_inf_bf16(uint32_t u) {
+    return ((u & 0x7fffu) == 0x7f80u) | ((u >> 16 & 0x7fffu) == 0x7f80u);
+}
+
+// Sums of split3 terms' products, 16 rows x 16 tokens a wave (lane (fq, fr):
+// tokens 4 fq + i of row fr): those that are NaN become the f32 products' sums
+// of columns [c0, c1) (whole 8s), since a later term of zero times an infinite
+// weight is NaN where x w is infinite. Only then: a token with a NaN, or a row
+// of finite weights, has no other sum. Four lanes a row, a token at a time.
+// wrow: this lane's row (a valid one, of which `row_ok` says whether it
+// counts); x: the tokens' rows, `tokens` of them; seen and bad: the tokens
+// looked at, and those with a NaN, kept from call to call. Every lane of the
+// wave calls. Us with finite inputs / a NaN in one token / in each / two
+// infinities in each / one infinite weight / NaN weights: 12 tokens x 9728 x
+// 2560 18 / 24 / 53 / 88 / 46 / 88; with every NaN summed again by its own lane
+// 18 / 575 / 2586 / 2287 / 168 / 2580.
+__device__ __forceinline__ void repair_nan(f32_acc4 &s, const uint16_t *wrow, bool row_ok, const float *x, int tokens,
+                                           int cols, int c0, int c1, int fq, unsigned &seen, unsigned &bad) {
+    if (__builtin_expect(!__any(s[0] != s[0] || s[1] != s[1] || s[2] != s[2] || s[3] != s[3]), 1)) return;
+    const int lane = threadIdx.x & 63;
+    int row_inf = -1;  // not looked at
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+#pragma unroll 1
+        for (int q = 0; q < 4; ++q) {
+            const int t = 4 * q + i;
+            if (t >= tokens || !__any(s[i] != s[i] && fq == q && row_ok)) continue;
+            const float *xr = x + (size_t)t * cols;
+            if (!(seen >> t & 1)) {
+                bool nan = false;
+                for (int c = c0 + 4 * lane; c < c1; c += 1024) {
+                    float4 v[4];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) v[k] = *reinterpret_cast<const float4 *>(xr + min(c + 256 * k, c1 - 4));
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) nan |= (v[k].x != v[k].x) | (v[k].y != v[k].y) | (v[k].z != v[k].z) | (v[k].w != v[k].w);
+                }
+                seen |= 1u << t;
+                if (__any(nan)) bad |= 1u << t;
+            }
+            if (bad >> t & 1) continue;
+            if (row_inf < 0) {
+                int inf = 0;
+                for (int c = c0 + 8 * fq; c < c1; c += 256) {
+                    uint4 w[8];
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) w[k] = *reinterpret_cast<const uint4 *>(wrow + min(c + 32 * k, c1 - 8));
+#pragma unroll
+                    for (int k = 0; k < 8; ++k)
+                        inf |= has_inf_bf16(w[k].x) | has_inf_bf16(w[k].y) | has_inf_bf16(w[k].z) | has_inf_bf16(w[k].w);
+                }
+                inf |= __shfl_xor(inf, 16, 64);
+                row_inf = inf | __shfl_xor(inf, 32, 64);
+            }
+            if (!__any(s[i] != s[i] && fq == q && row_ok && row_inf)) continue;
+            float d = 0.f;
+            for (int c = c0 + 8 * fq; c < c1; c += 128) {
+                uint4 w[4];
+                float4 u[4], v[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const int at = min(c + 32 * k, c1 - 8);
+                    w[k] = *reinterpret_cast<const uint4 *>(wrow + at);
+                    u[k] = *reinterpret_cast<const float4 *>(xr + at);
+                    v[k] = *reinterpret_cast<const float4 *>(xr + at + 4);
+                }
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    if (c + 32 * k >= c1) break;
+                    d = fmaf(bf16_lo(w[k].x), u[k].x, d);
+                    d = fmaf(bf16_hi(w[k].x), u[k].y, d);
+                    d = fmaf(bf16_lo(w[k].y), u[k].z, d);
+                    d = fmaf(bf16_hi(w[k].y), u[k].w, d);
+                    d = fmaf(bf16_lo(w[k].z), v[k].x, d);
+                    d = fmaf(bf16_hi(w[k].z), v[k].y, d);
+                    d = fmaf(bf16_lo(w[k].w), v[k].z, d);
+                    d = fmaf(bf16_hi(w[k].w), v[k].w, d);
+                }
+            }
+            d += __shfl_xor(d, 16, 64);
+            d += __shfl_xor(d, 32, 64);
+            if (s[i] != s[i] && fq == q && row_inf) s[i] = d;
+        }
+    }
 }
 
 // wave_sum's value, bit for bit, without its six LDS round trips: the same

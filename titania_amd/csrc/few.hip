@@ -17,7 +17,7 @@
 // so that their sum is the f32 value exactly), three products a weight
 // fragment: measured against 64 bits, the results are as close as the f32
 // GEMV's or closer (8.1e-8 against 1.0e-7 at 1096 columns), infinities and
-// NaN as the f32 products give them (plain_dot).
+// NaN as the f32 products give them (repair_nan).
 #include "few.h"
 
 #include "common.h"
@@ -128,6 +128,7 @@ __global__ __launch_bounds__(64 * WK) void few_kernel(Args a) {
     // Two (tile, chunk)s an iteration, from the two weight buffers; a tile is
     // gate and up with kSilu (chunks are then walked once for each).
     int part2 = 0;  // kSilu: 0 gate, 1 up
+    unsigned x_seen = 0, x_bad = 0;  // repair_nan's
     while (tile < a.tiles) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
@@ -165,16 +166,13 @@ __global__ __launch_bounds__(64 * WK) void few_kernel(Args a) {
                     f32x4 s = red[turn & 1][0][lane];
 #pragma unroll
                     for (int k = 1; k < WK; ++k) s += red[turn & 1][k][lane];
-                    if (__builtin_expect(s[0] != s[0] || s[1] != s[1] || s[2] != s[2] || s[3] != s[3], 0)) {
+                    {
                         const int seg = EPI == kSilu ? part2 : tile < a.tiles0 ? 0 : tile < a.tiles1 ? 1 : 2;
                         const int row = 16 * (EPI == kSilu ? tile : tile - (seg == 0 ? 0 : seg == 1 ? a.tiles0 : a.tiles1)) + fr;
                         const uint16_t *m = seg == 0 ? a.w[0] : seg == 1 ? a.w[1] : a.w[2];
                         const int rows = seg == 0 || EPI == kSilu ? a.rows[0] : seg == 1 ? a.rows[1] : a.rows[2];
-#pragma unroll
-                        for (int i = 0; i < 4; ++i)
-                            if (s[i] != s[i] && row < rows && t0 + 4 * fq + i < a.n)
-                                s[i] = plain_dot(m + (size_t)row * cols, xb + (size_t)(4 * fq + i) * cols, 32 * kb,
-                                                 32 * ke < cols ? 32 * ke : cols);
+                        repair_nan(s, m + (size_t)(row < rows ? row : rows - 1) * cols, row < rows, xb, a.n - t0, cols,
+                                   32 * kb, 32 * ke < cols ? 32 * ke : cols, fq, x_seen, x_bad);
                     }
                     if (EPI == kSilu && part2 == 0) {
                         gate = s;

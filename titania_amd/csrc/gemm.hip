@@ -765,17 +765,20 @@ __global__ __launch_bounds__(kF32Threads, 2) void gemm_f32_kernel(int gxy, int r
     if (half == 1) return;
     const int rows = sg.rows;
     float *out = ksplit > 1 ? part + (size_t)z * n * rows : sg.out;
+    unsigned x_seen = 0, x_bad = 0;  // repair_nan's
 #pragma unroll
     for (int q = 0; q < FN; ++q) {
-        const f32x4 s = acc[q] + ep[wave][q][lane];
+        f32x4 s = acc[q] + ep[wave][q][lane];
+        if constexpr (RAGGED) {
+            const int r = q * 16 + fr, last = rows - 1 - sg.local;
+            repair_nan(s, w + (size_t)min(r, last) * cols, r <= last, xk + (size_t)min(t0 + wm, n - 1) * cols,
+                       n - t0 - wm, cols, 0, min(nk * T::BK, cols - kb * T::BK), fq, x_seen, x_bad);
+        }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int t = t0 + wm + fq * 4 + i, r = q * 16 + fr;
             if (t >= n || (RAGGED && sg.local + r >= rows)) continue;
-            float v = s[i];
-            if (RAGGED && __builtin_expect(v != v, 0))
-                v = plain_dot(w + (size_t)r * cols, xk + (size_t)t * cols, 0, min(nk * T::BK, cols - kb * T::BK));
-            out[(size_t)t * rows + sg.local + r] = v;
+            out[(size_t)t * rows + sg.local + r] = s[i];
         }
     }
 }
