@@ -38,9 +38,18 @@ constexpr size_t kWeightsPerLayer = 11;
 // Tokens from which the prefill attention of an f32 cache goes through the
 // bf16 planes of its keys and values: with fewer, splitting every earlier
 // position once costs more than splitting the tiles that the few token tiles
-// read (Qwen3-0.6B, us a layer at position 300: 8 / 64 / 256 tokens 62.7 /
-// 75.9 / 87.7 with the planes, 58.3 / 70.7 / 78.0 without; Qwen3-4B, position
-// 4000: 11 / 128 / 200 tokens 140.4 / 209.8 / 272.2 and 131.7 / 201.1 / 271.0).
+// read. Us a layer with / without the planes (medians of ten runs), tokens at
+// position 0, 300, 2000, 8000, 16000:
+//   Qwen3-0.6B 64   62 /  62, 71 / 64,  83 /  72, 109 /  88, 142 / 104
+//              256  72 /  73, 86 / 75, 102 /  89, 144 / 132, 210 / 188
+//              400  92 /  93, 97 / 93, 119 / 116, 200 / 201
+//              700 130 / 132, 151 / 146, 181 / 181, 301 / 311
+//   Qwen3-4B   64  123 / 123, 134 / 124, 146 / 134, 176 / 158, 221 / 188
+//              300 210 / 209, 233 / 212, 258 / 242, 350 / 357, 487 / 504
+//              400 282 / 284, 301 / 296, 350 / 354, 496 / 517
+//              700 416 / 419, 438 / 435, 494 / 505, 705 / 753
+// Past 300 tokens the two are within 5% up to a few thousand positions, and
+// the planes are ahead from there.
 constexpr size_t kPlaneMinTokens = 320;
 
 struct Layer {
@@ -657,7 +666,12 @@ int enqueue_fused(th_state *s, const uint32_t *tokens, size_t n, size_t pos, con
             // The q/k/v GEMMs with the q/k norm + RoPE + KV append epilogue,
             // which also writes the new positions' planes.
             auto epilogue_planes = [&]() -> int {
-                if (!use_planes) return TH_OK;
+                // Tokens that do not start a 32-key slice would write their
+                // values' planes element by element: launch_attention_planes
+                // then takes every position from the caches (Qwen3-0.6B, us a
+                // layer, 512 / 1000 / 2000 tokens at 100: 116 / 188 / 298 -> 100
+                // / 163 / 269; at 32 99 / 159 / 263).
+                if (!use_planes || pos % 32) return TH_OK;
                 // Earlier positions from the caches first (its zeros past
                 // them precede the epilogue's writes).
                 TH_HIP(th::launch_kv_planes(st, aa, pos, s->kv_planes, s->kv_planes_bytes, s->max_len));
