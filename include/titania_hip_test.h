@@ -107,6 +107,17 @@ TH_API int th_test_attention_prefill(th_device *dev, const th_buffer *q, const t
                                      const th_buffer *v_cache, size_t max_len, size_t pos, size_t n, size_t n_heads,
                                      size_t n_kv_heads, int planes, th_buffer *out);
 
+/* The kernel that th_matmul takes for n (2 or more) tokens of a [rows, cols]
+ * weight, and its parts of K: 0 the scalar GEMV, 1 the GEMV, 2 the few-token
+ * kernel, 3 the GEMM for matrices that are not whole tiles, 4 the small-tile
+ * GEMM on f32 activations, 5 to 7 the small, large and huge tiles on split
+ * activations. Needs no GPU. */
+TH_API int th_test_matmul_route(size_t n, size_t rows, size_t cols, int *kernel, int *ksplit);
+
+/* Whether n tokens of n_outs matrices of `rows` rows in all go to the
+ * few-token kernel where the GEMM would take them too. Needs no GPU. */
+TH_API int th_test_few_preferred(size_t n, size_t rows, size_t cols, int n_outs, int *few);
+
 #ifdef __cplusplus
 }
 #endif

@@ -147,6 +147,15 @@ size_t argmax_partials(size_t n);
 hipError_t launch_argmax(hipStream_t s, const float *x, size_t n, uint64_t *partials, uint32_t *token);
 hipError_t launch_argmax_partials(hipStream_t s, const float *x, size_t n, uint64_t *partials);
 
+// The kernel that launch_matmul takes, and its parts of K (kMatmulGemm's are
+// gemm_outs_plan's), with room for partials or without.
+enum MatmulKernel { kMatmulScalar, kMatmulGemv, kMatmulFew, kMatmulRagged, kMatmulGemm };
+struct MatmulRoute {
+    MatmulKernel kernel;
+    int ksplit;
+};
+MatmulRoute matmul_route(size_t n, size_t rows, size_t cols, bool part);
+
 // out[t*rows + r] = dot(w[r], x[t]) for t < n. Where it splits K, the partials
 // go to part (kPartFloats long; null: it does not split).
 hipError_t launch_matmul(hipStream_t s, float *out, const uint16_t *w, size_t rows, size_t cols, const float *x,

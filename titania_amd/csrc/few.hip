@@ -256,13 +256,24 @@ int few_ksplit(size_t n, size_t rows, size_t cols) {
 bool few_preferred(size_t n, size_t rows, size_t cols, int n_outs) {
     if (n < kGemmMinTokens) return true;
     if (n > 64) return false;
-    // The GEMM splits the K of a single matrix, this kernel reads each weight
-    // once for every 16 tokens. Calls of 16 / 36 / 64 tokens: x 4096 x 1024
-    // 6.1 / 8.2 / 9.0 us against the GEMM's 10.3 unsplit (8.4 in four parts
-    // with their sum); x 6144 x 2560, 64 tokens, 21.9 against 23.9; but x 2560
-    // x 9728, 32 tokens, 22.8 against 17, and x 19456 x 2560, 64 tokens, 53
-    // against 45.
-    return n_outs == 1 ? cols <= 1024 : rows * cols <= ((size_t)32 << 20) || n <= 32;
+    // The GEMM splits the K of a single matrix and reads each weight once for
+    // 64 tokens, this kernel once for every 16: so many tiles of 16 tokens
+    // times rows. Us, this kernel / that one, weights from HBM: one matrix of
+    // 1024 columns, 6144 rows and 33 / 64 tokens 10.8 / 10.0, 11.1 / 12.0;
+    // 16384 and 16 / 17 / 64 tokens 10.0 / 12.1, 13.1 / 12.8, 24.5 / 15.1;
+    // 151936 and 16 / 64 67.6 / 77.7, 197.7 / 93.5. Of more columns, 1024 x
+    // 2048 and 16 tokens 9.0 / 7.4, 2560 x 9728 36.5 / 21.9.
+    const size_t work = (n + kTokens - 1) / kTokens * rows;
+    if (n_outs == 1) return cols <= 1024 && (n <= (size_t)kTokens || work <= 24576);
+    // Several matrices: the GEMM does not split K, and gate and up then take a
+    // launch more. Gate and up of 16384 x 1024, 17 / 33 / 64 tokens 21.8 / 19.0,
+    // 31.7 / 20.3, 38.7 / 23.9, of 8192 12.6 / 15.0, 19.2 / 15.5, 21.3 / 16.3, of
+    // 4096 8.2 / 12.2, 12.2 / 12.4, 12.2 / 12.8; 9728 x 2560, 32 / 33 tokens 35.1
+    // / 36.8, 44.5 / 36.9; q, k and v of 6144 x 2560, 64 tokens 25.2 / 30.9, of
+    // 12288 x 1024, 33 tokens 20.7 / 14.9. Past 2560 columns it goes in chunks:
+    // gate and up of 2048 x 4096, 32 / 33 tokens 31.5 / 41.2, 54.4 / 41.0; of
+    // 8192 x 4096, 17 tokens 101.7 / 47.6.
+    return work <= (cols > 2560 ? 8192 : n <= 32 ? 40960 : 32768);
 }
 
 double few_us(size_t n, size_t rows, size_t cols) {

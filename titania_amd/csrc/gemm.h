@@ -44,6 +44,12 @@ hipError_t launch_gemm_f32(hipStream_t s, const float *x, size_t n, size_t cols,
 hipError_t launch_gemm_outs(hipStream_t s, const float *x, size_t n, size_t cols, const GemmOut *outs, int n_outs,
                             float *part);
 
+// What launch_gemm_outs takes: the small tile on f32 activations, or the plan of
+// launch_gemm_multi (small, large or huge tiles on split activations), and the
+// parts of K.
+enum GemmTile { kGemmF32, kGemmSmall, kGemmLarge, kGemmHuge };
+GemmTile gemm_outs_plan(size_t n, size_t cols, const GemmOut *outs, int n_outs, bool part, int *ksplit);
+
 // The GEMM on f32 activations for a matrix of any number of rows, of columns
 // in whole 16-byte chunks: x enters as three bf16 terms, exactly. K in ksplit
 // parts as launch_gemm_f32 (gemm_ragged_ksplit: those that fill the chip).

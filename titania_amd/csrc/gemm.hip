@@ -923,8 +923,9 @@ double mid_cost(size_t blocks) { return tile_cost(blocks, 64 * 128, 1, 1.5); }
 double wide_cost(size_t blocks) { return tile_cost(blocks, 64 * 192, 1, 1.3); }
 double large_cost(size_t blocks) { return tile_cost(blocks, 128 * 128, 1, 1.1); }
 
-// Whether the plan for these matrices is the small tile.
-bool small_plan(size_t n, size_t cols, const GemmOut *outs, int n_outs, int *ksplit) {
+}  // namespace
+
+GemmTile gemm_outs_plan(size_t n, size_t cols, const GemmOut *outs, int n_outs, bool part, int *ksplit) {
     size_t total = 0;
     bool rows_large = true, rows_huge = true;
     for (int i = 0; i < n_outs; ++i) {
@@ -933,14 +934,21 @@ bool small_plan(size_t n, size_t cols, const GemmOut *outs, int n_outs, int *ksp
         rows_huge = rows_huge && outs[i].rows % Huge::BN == 0;
     }
     const Plan plan = gemm_plan(n, total, cols, n_outs, rows_large, rows_huge);
+    // Small tiles take the f32 activations as they are, with partials in the
+    // caller's scratch: 64 tokens x 2560 x 9728, 29.6 -> 17.5 us a call (the
+    // launch that split the activations gone, K in six parts instead of four),
+    // and where a call ran for less than its stream-ordered allocation took,
+    // x 1024 x 3072, 26.0 -> 9.0.
+    const bool near = plan.large && !plan.huge && plan.gain <= kSplitLaunchUs;
+    const int ks = near ? small_ksplit(n, total, cols) : plan.ksplit;
+    if ((near || !plan.large) && total / Small::BN <= 0xffff && (n + Small::BM - 1) / Small::BM <= 0xffff &&
+        n <= ((size_t)1 << 24) && (ks == 1 || (part && (size_t)ks * n * total <= kPartFloats))) {
+        *ksplit = ks;
+        return kGemmF32;
+    }
     *ksplit = plan.ksplit;
-    if (plan.large && !plan.huge && plan.gain <= kSplitLaunchUs) *ksplit = small_ksplit(n, total, cols);
-    else if (plan.large || plan.huge) return false;
-    return total / Small::BN <= 0xffff && (n + Small::BM - 1) / Small::BM <= 0xffff &&
-           n <= ((size_t)1 << 24);
+    return plan.huge ? kGemmHuge : plan.large ? kGemmLarge : kGemmSmall;
 }
-
-}  // namespace
 
 size_t gemm_scratch_bytes(size_t n, size_t cols, size_t rows) {
     // K in two parts at any size, in more within kSplitFloats (the large tile)
@@ -1210,14 +1218,8 @@ hipError_t launch_gemm_outs(hipStream_t s, const float *x, size_t n, size_t cols
         if (!gemm_supported(outs[i].rows, cols)) return hipErrorInvalidValue;
         total += outs[i].rows;
     }
-    // Small tiles take the f32 activations as they are, with partials in the
-    // caller's scratch: 64 tokens x 2560 x 9728, 29.6 -> 17.5 us a call (the
-    // launch that split the activations gone, K in six parts instead of four),
-    // and where a call ran for less than its stream-ordered allocation took,
-    // x 1024 x 3072, 26.0 -> 9.0.
     int ksplit = 1;
-    if (small_plan(n, cols, outs, n_outs, &ksplit) &&
-        (ksplit == 1 || (part && (size_t)ksplit * n * total <= kPartFloats))) {
+    if (gemm_outs_plan(n, cols, outs, n_outs, part != nullptr, &ksplit) == kGemmF32) {
         const hipError_t e = launch_gemm_f32(s, x, n, cols, outs, n_outs, part, ksplit);
         return e != hipSuccess || ksplit == 1 ? e : launch_splitk_sum(s, part, outs[0].out, n * total, ksplit);
     }

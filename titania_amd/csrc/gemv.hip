@@ -94,49 +94,55 @@ static hipError_t gemv(hipStream_t s, float *out, const uint16_t *w, size_t rows
     return hipGetLastError();
 }
 
-hipError_t launch_matmul(hipStream_t s, float *out, const uint16_t *w, size_t rows, size_t cols, const float *x,
-                         size_t n, float *part) {
-    if (n == 0 || rows == 0) return hipSuccess;
-    if (cols % 8 != 0) {
-        gemv_scalar_kernel<<<dim3((unsigned)((rows + 3) / 4)), 256, 0, s>>>(out, w, rows, cols, x, n);
-        return hipGetLastError();
-    }
-    if (n >= kGemmMinTokens && gemm_supported(rows, cols) && !few_preferred(n, rows, cols, 1))
-        return launch_gemm(s, out, w, rows, cols, x, n, part);
-    if (n == 1) {
-        // Enough waves to cover the chip (256 CUs x 4 SIMDs) before packing rows.
-        if (rows >= 16384) return gemv<4, 1>(s, out, w, rows, cols, x, 1, rows);
-        if (rows >= 4096) return gemv<2, 1>(s, out, w, rows, cols, x, 1, rows);
-        return gemv<1, 1>(s, out, w, rows, cols, x, 1, rows);
-    }
-    // Two and three tokens stay here (x 4096 x 1024, 2 / 4 / 8 tokens: 4.2 /
-    // 5.6 / 8.7 us against few.hip's 5.5 / 5.6 / 5.7; 19456 x 2560, 2 / 3 / 4 /
-    // 8: 21.4 / 25.9 / 29.8 / 46.8 against 25.8 / 25.7 / 25.9 / 26.1).
-    if (n == 2) return gemv<2, 2>(s, out, w, rows, cols, x, 2, rows);
-    if (n == 3 || !few_supported(n, rows, cols)) {
-        for (size_t t0 = 0; t0 < n; t0 += 4) {
-            const hipError_t e = gemv<2, 4>(s, out + t0 * rows, w, rows, cols, x + t0 * cols,
-                                            (int)std::min<size_t>(4, n - t0), rows);
-            if (e != hipSuccess) return e;
-        }
-        return hipSuccess;
-    }
+MatmulRoute matmul_route(size_t n, size_t rows, size_t cols, bool part) {
+    if (cols % 8 != 0) return {kMatmulScalar, 1};
+    if (n >= kGemmMinTokens && gemm_supported(rows, cols) && !few_preferred(n, rows, cols, 1)) return {kMatmulGemm, 1};
+    // Two and three tokens stay on the GEMV (x 4096 x 1024, 2 / 4 / 8 tokens:
+    // 4.2 / 5.6 / 8.7 us against few.hip's 5.5 / 5.6 / 5.7; 19456 x 2560, 2 / 3 / 4
+    // / 8: 21.4 / 25.9 / 29.8 / 46.8 against 25.8 / 25.7 / 25.9 / 26.1).
+    if (n <= 3 || !few_supported(n, rows, cols)) return {kMatmulGemv, 1};
     // The partials' room and their sum's 16-byte chunks.
     auto fits = [&](int k) { return part && n * rows % 4 == 0 && (size_t)k * n * rows <= kPartFloats; };
     int ksplit = n < kGemmMinTokens ? few_ksplit(n, rows, cols) : 1;
     if (!fits(ksplit)) ksplit = 1;
-    bool ragged = false;
     if (n > 16 && gemm_ragged_supported(n, rows, cols) && !gemm_supported(rows, cols)) {
         int k = gemm_ragged_ksplit(n, rows, cols);
         if (!fits(k)) k = 1;
-        ragged = gemm_ragged_us(n, rows, cols, k) + 2 < few_us(n, rows, cols);
-        if (ragged) ksplit = k;
+        if (gemm_ragged_us(n, rows, cols, k) + 2 < few_us(n, rows, cols)) return {kMatmulRagged, k};
     }
-    const GemmOut o{w, rows, out};
-    const hipError_t e = ragged ? launch_gemm_ragged(s, x, n, cols, w, rows, out, part, ksplit)
-                                : launch_few(s, x, n, cols, &o, 1, part, ksplit);
-    if (e != hipSuccess || ksplit == 1) return e;
-    return launch_splitk_sum(s, part, out, n * rows, ksplit);
+    return {kMatmulFew, ksplit};
+}
+
+hipError_t launch_matmul(hipStream_t s, float *out, const uint16_t *w, size_t rows, size_t cols, const float *x,
+                         size_t n, float *part) {
+    if (n == 0 || rows == 0) return hipSuccess;
+    const MatmulRoute r = matmul_route(n, rows, cols, part != nullptr);
+    hipError_t e = hipSuccess;
+    switch (r.kernel) {
+    case kMatmulScalar:
+        gemv_scalar_kernel<<<dim3((unsigned)((rows + 3) / 4)), 256, 0, s>>>(out, w, rows, cols, x, n);
+        return hipGetLastError();
+    case kMatmulGemm: return launch_gemm(s, out, w, rows, cols, x, n, part);
+    case kMatmulGemv:
+        if (n == 1) {
+            // Enough waves to cover the chip (256 CUs x 4 SIMDs) before packing rows.
+            if (rows >= 16384) return gemv<4, 1>(s, out, w, rows, cols, x, 1, rows);
+            if (rows >= 4096) return gemv<2, 1>(s, out, w, rows, cols, x, 1, rows);
+            return gemv<1, 1>(s, out, w, rows, cols, x, 1, rows);
+        }
+        if (n == 2) return gemv<2, 2>(s, out, w, rows, cols, x, 2, rows);
+        for (size_t t0 = 0; t0 < n && e == hipSuccess; t0 += 4)
+            e = gemv<2, 4>(s, out + t0 * rows, w, rows, cols, x + t0 * cols, (int)std::min<size_t>(4, n - t0), rows);
+        return e;
+    case kMatmulRagged: e = launch_gemm_ragged(s, x, n, cols, w, rows, out, part, r.ksplit); break;
+    case kMatmulFew: {
+        const GemmOut o{w, rows, out};
+        e = launch_few(s, x, n, cols, &o, 1, part, r.ksplit);
+        break;
+    }
+    }
+    if (e != hipSuccess || r.ksplit == 1) return e;
+    return launch_splitk_sum(s, part, out, n * rows, r.ksplit);
 }
 
 }  // namespace th

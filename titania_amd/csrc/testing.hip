@@ -12,6 +12,7 @@
 
 #include "../../include/titania_hip_test.h"
 #include "common.h"
+#include "few.h"
 #include "fused.h"
 #include "gemm.h"
 #include "step.h"
@@ -398,6 +399,24 @@ int th_test_attention_prefill(th_device *dev, const th_buffer *q, const th_buffe
         TH_HIP(th::launch_attention(dev->stream, a, n, hd));
     }
     TH_HIP(hipStreamSynchronize(dev->stream));
+    return TH_OK;
+}
+
+int th_test_matmul_route(size_t n, size_t rows, size_t cols, int *kernel, int *ksplit) {
+    TH_REQUIRE(n > 0 && rows > 0 && cols > 0 && kernel && ksplit, "th_test_matmul_route: empty or null argument");
+    const th::MatmulRoute r = th::matmul_route(n, rows, cols, true);
+    *kernel = (int)r.kernel;
+    *ksplit = r.ksplit;
+    if (r.kernel == th::kMatmulGemm) {
+        const th::GemmOut o{nullptr, rows, nullptr};
+        *kernel += (int)th::gemm_outs_plan(n, cols, &o, 1, true, ksplit);
+    }
+    return TH_OK;
+}
+
+int th_test_few_preferred(size_t n, size_t rows, size_t cols, int n_outs, int *few) {
+    TH_REQUIRE(n_outs >= 1 && n_outs <= 3 && few, "th_test_few_preferred: 1 to 3 matrices");
+    *few = th::few_preferred(n, rows, cols, n_outs);
     return TH_OK;
 }
 
