@@ -299,7 +299,7 @@ def test_add_rmsnorm_rows(hip, rows, dim, parts):
 
 @pytest.mark.parametrize("n", [2, 3, 4, 15, 16, 17, 50])
 @pytest.mark.parametrize("rows,cols", [(1, 8), (15, 24), (16, 504), (17, 512), (100, 520), (33, 768), (40, 1032),
-                                       (257, 1528), (16, 2056), (48, 2568), (5000, 1096), (24, 9736)])
+                                       (257, 1528), (16, 2056), (48, 2568), (5000, 1096), (24, 9736), (1003, 2968)])
 def test_few_token_matmul(hip, rows, cols, n):
     """Row, column and token counts around the few-token kernel's tiles (16
     rows, 32 columns a step, 2 to 10 steps a wave and eight waves a block,

@@ -51,3 +51,9 @@ def test_tall_matrix_reads_its_weights_once(n):
     (33, 6144, 4096, False), (65, 64, 64, False), (15, 2 * 8192, 4096, True)])
 def test_several_matrices(n, rows, cols, few):
     assert few_preferred(n, rows, cols, 2) == few and few_preferred(n, rows, cols, 3) == few
+
+
+@pytest.mark.parametrize("n,rows,cols", [(5, 5003, 2968), (7, 1003, 4552), (17, 5003, 2968), (33, 5003, 2968)])
+def test_odd_products_split_k(n, rows, cols):
+    """An odd number of results does not keep K in one part."""
+    assert n * rows % 2 and route(n, rows, cols)[1] > 1

@@ -108,7 +108,7 @@ hipError_t launch_gemm_qkv_huge(hipStream_t s, const uint16_t *hi, const uint16_
                                 const uint16_t *wq, const uint16_t *wk, const uint16_t *wv, const QkvPostArgs &a);
 
 // out[i] = part[i] + part[m + i] + ... over ksplit partials of m values, in
-// order (m a multiple of 4).
+// order.
 hipError_t launch_splitk_sum(hipStream_t s, const float *part, float *out, size_t m, int ksplit);
 
 // Bytes of scratch launch_gemm_multi needs for n tokens of `cols` columns and

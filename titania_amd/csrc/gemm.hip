@@ -806,6 +806,17 @@ __global__ void splitk_sum_kernel(const float4 *__restrict__ part, float4 *__res
     }
 }
 
+// The same for any m, one a thread.
+__global__ void splitk_sum_odd_kernel(const float *__restrict__ part, float *__restrict__ out, size_t m, int ksplit) {
+    const size_t stride = (size_t)gridDim.x * blockDim.x;
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < m; i += stride) {
+        float acc = part[i];
+#pragma unroll 4
+        for (int z = 1; z < ksplit; ++z) acc += part[(size_t)z * m + i];
+        out[i] = acc;
+    }
+}
+
 }  // namespace
 
 bool gemm_supported(size_t rows, size_t cols) {
@@ -1126,7 +1137,11 @@ hipError_t launch_gemm_qkv(hipStream_t s, const uint16_t *hi, const uint16_t *lo
 
 hipError_t launch_splitk_sum(hipStream_t s, const float *part, float *out, size_t m, int ksplit) {
     if (m == 0) return hipSuccess;
-    if (m % 4 || ((uintptr_t)part | (uintptr_t)out) % 16) return hipErrorInvalidValue;
+    if (m % 4) {
+        splitk_sum_odd_kernel<<<(unsigned)std::min<size_t>((m + 255) / 256, 8192), 256, 0, s>>>(part, out, m, ksplit);
+        return hipGetLastError();
+    }
+    if (((uintptr_t)part | (uintptr_t)out) % 16) return hipErrorInvalidValue;
     const size_t m4 = m / 4;
     splitk_sum_kernel<<<(unsigned)std::min<size_t>((m4 + 255) / 256, 4096), 256, 0, s>>>(
         reinterpret_cast<const float4 *>(part), reinterpret_cast<float4 *>(out), m4, ksplit);

@@ -101,8 +101,7 @@ MatmulRoute matmul_route(size_t n, size_t rows, size_t cols, bool part) {
     // 4.2 / 5.6 / 8.7 us against few.hip's 5.5 / 5.6 / 5.7; 19456 x 2560, 2 / 3 / 4
     // / 8: 21.4 / 25.9 / 29.8 / 46.8 against 25.8 / 25.7 / 25.9 / 26.1).
     if (n <= 3 || !few_supported(n, rows, cols)) return {kMatmulGemv, 1};
-    // The partials' room and their sum's 16-byte chunks.
-    auto fits = [&](int k) { return part && n * rows % 4 == 0 && (size_t)k * n * rows <= kPartFloats; };
+    auto fits = [&](int k) { return part && (size_t)k * n * rows <= kPartFloats; };
     int ksplit = n < kGemmMinTokens ? few_ksplit(n, rows, cols) : 1;
     if (!fits(ksplit)) ksplit = 1;
     if (n > 16 && gemm_ragged_supported(n, rows, cols) && !gemm_supported(rows, cols)) {
