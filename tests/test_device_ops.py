@@ -368,6 +368,29 @@ def test_few_token_matmul_not_finite(hip, n):
     assert np.array_equal(got[infinite], exp[infinite]) and np.all(np.isfinite(got[np.isfinite(exp)]))
 
 
+@pytest.mark.parametrize("n", [3, 15, 20])
+def test_gate_up_silu_not_finite(hip, n):
+    """Infinite and NaN weights and activations through the joint gate and up
+    launch: what their products, sums and silu in f32 give."""
+    H, I = 520, 1000
+    rng = np.random.default_rng(n)
+    g, u = (bf16_to_f32(normal_bf16(I * H, 7, k, 0.05)).reshape(I, H).copy() for k in ("ig", "iu"))
+    x = np.round(rng.standard_normal((n, H)).astype(np.float32) * 4) / 4 + np.float32(0.125)  # no zero; bf16 exactly
+    g[3, 500], g[5, 10], g[7, 30], u[5, 11], u[9, 40], u[990, 3], g[999, 519] = (np.inf, -np.inf, np.nan, np.inf, -np.inf,
+                                                                                 np.inf, np.inf)
+    x[1, 200], x[2, 519] = np.inf, np.nan
+    with np.errstate(invalid="ignore", over="ignore"):
+        a, b = ((w[None].astype(np.float64) * x[:, None].astype(np.float64)).sum(-1) for w in (g, u))
+        exp = a / (1 + np.exp(-a)) * b
+    bx, bg, bu = hip.alloc(n * H), hip.alloc(n * I), hip.alloc(n * I)
+    hip.write(bx, x)
+    hip.gate_up_silu(bg, bu, *(hip.upload(Tensor((I, H), f32_to_bf16(w.reshape(-1)))) for w in (g, u)), bx)
+    got = hip.read(bg).reshape(n, I).astype(np.float64)
+    assert np.array_equal(np.isnan(got), np.isnan(exp))
+    infinite = np.isinf(exp)
+    assert np.array_equal(got[infinite], exp[infinite]) and np.all(np.isfinite(got[np.isfinite(exp)]))
+
+
 @pytest.mark.parametrize("n,rows,cols", [(12, 9728, 2560), (40, 5003, 2968)])
 def test_few_token_matmul_not_finite_time(hip, n, rows, cols):
     """Inputs that make every result NaN take no more than a pass over each

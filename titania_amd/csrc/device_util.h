@@ -193,9 +193,28 @@ __device__ __forceinline__ void split3(const uint4 &a, const uint4 &b, bf16_term
     }
 }
 
-// Whether one of the word's two bf16 is infinite.
-__device__ __forceinline__ int has_inf_bf16(uint32_t u) {
-    return ((u & 0x7fffu) == 0x7f80u) | ((u >> 16 & 0x7fffu) == 0x7f80u);
+// Whether one of the wave's sums is NaN: repair_nan is then called.
+__device__ __forceinline__ bool any_nan(const f32_acc4 &s) {
+    return __builtin_expect(__any(s[0] != s[0] || s[1] != s[1] || s[2] != s[2] || s[3] != s[3]), 0);
+}
+
+// Whether columns [c0, c1) (whole 8s) of a row hold an infinity: four lanes a row.
+__device__ __forceinline__ bool row_has_inf(const uint16_t *wrow, int c0, int c1, int fq) {
+    uint32_t least = ~0u;  // of the distances from infinity, bit by bit
+    for (int c = c0 + 8 * fq; c < c1; c += 128) {
+        uint4 w[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) w[k] = *reinterpret_cast<const uint4 *>(wrow + min(c + 32 * k, c1 - 8));
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const uint32_t u[4] = {w[k].x, w[k].y, w[k].z, w[k].w};
+#pragma unroll
+            for (int h = 0; h < 4; ++h)
+                least = min(least, min((u[h] ^ 0x7f80u) & 0x7fffu, (u[h] >> 16 ^ 0x7f80u) & 0x7fffu));
+        }
+    }
+    least = min(least, (uint32_t)__shfl_xor((int)least, 16, 64));
+    return min(least, (uint32_t)__shfl_xor((int)least, 32, 64)) == 0;
 }
 
 // Sums of split3 terms' products, 16 rows x 16 tokens a wave (lane (fq, fr):
@@ -204,78 +223,72 @@ __device__ __forceinline__ int has_inf_bf16(uint32_t u) {
 // weight is NaN where x w is infinite. Only then: a token with a NaN, or a row
 // of finite weights, has no other sum. Four lanes a row, a token at a time.
 // wrow: this lane's row (a valid one, of which `row_ok` says whether it
-// counts); x: the tokens' rows, `tokens` of them; seen and bad: the tokens
-// looked at, and those with a NaN, kept from call to call. Every lane of the
-// wave calls. Us with finite inputs / a NaN in one token / in each / two
-// infinities in each / one infinite weight / NaN weights: 12 tokens x 9728 x
-// 2560 18 / 24 / 53 / 88 / 46 / 88; with every NaN summed again by its own lane
-// 18 / 575 / 2586 / 2287 / 168 / 2580.
-__device__ __forceinline__ void repair_nan(f32_acc4 &s, const uint16_t *wrow, bool row_ok, const float *x, int tokens,
-                                           int cols, int c0, int c1, int fq, unsigned &seen, unsigned &bad) {
-    if (__builtin_expect(!__any(s[0] != s[0] || s[1] != s[1] || s[2] != s[2] || s[3] != s[3]), 1)) return;
+// counts); other: a row whose infinities count as this one's; x: the tokens'
+// rows, `tokens` of them; looked: the tokens looked at, and in its upper half
+// those with a NaN, kept from call to call. Every lane of the wave calls. Us
+// with finite inputs / a NaN in one token / in each / two infinities in each /
+// one infinite weight / NaN weights: 12 tokens x 9728 x 2560 18 / 22 / 29 / 43 /
+// 39 / 43; with every NaN summed again by its own lane 18 / 575 / 2586 / 2287 /
+// 168 / 2580.
+__device__ __forceinline__ void repair_nan(f32_acc4 &s, const uint16_t *wrow, const uint16_t *other, bool row_ok,
+                                           const float *x, int tokens, int cols, int c0, int c1, int fq,
+                                           unsigned &looked) {
     const int lane = threadIdx.x & 63;
     int row_inf = -1;  // not looked at
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
 #pragma unroll 1
-        for (int q = 0; q < 4; ++q) {
-            const int t = 4 * q + i;
-            if (t >= tokens || !__any(s[i] != s[i] && fq == q && row_ok)) continue;
-            const float *xr = x + (size_t)t * cols;
-            if (!(seen >> t & 1)) {
-                bool nan = false;
-                for (int c = c0 + 4 * lane; c < c1; c += 1024) {
-                    float4 v[4];
+    for (int t = 0; t < (tokens < 16 ? tokens : 16); ++t) {
+        const int i = t & 3;
+        const float v_t = i == 0 ? s[0] : i == 1 ? s[1] : i == 2 ? s[2] : s[3];
+        const bool mine = v_t != v_t && fq == t >> 2 && row_ok;
+        if (!__any(mine)) continue;
+        const float *xr = x + (size_t)t * cols;
+        if (!(looked >> t & 1)) {
+            uint32_t most = 0;  // magnitudes as words: integer maxima, not a mask for each comparison
+            for (int c = c0 + 4 * lane; c < c1; c += 1024) {
+                uint4 v[4];
 #pragma unroll
-                    for (int k = 0; k < 4; ++k) v[k] = *reinterpret_cast<const float4 *>(xr + min(c + 256 * k, c1 - 4));
+                for (int k = 0; k < 4; ++k) v[k] = *reinterpret_cast<const uint4 *>(xr + min(c + 256 * k, c1 - 4));
 #pragma unroll
-                    for (int k = 0; k < 4; ++k) nan |= (v[k].x != v[k].x) | (v[k].y != v[k].y) | (v[k].z != v[k].z) | (v[k].w != v[k].w);
-                }
-                seen |= 1u << t;
-                if (__any(nan)) bad |= 1u << t;
+                for (int k = 0; k < 4; ++k)
+                    most = max(max(max(v[k].x & 0x7fffffffu, v[k].y & 0x7fffffffu),
+                                   max(v[k].z & 0x7fffffffu, v[k].w & 0x7fffffffu)), most);
             }
-            if (bad >> t & 1) continue;
-            if (row_inf < 0) {
-                int inf = 0;
-                for (int c = c0 + 8 * fq; c < c1; c += 256) {
-                    uint4 w[8];
+            looked |= (__any(most > 0x7f800000u) ? 0x10001u : 1u) << t;
+        }
+        if (looked >> t & 0x10000u) continue;
+        if (row_inf < 0) row_inf = row_has_inf(wrow, c0, c1, fq) || (other != wrow && row_has_inf(other, c0, c1, fq));
+        if (!__any(mine && row_inf)) continue;
+        float d = 0.f;
+        for (int c = c0 + 8 * fq; c < c1; c += 128) {
+            uint4 w[4];
+            float4 u[4], v[4];
 #pragma unroll
-                    for (int k = 0; k < 8; ++k) w[k] = *reinterpret_cast<const uint4 *>(wrow + min(c + 32 * k, c1 - 8));
-#pragma unroll
-                    for (int k = 0; k < 8; ++k)
-                        inf |= has_inf_bf16(w[k].x) | has_inf_bf16(w[k].y) | has_inf_bf16(w[k].z) | has_inf_bf16(w[k].w);
-                }
-                inf |= __shfl_xor(inf, 16, 64);
-                row_inf = inf | __shfl_xor(inf, 32, 64);
+            for (int k = 0; k < 4; ++k) {
+                const int at = min(c + 32 * k, c1 - 8);
+                w[k] = *reinterpret_cast<const uint4 *>(wrow + at);
+                u[k] = *reinterpret_cast<const float4 *>(xr + at);
+                v[k] = *reinterpret_cast<const float4 *>(xr + at + 4);
             }
-            if (!__any(s[i] != s[i] && fq == q && row_ok && row_inf)) continue;
-            float d = 0.f;
-            for (int c = c0 + 8 * fq; c < c1; c += 128) {
-                uint4 w[4];
-                float4 u[4], v[4];
 #pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    const int at = min(c + 32 * k, c1 - 8);
-                    w[k] = *reinterpret_cast<const uint4 *>(wrow + at);
-                    u[k] = *reinterpret_cast<const float4 *>(xr + at);
-                    v[k] = *reinterpret_cast<const float4 *>(xr + at + 4);
-                }
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    if (c + 32 * k >= c1) break;
-                    d = fmaf(bf16_lo(w[k].x), u[k].x, d);
-                    d = fmaf(bf16_hi(w[k].x), u[k].y, d);
-                    d = fmaf(bf16_lo(w[k].y), u[k].z, d);
-                    d = fmaf(bf16_hi(w[k].y), u[k].w, d);
-                    d = fmaf(bf16_lo(w[k].z), v[k].x, d);
-                    d = fmaf(bf16_hi(w[k].z), v[k].y, d);
-                    d = fmaf(bf16_lo(w[k].w), v[k].z, d);
-                    d = fmaf(bf16_hi(w[k].w), v[k].w, d);
-                }
+            for (int k = 0; k < 4; ++k) {
+                if (c + 32 * k >= c1) break;
+                d = fmaf(bf16_lo(w[k].x), u[k].x, d);
+                d = fmaf(bf16_hi(w[k].x), u[k].y, d);
+                d = fmaf(bf16_lo(w[k].y), u[k].z, d);
+                d = fmaf(bf16_hi(w[k].y), u[k].w, d);
+                d = fmaf(bf16_lo(w[k].z), v[k].x, d);
+                d = fmaf(bf16_hi(w[k].z), v[k].y, d);
+                d = fmaf(bf16_lo(w[k].w), v[k].z, d);
+                d = fmaf(bf16_hi(w[k].w), v[k].w, d);
             }
-            d += __shfl_xor(d, 16, 64);
-            d += __shfl_xor(d, 32, 64);
-            if (s[i] != s[i] && fq == q && row_inf) s[i] = d;
+        }
+        d += __shfl_xor(d, 16, 64);
+        d += __shfl_xor(d, 32, 64);
+        if (mine && row_inf) {
+            s[0] = i == 0 ? d : s[0];
+            s[1] = i == 1 ? d : s[1];
+            s[2] = i == 2 ? d : s[2];
+            s[3] = i == 3 ? d : s[3];
         }
     }
 }

@@ -128,7 +128,7 @@ __global__ __launch_bounds__(64 * WK) void few_kernel(Args a) {
     // Two (tile, chunk)s an iteration, from the two weight buffers; a tile is
     // gate and up with kSilu (chunks are then walked once for each).
     int part2 = 0;  // kSilu: 0 gate, 1 up
-    unsigned x_seen = 0, x_bad = 0;  // repair_nan's
+    bool nan = false;
     while (tile < a.tiles) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
@@ -166,14 +166,7 @@ __global__ __launch_bounds__(64 * WK) void few_kernel(Args a) {
                     f32x4 s = red[turn & 1][0][lane];
 #pragma unroll
                     for (int k = 1; k < WK; ++k) s += red[turn & 1][k][lane];
-                    {
-                        const int seg = EPI == kSilu ? part2 : tile < a.tiles0 ? 0 : tile < a.tiles1 ? 1 : 2;
-                        const int row = 16 * (EPI == kSilu ? tile : tile - (seg == 0 ? 0 : seg == 1 ? a.tiles0 : a.tiles1)) + fr;
-                        const uint16_t *m = seg == 0 ? a.w[0] : seg == 1 ? a.w[1] : a.w[2];
-                        const int rows = seg == 0 || EPI == kSilu ? a.rows[0] : seg == 1 ? a.rows[1] : a.rows[2];
-                        repair_nan(s, m + (size_t)(row < rows ? row : rows - 1) * cols, row < rows, xb, a.n - t0, cols,
-                                   32 * kb, 32 * ke < cols ? 32 * ke : cols, fq, x_seen, x_bad);
-                    }
+                    nan |= any_nan(s);
                     if (EPI == kSilu && part2 == 0) {
                         gate = s;
                     } else {
@@ -201,13 +194,44 @@ __global__ __launch_bounds__(64 * WK) void few_kernel(Args a) {
             part2 = next_part;
         }
     }
+    if (__builtin_expect(!nan, 1)) return;
+    // This wave's tiles again, for what infinite weights made NaN (here and not
+    // in the loop, whose registers and instructions it would add to).
+    const int c0 = 32 * kb, c1 = 32 * ke < cols ? 32 * ke : cols;
+    unsigned looked = 0;
+    for (tile = blockIdx.x + wk * gridDim.x; tile < a.tiles; tile += WK * gridDim.x) {
+        const int seg = EPI == kSilu || tile < a.tiles0 ? 0 : tile < a.tiles1 ? 1 : 2;
+        const int row = 16 * (tile - (seg == 0 ? 0 : seg == 1 ? a.tiles0 : a.tiles1)) + fr;
+        const int rows = seg == 0 ? a.rows[0] : seg == 1 ? a.rows[1] : a.rows[2];
+        float *out = seg == 0 ? a.out[0] + (size_t)z * a.n * rows : seg == 1 ? a.out[1] : a.out[2];
+        const size_t at = (size_t)(row < rows ? row : rows - 1) * cols;
+        const uint16_t *wr = (seg == 0 ? a.w[0] : seg == 1 ? a.w[1] : a.w[2]) + at;
+        const uint16_t *up = EPI == kSilu ? a.w[1] + at : wr;
+        f32x4 s = zero;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (row < rows && t0 + 4 * fq + i < a.n) s[i] = out[(size_t)(t0 + 4 * fq + i) * rows + row];
+        if (!any_nan(s)) continue;
+        const f32x4 was = s;
+        repair_nan(s, wr, up, row < rows, xb, a.n - t0, cols, c0, c1, fq, looked);
+        if (EPI == kSilu) {
+            f32x4 u = was;
+            repair_nan(u, up, wr, row < rows, xb, a.n - t0, cols, c0, c1, fq, looked);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s[i] = silu(s[i]) * u[i];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (was[i] != was[i] && row < rows && t0 + 4 * fq + i < a.n)
+                out[(size_t)(t0 + 4 * fq + i) * rows + row] = s[i];
+    }
 }
 
 // K steps of a wave for a block's K of `steps` steps: the fewest instances
 // whose eight waves hold it, since idle steps still issue (11 tokens x 1024 x
 // 2048 in four parts of 16 steps: 4.3 / 4.8 / 5.1 / 5.9 / 7.2 us with 2 / 3 /
 // 4 / 6 / 10 steps a wave; four waves of 8, 5.7). Past 80, chunks.
-constexpr int kWaves = 8;
+constexpr int kWaves = 8, kMaxSteps = 10 * kWaves;
 
 template <int EPI, bool NT>
 hipError_t few_launch(hipStream_t s, const Args &a, dim3 grid, int steps) {

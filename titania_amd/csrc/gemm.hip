@@ -765,21 +765,36 @@ __global__ __launch_bounds__(kF32Threads, 2) void gemm_f32_kernel(int gxy, int r
     if (half == 1) return;
     const int rows = sg.rows;
     float *out = ksplit > 1 ? part + (size_t)z * n * rows : sg.out;
-    unsigned x_seen = 0, x_bad = 0;  // repair_nan's
+    bool nan = false;
 #pragma unroll
     for (int q = 0; q < FN; ++q) {
-        f32x4 s = acc[q] + ep[wave][q][lane];
-        if constexpr (RAGGED) {
-            const int r = q * 16 + fr, last = rows - 1 - sg.local;
-            repair_nan(s, w + (size_t)min(r, last) * cols, r <= last, xk + (size_t)min(t0 + wm, n - 1) * cols,
-                       n - t0 - wm, cols, 0, min(nk * T::BK, cols - kb * T::BK), fq, x_seen, x_bad);
-        }
+        const f32x4 s = acc[q] + ep[wave][q][lane];
+        if constexpr (RAGGED) nan |= any_nan(s);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int t = t0 + wm + fq * 4 + i, r = q * 16 + fr;
             if (t >= n || (RAGGED && sg.local + r >= rows)) continue;
             out[(size_t)t * rows + sg.local + r] = s[i];
         }
+    }
+    if (!RAGGED || __builtin_expect(!nan, 1)) return;
+    // The wave's sums again, for what infinite weights made NaN.
+    const int last = rows - 1 - sg.local, tokens = n - t0 - wm;
+    unsigned looked = 0;
+#pragma unroll 1
+    for (int r = fr; r - fr < T::BN; r += 16) {
+        float *o = out + (size_t)(t0 + wm) * rows + sg.local + r;
+        f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (r <= last && fq * 4 + i < tokens) s[i] = o[(size_t)(fq * 4 + i) * rows];
+        if (!any_nan(s)) continue;
+        const uint16_t *wr = w + (size_t)min(r, last) * cols;
+        repair_nan(s, wr, wr, r <= last, xk + (size_t)(t0 + wm) * cols, tokens, cols, 0,
+                   min(nk * T::BK, cols - kb * T::BK), fq, looked);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (r <= last && fq * 4 + i < tokens) o[(size_t)(fq * 4 + i) * rows] = s[i];
     }
 }
 
