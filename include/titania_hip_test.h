@@ -118,6 +118,11 @@ TH_API int th_test_matmul_route(size_t n, size_t rows, size_t cols, int *kernel,
  * few-token kernel where the GEMM would take them too. Needs no GPU. */
 TH_API int th_test_few_preferred(size_t n, size_t rows, size_t cols, int n_outs, int *few);
 
+/* Whether n tokens of gate and up (rows2 0), or of q, k and v, of these rows
+ * share a launch of the few-token kernel where the GEMM does not take them.
+ * Needs no GPU. */
+TH_API int th_test_few_together(size_t n, size_t rows0, size_t rows1, size_t rows2, size_t cols, int *few);
+
 #ifdef __cplusplus
 }
 #endif

@@ -45,6 +45,7 @@ TEST_SIGNATURES = {
     "th_test_attention_prefill": [_P, _P, _P, _P, _SZ, _SZ, _SZ, _SZ, _SZ, C.c_int, _P],
     "th_test_matmul_route": [_SZ, _SZ, _SZ, C.POINTER(C.c_int), C.POINTER(C.c_int)],
     "th_test_few_preferred": [_SZ, _SZ, _SZ, C.c_int, C.POINTER(C.c_int)],
+    "th_test_few_together": [_SZ, _SZ, _SZ, _SZ, _SZ, C.POINTER(C.c_int)],
 }
 EPS = 1e-6
 

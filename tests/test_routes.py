@@ -30,6 +30,40 @@ def few_preferred(n, rows, cols, n_outs):
     return bool(few.value)
 
 
+def few_together(n, rows, cols):
+    few = C.c_int()
+    f = C.CDLL(str(LIB_PATH)).th_test_few_together
+    f.argtypes = [C.c_size_t] * 5 + [C.POINTER(C.c_int)]
+    check(f(n, *rows, *[0] * (3 - len(rows)), cols, C.byref(few)))
+    return bool(few.value)
+
+
+@pytest.mark.parametrize("n,rows,cols,kernel", [
+    (2, 1024, 1024, GEMV), (3, 9728, 2560, GEMV), (4, 1024, 1024, GEMV), (4, 9728, 2560, GEMV), (4, 5003, 2968, GEMV),
+    (4, 151936, 512, GEMV), (5, 1024, 1024, FEW), (4, 16384, 1024, FEW), (4, 8192, 3072, FEW), (15, 9001, 3000, FEW),
+    (3, 100, 12, SCALAR), (40, 100, 12, SCALAR)])
+def test_single_matrix_of_few_tokens(n, rows, cols, kernel):
+    assert route(n, rows, cols)[0] == kernel
+
+
+@pytest.mark.parametrize("n,rows,cols", [(4, 8192, 3072), (8, 9001, 3000), (15, 4096, 8192), (5, 64000, 4096),
+                                         (9, 40, 9736)])
+def test_few_tokens_hold_their_columns(n, rows, cols):
+    """K in parts of at most 2560 columns, which the registers hold."""
+    kernel, ksplit = route(n, rows, cols)
+    assert kernel == FEW and (cols + 31) // 32 <= 80 * ksplit
+
+
+@pytest.mark.parametrize("n,rows,cols,few", [
+    (2, (9728, 9728), 2560, False), (3, (9728, 9728), 2560, True), (2, (3072, 3072), 1024, True),
+    (15, (1000, 1000), 520, True), (2, (8192, 8192), 4096, False), (15, (2048, 2048), 4096, False),
+    (2, (4096, 1024, 1024), 4096, False), (3, (4096, 1024, 1024), 4096, True), (4, (4096, 1024, 1024), 4096, True), (8, (8192, 1024, 1024), 8192, False),
+    (20, (1003, 1003), 1096, True), (700, (5003, 5003), 2968, False),
+    (64, (9728, 9728), 2560, False), (1, (64, 64), 64, False)])
+def test_matrices_share_a_launch(n, rows, cols, few):
+    assert few_together(n, rows, cols) == few
+
+
 @pytest.mark.parametrize("n,rows,cols,kernel", [
     (16, 6144, 1024, FEW), (33, 6144, 1024, FEW), (64, 6144, 1024, FEW), (64, 2048, 1024, FEW), (16, 16384, 1024, FEW),
     (16, 151936, 1024, FEW), (32, 16384, 1024, GEMM_F32), (64, 32768, 512, GEMM_F32), (64, 16384, 1024, GEMM_F32),

@@ -155,6 +155,8 @@ struct MatmulRoute {
     int ksplit;
 };
 MatmulRoute matmul_route(size_t n, size_t rows, size_t cols, bool part);
+// About how long launch_matmul takes, with room for partials.
+double matmul_us(size_t n, size_t rows, size_t cols);
 
 // out[t*rows + r] = dot(w[r], x[t]) for t < n. Where it splits K, the partials
 // go to part (kPartFloats long; null: it does not split).

@@ -564,15 +564,15 @@ int th_qkv_rope_append(th_device *dev, th_buffer *q, th_buffer *k, th_buffer *v,
         TH_NOT_CAPTURING(dev, "a projection of 16 or more tokens (stream-ordered scratch)");
         const th::GemmOut o[3] = {{wq->ptr, qd, q->ptr}, {wk->ptr, kvd, k->ptr}, {wv->ptr, kvd, v->ptr}};
         TH_HIP(th::launch_gemm_outs(dev->stream, xb->ptr, n, H, o, 3, dev->part));
-    } else if (n > 1 && th::few_supported(n, qd, H)) {
+    } else if (const size_t each[3] = {qd, kvd, kvd}; th::few_together(n, each, 3, H)) {
         if (n >= th::kGemmMinTokens) TH_NOT_CAPTURING(dev, "a projection of 16 or more tokens (stream-ordered scratch)");
         const th::GemmOut o[3] = {{wq->ptr, qd, q->ptr}, {wk->ptr, kvd, k->ptr}, {wv->ptr, kvd, v->ptr}};
         TH_HIP(th::launch_few(dev->stream, xb->ptr, n, H, o, 3, nullptr, 1));
     } else {
         if (n >= th::kGemmMinTokens) TH_NOT_CAPTURING(dev, "a projection of 16 or more tokens (stream-ordered scratch)");
-        TH_HIP(th::launch_matmul(dev->stream, q->ptr, wq->ptr, qd, H, xb->ptr, n));
-        TH_HIP(th::launch_matmul(dev->stream, k->ptr, wk->ptr, kvd, H, xb->ptr, n));
-        TH_HIP(th::launch_matmul(dev->stream, v->ptr, wv->ptr, kvd, H, xb->ptr, n));
+        TH_HIP(th::launch_matmul(dev->stream, q->ptr, wq->ptr, qd, H, xb->ptr, n, dev->part));
+        TH_HIP(th::launch_matmul(dev->stream, k->ptr, wk->ptr, kvd, H, xb->ptr, n, dev->part));
+        TH_HIP(th::launch_matmul(dev->stream, v->ptr, wv->ptr, kvd, H, xb->ptr, n, dev->part));
     }
     // The q/k norms, the rotations and the appends (model.rs:111-120), one
     // wave per (token, head), into the trait's position-major caches.
@@ -616,15 +616,15 @@ int th_gate_up_silu(th_device *dev, th_buffer *gate, th_buffer *up, const th_wei
         TH_NOT_CAPTURING(dev, "a projection of 16 or more tokens (stream-ordered scratch)");
         const th::GemmOut o[2] = {{w_gate->ptr, I, gate->ptr}, {w_up->ptr, I, up->ptr}};
         TH_HIP(th::launch_gemm_outs(dev->stream, xb->ptr, n, H, o, 2, dev->part));
-    } else if (n > 1 && th::few_supported(n, I, H)) {
+    } else if (const size_t each[2] = {I, I}; th::few_together(n, each, 2, H)) {
         if (n >= th::kGemmMinTokens) TH_NOT_CAPTURING(dev, "a projection of 16 or more tokens (stream-ordered scratch)");
         // Both projections and silu(gate) * up in one launch; up unused.
         TH_HIP(th::launch_few_silu(dev->stream, xb->ptr, n, H, w_gate->ptr, w_up->ptr, I, gate->ptr));
         return TH_OK;
     } else {
         if (n >= th::kGemmMinTokens) TH_NOT_CAPTURING(dev, "a projection of 16 or more tokens (stream-ordered scratch)");
-        TH_HIP(th::launch_matmul(dev->stream, gate->ptr, w_gate->ptr, I, H, xb->ptr, n));
-        TH_HIP(th::launch_matmul(dev->stream, up->ptr, w_up->ptr, I, H, xb->ptr, n));
+        TH_HIP(th::launch_matmul(dev->stream, gate->ptr, w_gate->ptr, I, H, xb->ptr, n, dev->part));
+        TH_HIP(th::launch_matmul(dev->stream, up->ptr, w_up->ptr, I, H, xb->ptr, n, dev->part));
     }
     TH_HIP(th::launch_silu_mul(dev->stream, gate->ptr, up->ptr, n * I));
     return TH_OK;

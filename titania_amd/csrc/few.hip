@@ -270,10 +270,13 @@ int few_ksplit(size_t n, size_t rows, size_t cols) {
     // Few row tiles leave CUs idle and make each read all of x: K in up to
     // four parts of at least 16 steps (11 tokens, one part / two / four: x
     // 1024 x 2048 8.1 / 6.4 / 4.3 us, 1024 x 3072 16.0 / 7.2 / 5.2, 2560 x
-    // 4096 17.7 / 10.1 / 8.6, 2560 x 9728 31.5 / 32.3 / 16.6).
+    // 4096 17.7 / 10.1 / 8.6, 2560 x 9728 31.5 / 32.3 / 16.6). And K that the
+    // registers do not hold (chunks read x again for every 16 rows), in as many
+    // parts as they do: 8 tokens x 8192 x 3072 25.1 -> 15.0 us, x 9001 x 3000 34.2
+    // -> 20.1, x 4096 x 8192 32.2 -> 19.3, x 64000 x 4096 172 -> 95.
     const size_t tiles = (rows + 15) / 16 * ((n + kTokens - 1) / kTokens), steps = (cols + 31) / 32;
     int k = 1;
-    while (k < kFewMaxSplitK && tiles * k < 512 && steps / (2 * k) >= 16) k *= 2;
+    while (k < kFewMaxSplitK && steps / (2 * k) >= 16 && (tiles * k < 512 || steps > kMaxSteps * k)) k *= 2;
     return k;
 }
 
@@ -300,12 +303,37 @@ bool few_preferred(size_t n, size_t rows, size_t cols, int n_outs) {
     return work <= (cols > 2560 ? 8192 : n <= 32 ? 40960 : 32768);
 }
 
-double few_us(size_t n, size_t rows, size_t cols) {
+bool few_together(size_t n, const size_t *rows, int n_outs, size_t cols) {
+    size_t total = 0;
+    bool whole = true;
+    double each = n_outs == 2 ? 3 : 0;  // silu_mul
+    for (int i = 0; i < n_outs; ++i) {
+        if (n < 2 || !few_supported(n, rows[i], cols)) return false;
+        total += rows[i];
+        whole = whole && gemm_supported(rows[i], cols);
+        each += matmul_us(n, rows[i], cols);
+    }
+    if (n >= kGemmMinTokens && whole) return few_preferred(n, total, cols, n_outs);
+    // Launches together do not split K: past what the registers hold, in
+    // chunks. Us together / each: gate and up of 8192 x 4096, 2 / 3 / 8 tokens
+    // 40.4 / 32.6, 40.8 / 38.2, 46.5 / 40.0, of 2048 x 4096 22.6 / 18.9, 23.1 /
+    // 21.7, 26.1 / 20.5; q, k and v of 12288 x 4096, 2 / 3 tokens 36.7 / 32.7, 36.9
+    // / 36.4, of 6144 x 4096 27.6 / 29.2, 28.1 / 33.2, of 10240 x 8192, 3 / 8
+    // tokens 64.6 / 66.1, 71.7 / 56.7. And of two tokens the GEMV is as fast where the
+    // weights are many: gate and up of 9728 x 2560 28.1 / 26.3, of 3072 x 1024 6.2
+    // / 10.2.
+    if (n == 2 && (cols > 2560 || total * cols > ((size_t)40 << 20))) return false;
+    if (n_outs == 2 && cols > 2560) return false;
+    return n == 3 || (n < kGemmMinTokens && cols <= 2560) || few_us(n, total, cols) <= each;
+}
+
+double few_us(size_t n, size_t rows, size_t cols, int ksplit) {
     // Rounds of row tiles, past the chunks that the registers hold three times
-    // as long a column; besides, the launch and the first read of x.
-    const size_t y = (n + kTokens - 1) / kTokens, slots = std::max<size_t>(1, 256 / y);
-    const double rounds = (double)(((rows + 15) / 16 + slots - 1) / slots), c = 1e-3 * (double)cols;
-    return cols > 2560 ? 4 + 3 * rounds * c : 4 + 2 * c + rounds * std::max(0.9 * c, 0.5);
+    // as long a column; besides, the launch and the first read of x, and the
+    // sum of the parts.
+    const size_t y = (n + kTokens - 1) / kTokens * (size_t)ksplit, slots = std::max<size_t>(1, 256 / y);
+    const double rounds = (double)(((rows + 15) / 16 + slots - 1) / slots), c = 1e-3 * (double)cols / ksplit;
+    return (c > 2.56 ? 4 + 3 * rounds * c : 4 + 2 * c + rounds * std::max(0.9 * c, 0.5)) + (ksplit > 1 ? 2 : 0);
 }
 
 hipError_t launch_few(hipStream_t s, const float *x, size_t n, size_t cols, const GemmOut *outs, int n_outs,

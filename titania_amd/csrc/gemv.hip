@@ -97,19 +97,31 @@ static hipError_t gemv(hipStream_t s, float *out, const uint16_t *w, size_t rows
 MatmulRoute matmul_route(size_t n, size_t rows, size_t cols, bool part) {
     if (cols % 8 != 0) return {kMatmulScalar, 1};
     if (n >= kGemmMinTokens && gemm_supported(rows, cols) && !few_preferred(n, rows, cols, 1)) return {kMatmulGemm, 1};
-    // Two and three tokens stay on the GEMV (x 4096 x 1024, 2 / 4 / 8 tokens:
-    // 4.2 / 5.6 / 8.7 us against few.hip's 5.5 / 5.6 / 5.7; 19456 x 2560, 2 / 3 / 4
-    // / 8: 21.4 / 25.9 / 29.8 / 46.8 against 25.8 / 25.7 / 25.9 / 26.1).
+    // Two and three tokens stay on the GEMV, and four of few enough rows and
+    // columns (weights from HBM, this / few.hip, 2 / 3 / 4 / 5 tokens: x 1024 x
+    // 1024 3.6, 4.5, 4.8 / 5.9, 6.6 / 6.0; 9728 x 2560, 4 and 5 16.3 / 18.4, 21.5 /
+    // 18.4; 16384 x 1024, 4 11.3 / 9.5; 5003 x 2968 12.8 / 14.2; 8192 x 3072 16.0
+    // / 14.9; 151936 x 512 46.3 / 50.8).
     if (n <= 3 || !few_supported(n, rows, cols)) return {kMatmulGemv, 1};
+    if (n == 4 && ((cols < 3072 && rows <= 12288) || cols <= 512)) return {kMatmulGemv, 1};
     auto fits = [&](int k) { return part && (size_t)k * n * rows <= kPartFloats; };
-    int ksplit = n < kGemmMinTokens ? few_ksplit(n, rows, cols) : 1;
+    int ksplit = n < kGemmMinTokens || (n == kGemmMinTokens && !gemm_supported(rows, cols)) ? few_ksplit(n, rows, cols) : 1;
     if (!fits(ksplit)) ksplit = 1;
     if (n > 16 && gemm_ragged_supported(n, rows, cols) && !gemm_supported(rows, cols)) {
         int k = gemm_ragged_ksplit(n, rows, cols);
         if (!fits(k)) k = 1;
-        if (gemm_ragged_us(n, rows, cols, k) + 2 < few_us(n, rows, cols)) return {kMatmulRagged, k};
+        if (gemm_ragged_us(n, rows, cols, k) + 2 < few_us(n, rows, cols, ksplit)) return {kMatmulRagged, k};
     }
     return {kMatmulFew, ksplit};
+}
+
+double matmul_us(size_t n, size_t rows, size_t cols) {
+    const MatmulRoute r = matmul_route(n, rows, cols, true);
+    if (r.kernel == kMatmulFew) return few_us(n, rows, cols, r.ksplit);
+    if (r.kernel == kMatmulRagged) return gemm_ragged_us(n, rows, cols, r.ksplit);
+    if (r.kernel == kMatmulGemm) return gemm_ragged_us(n, rows, cols, gemm_ragged_ksplit(n, rows, cols));  // much alike
+    // The GEMV's bytes, 4 tokens a pass.
+    return (double)((n + 3) / 4) * (3.5 + (double)(rows * cols) * 2 / 4.5e6);
 }
 
 hipError_t launch_matmul(hipStream_t s, float *out, const uint16_t *w, size_t rows, size_t cols, const float *x,

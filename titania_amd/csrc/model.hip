@@ -584,6 +584,8 @@ int enqueue_fused(th_state *s, const uint32_t *tokens, size_t n, size_t pos, con
     // q/k/v and gate/up in a launch each; o and down may split K, their
     // partials (in the GEMM's scratch) summed by the norm that follows.
     auto few = [&](size_t rows, size_t cols) { return n > 1 && th::few_supported(n, rows, cols); };
+    const size_t qkv_rows[3] = {qd, nkv * hd, nkv * hd}, mlp_rows[2] = {I, I};
+    const bool qkv_few = th::few_together(n, qkv_rows, 3, H), mlp_few = th::few_together(n, mlp_rows, 2, H);
     auto one_residual = [&]() {
         res = s->fy;
         nres = 1;
@@ -605,7 +607,7 @@ int enqueue_fused(th_state *s, const uint32_t *tokens, size_t n, size_t pos, con
                 res_stride = n * H;
             }
         } else {
-            TH_HIP(th::launch_matmul(st, s->fy, w, H, cols, x, n));
+            TH_HIP(th::launch_matmul(st, s->fy, w, H, cols, x, n, d->part));
         }
         return TH_OK;
     };
@@ -703,14 +705,14 @@ int enqueue_fused(th_state *s, const uint32_t *tokens, size_t n, size_t pos, con
                 const th::GemmOut o[3] = {
                     {L.q->ptr, qd, s->fq}, {L.k->ptr, nkv * hd, s->fk}, {L.v->ptr, nkv * hd, s->fv}};
                 TH_HIP(th::launch_gemm_multi(st, s->fxb, n, H, o, 3, s->fsplit, s->fsplit_bytes));
-            } else if (few(qd, H)) {
+            } else if (qkv_few) {
                 const th::GemmOut o[3] = {
                     {L.q->ptr, qd, s->fq}, {L.k->ptr, nkv * hd, s->fk}, {L.v->ptr, nkv * hd, s->fv}};
                 TH_HIP(th::launch_few(st, s->fxb, n, H, o, 3, nullptr, 1));
             } else {
-                TH_HIP(th::launch_matmul(st, s->fq, L.q->ptr, qd, H, s->fxb, n));
-                TH_HIP(th::launch_matmul(st, s->fk, L.k->ptr, nkv * hd, H, s->fxb, n));
-                TH_HIP(th::launch_matmul(st, s->fv, L.v->ptr, nkv * hd, H, s->fxb, n));
+                TH_HIP(th::launch_matmul(st, s->fq, L.q->ptr, qd, H, s->fxb, n, d->part));
+                TH_HIP(th::launch_matmul(st, s->fk, L.k->ptr, nkv * hd, H, s->fxb, n, d->part));
+                TH_HIP(th::launch_matmul(st, s->fv, L.v->ptr, nkv * hd, H, s->fxb, n, d->part));
             }
             TH_HIP(th::launch_qk_norm_rope_append(st, qa));
         }
@@ -752,11 +754,11 @@ int enqueue_fused(th_state *s, const uint32_t *tokens, size_t n, size_t pos, con
             const th::GemmOut o[2] = {{L.gate->ptr, I, s->fgate}, {L.up->ptr, I, s->fup}};
             TH_HIP(th::launch_gemm_multi(st, s->fxb, n, H, o, 2, s->fsplit, s->fsplit_bytes));
             TH_HIP(th::launch_silu_mul(st, s->fgate, s->fup, n * I));
-        } else if (few(I, H)) {
+        } else if (mlp_few) {
             TH_HIP(th::launch_few_silu(st, s->fxb, n, H, L.gate->ptr, L.up->ptr, I, s->fgate));
         } else {
-            TH_HIP(th::launch_matmul(st, s->fgate, L.gate->ptr, I, H, s->fxb, n));
-            TH_HIP(th::launch_matmul(st, s->fup, L.up->ptr, I, H, s->fxb, n));
+            TH_HIP(th::launch_matmul(st, s->fgate, L.gate->ptr, I, H, s->fxb, n, d->part));
+            TH_HIP(th::launch_matmul(st, s->fup, L.up->ptr, I, H, s->fxb, n, d->part));
             TH_HIP(th::launch_silu_mul(st, s->fgate, s->fup, n * I));
         }
         if (!few_path && use_gemm(I) && th::gemm_supported(H, I)) {

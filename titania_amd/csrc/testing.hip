@@ -420,4 +420,11 @@ int th_test_few_preferred(size_t n, size_t rows, size_t cols, int n_outs, int *f
     return TH_OK;
 }
 
+int th_test_few_together(size_t n, size_t rows0, size_t rows1, size_t rows2, size_t cols, int *few) {
+    TH_REQUIRE(few && rows0 > 0 && rows1 > 0, "th_test_few_together: two or three matrices");
+    const size_t rows[3] = {rows0, rows1, rows2};
+    *few = th::few_together(n, rows, rows2 ? 3 : 2, cols);
+    return TH_OK;
+}
+
 }  // extern "C"
