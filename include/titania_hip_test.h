@@ -123,6 +123,9 @@ TH_API int th_test_few_preferred(size_t n, size_t rows, size_t cols, int n_outs,
  * Needs no GPU. */
 TH_API int th_test_few_together(size_t n, size_t rows0, size_t rows1, size_t rows2, size_t cols, int *few);
 
+/* Splits that th_attention takes for n tokens at pos, head_dim 128. Needs no GPU. */
+TH_API int th_test_attention_splits(size_t n, size_t n_heads, size_t n_kv_heads, size_t pos, int *splits);
+
 #ifdef __cplusplus
 }
 #endif

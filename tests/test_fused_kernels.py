@@ -46,6 +46,7 @@ TEST_SIGNATURES = {
     "th_test_matmul_route": [_SZ, _SZ, _SZ, C.POINTER(C.c_int), C.POINTER(C.c_int)],
     "th_test_few_preferred": [_SZ, _SZ, _SZ, C.c_int, C.POINTER(C.c_int)],
     "th_test_few_together": [_SZ, _SZ, _SZ, _SZ, _SZ, C.POINTER(C.c_int)],
+    "th_test_attention_splits": [_SZ, _SZ, _SZ, _SZ, C.POINTER(C.c_int)],
 }
 EPS = 1e-6
 

@@ -91,3 +91,16 @@ def test_several_matrices(n, rows, cols, few):
 def test_odd_products_split_k(n, rows, cols):
     """An odd number of results does not keep K in one part."""
     assert n * rows % 2 and route(n, rows, cols)[1] > 1
+
+
+@pytest.mark.parametrize("n,heads,kv_heads,pos,low,high", [
+    (16, 64, 8, 1500, 8, 12), (24, 64, 8, 1000, 6, 9), (300, 4, 2, 700, 6, 8), (500, 4, 2, 500, 6, 8),  # 1024 rows or more
+    (11, 32, 8, 700, 12, 12), (11, 32, 8, 4000, 20, 32), (64, 16, 8, 30000, 16, 32), (64, 16, 8, 60, 1, 1)])
+def test_attention_splits(n, heads, kv_heads, pos, low, high):
+    """Within a few percent of the best measured count: fewer for many (token,
+    head) rows, whose combine takes longer for each."""
+    splits = C.c_int()
+    f = C.CDLL(str(LIB_PATH)).th_test_attention_splits
+    f.argtypes = [C.c_size_t] * 4 + [C.POINTER(C.c_int)]
+    check(f(n, heads, kv_heads, pos, C.byref(splits)))
+    assert low <= splits.value <= high

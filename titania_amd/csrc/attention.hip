@@ -582,6 +582,8 @@ __global__ __launch_bounds__(64) void attn_combine_lanes_kernel(float *__restric
 // attention_splits_at: most splits, and most blocks (of kGqaRows rows and a
 // split each) where that is more than one.
 constexpr size_t kMaxRoundSplits = 64, kMaxRoundBlocks = 1024;
+// (token, head) rows from which the combine gives each a wave of its own.
+constexpr size_t kCombineWaveRows = 1024;
 
 int attention_splits(size_t n, size_t n_heads, size_t n_kv_heads, size_t max_len, size_t head_dim) {
     // Several tokens on the matrix cores: split the keys until the launch has
@@ -630,12 +632,19 @@ int attention_splits_at(size_t n, size_t n_heads, size_t n_kv_heads, size_t pos,
     // at 2500, 256 blocks: 4.78 ms in two splits, 4.99 in one).
     if (blocks > 96) return least;
     const size_t tiles = (pos + n + kGqaKeys - 1) / kGqaKeys;
+    // The combine of many rows (a wave each: launch_attn_combine) reads a
+    // row's splits one after another: its time goes by their count, where the
+    // other's goes by the partials' bytes (16 tokens at 1500 of 64 / 8 heads in
+    // 24 / 12 / 8 splits 22.7 / 19.3 / 20.2 us, 500 at 500 of 4 / 2 in 16 / 8 21.0
+    // / 19.0).
+    const double rows = (double)(n * n_heads);
+    const bool wave = n * n_heads >= kCombineWaveRows;
     double best = 1e30;
     size_t ns = 1;
     for (size_t k = 1; k <= std::min(tiles, kMaxRoundSplits) && (k == 1 || blocks * k <= kMaxRoundBlocks); ++k) {
         const double rounds = (double)((blocks * k + 255) / 256);
-        const double cost = rounds * (double)((tiles + k - 1) / k + 2) +
-                            (k > 1 ? 1.4 + (double)(n * n_heads * k) * 5.2e-5 : 0.);
+        const double combine = wave ? 0.8 + (double)k * (0.12 + rows * 2e-5) : 1.4 + (double)k * rows * 5.2e-5;
+        const double cost = rounds * (double)((tiles + k - 1) / k + 2) + (k > 1 ? combine : 0.);
         if (cost < best) {
             best = cost;
             ns = k;
@@ -654,7 +663,7 @@ size_t attention_scratch(size_t n, size_t n_heads, size_t head_dim, int nsplit) 
 hipError_t launch_attn_combine(hipStream_t s, float *out, const float *part_acc, const float *part_ml, size_t heads,
                                int nsplit, int hd, uint16_t *hi, uint16_t *lo) {
     if (nsplit > kMaxSplits || (!hi != !lo)) return hipErrorInvalidValue;
-    if (heads >= 1024 && nsplit <= 64 && (hd == 64 || hd == 128 || hd == 256)) {
+    if (heads >= kCombineWaveRows && nsplit <= 64 && (hd == 64 || hd == 128 || hd == 256)) {
         const dim3 grid((unsigned)((heads + 3) / 4));
         switch (hd) {
         case 64: attn_combine_wave_kernel<64><<<grid, 256, 0, s>>>(out, part_acc, part_ml, nsplit, heads, hi, lo); break;

@@ -427,4 +427,10 @@ int th_test_few_together(size_t n, size_t rows0, size_t rows1, size_t rows2, siz
     return TH_OK;
 }
 
+int th_test_attention_splits(size_t n, size_t n_heads, size_t n_kv_heads, size_t pos, int *splits) {
+    TH_REQUIRE(n > 0 && n_heads > 0 && n_kv_heads > 0 && splits, "th_test_attention_splits: empty or null argument");
+    *splits = th::attention_splits_at(n, n_heads, n_kv_heads, pos, 128);
+    return TH_OK;
+}
+
 }  // extern "C"
