@@ -9,6 +9,7 @@ error is ~1e-5, so on these seeds the streams must match exactly.
 
 from __future__ import annotations
 
+import ctypes as C
 import os
 
 import numpy as np
@@ -156,6 +157,27 @@ def test_qwen06_prompt_at_any_position(qwen06):
     times = [(ms(96), ms(100)) for _ in range(8)]
     assert min(b for _, b in times) < 1.1 * min(a for a, _ in times)
     st.close()
+
+
+def test_qwen06_short_states_keep_no_planes(qwen06):
+    """States too short for a prompt that takes the attention's planes (320
+    tokens) do not hold any: 2.6 MB a state."""
+    m, _ = qwen06
+    hiprt, free, total = C.CDLL("libamdhip64.so"), C.c_size_t(), C.c_size_t()
+
+    def used(max_len, n=24):
+        hiprt.hipMemGetInfo(C.byref(free), C.byref(total))
+        before = free.value
+        states = [State(m, max_len) for _ in range(n)]
+        for st in states:
+            m.forward(st, [1, 2], 0, TH_PATH_FUSED, want_logits=False)
+        hiprt.hipMemGetInfo(C.byref(free), C.byref(total))
+        for st in states:
+            st.close()
+        return before - free.value
+
+    used(320)
+    assert used(319) < used(320) - 24 * (2 << 20)
 
 
 def test_qwen06_greedy(qwen06):

@@ -334,7 +334,7 @@ int ensure_fused_state(th_state *s) {
             std::max(s->attn_part_floats, th::attention_scratch(n, (size_t)c.num_attention_heads, hd, ns));
     }
     if (s->attn_part_floats) TH_HIP(hipMalloc(&s->attn_part, s->attn_part_floats * sizeof(float)));
-    if (s->kv_dtype == TH_KV_F32 && s->fb >= th::kGemmMinTokens && hd == 128) {
+    if (s->kv_dtype == TH_KV_F32 && s->fb >= kPlaneMinTokens && hd == 128) {
         s->kv_planes_bytes = th::attention_planes_bytes(s->max_len, (size_t)c.num_key_value_heads);
         TH_HIP(hipMalloc(&s->kv_planes, s->kv_planes_bytes));
         // Zeroed: the attention reads whole 64-key tiles, and the keys of a
