@@ -107,6 +107,11 @@ TH_API int th_test_attention_prefill(th_device *dev, const th_buffer *q, const t
                                      const th_buffer *v_cache, size_t max_len, size_t pos, size_t n, size_t n_heads,
                                      size_t n_kv_heads, int planes, th_buffer *out);
 
+/* The GEMM for matrices that are not whole tiles: out = w . x for n rows of x,
+ * K in ksplit parts. */
+TH_API int th_test_gemm_ragged(th_device *dev, const th_weight *w, const th_buffer *x, size_t n, int ksplit,
+                               th_buffer *out);
+
 /* The kernel that th_matmul takes for n (2 or more) tokens of a [rows, cols]
  * weight, and its parts of K: 0 the scalar GEMV, 1 the GEMV, 2 the few-token
  * kernel, 3 the GEMM for matrices that are not whole tiles, 4 the small-tile

@@ -11,11 +11,15 @@ allows).
 
 from __future__ import annotations
 
+import ctypes as C
+
 import numpy as np
 import pytest
 
 from oracle import ref
+from test_routes import FEW, GEMM_F32, GEMM_LARGE, RAGGED, route
 from titania_amd import InvalidArgument, Tensor
+from titania_amd._lib import LIB_PATH, check
 from titania_amd.synth import bf16_to_f32, f32_to_bf16, normal_bf16
 from util import assert_close, numbers, rel_error, tensor
 
@@ -249,11 +253,13 @@ def test_qwen4b_prefill_gemm(hip, name, n):
     assert np.all(np.abs(got.astype(np.float64) - expected) <= 3e-5 * bound + 1e-6)
 
 
-@pytest.mark.parametrize("rows,cols,n", [(2560, 9728, 500), (9728, 2560, 129), (2560, 4160, 700), (1152, 6208, 1900)])
-def test_large_tile_split_k(hip, rows, cols, n):
-    """Matrices whose large-tile launch takes K in 3 or more parts (two for the
-    last), uneven ones and tokens past a tile's edge; the bound of
-    test_split_k_matmul."""
+@pytest.mark.parametrize("rows,cols,n,parts", [(2560, 9728, 500, 3), (9728, 2560, 129, 0), (2560, 4160, 700, 2),
+                                               (1152, 6208, 1900, 3), (1408, 9728, 400, 5), (1152, 12288, 400, 7)])
+def test_large_tile_split_k(hip, rows, cols, n, parts):
+    """Matrices whose large-tile launch takes K in 2 to 7 parts, uneven ones and
+    tokens past a tile's edge, and one whose rows the small tile takes (parts
+    0); the bound of test_split_k_matmul."""
+    assert route(n, rows, cols) == ((GEMM_LARGE, parts) if parts else (GEMM_F32, 1))
     test_split_k_matmul(hip, rows, cols, n)
 
 
@@ -261,8 +267,8 @@ def test_large_tile_split_k(hip, rows, cols, n):
 @pytest.mark.parametrize("rows,cols", [(64, 64), (64, 1088), (192, 1280), (1088, 2048), (2560, 1152), (64, 4160)])
 def test_split_k_matmul(hip, rows, cols, n):
     """Whole-tile matrices around the small GEMM tile's split of K (1 to 16
-    parts, uneven ones, one K step), one and several token tiles, tokens past
-    a tile's edge. Two bf16 terms of x are within 2^-17 of it; the f32 sums
+    parts, uneven ones, one K step: 64 x 64 from 65 tokens, the few-token kernel
+    below), one and several token tiles, tokens past a tile's edge. Two bf16 terms of x are within 2^-17 of it; the f32 sums
     add cols * 2^-24 of sum |w x| at most."""
     rng = np.random.default_rng(rows + cols + n)
     w = normal_bf16(rows * cols, 4, "splitk", 0.05)
@@ -330,10 +336,57 @@ def test_few_token_matmul(hip, rows, cols, n):
 @pytest.mark.parametrize("n", [33, 64, 65, 130, 300])
 @pytest.mark.parametrize("rows,cols", [(1, 8), (63, 64), (65, 72), (100, 1096), (40, 3000), (1003, 520), (300, 4088)])
 def test_ragged_matmul(hip, rows, cols, n):
-    """More than a few tokens of matrices that are not whole tiles: rows and
-    columns past a tile's edge by one row or chunk, K split or not, tokens
-    past a tile. Three bf16 terms are x exactly; the f32 sums add cols * 2^-24
-    of sum |w x| at most."""
+    """More than a few tokens of matrices that are not whole tiles, by the
+    kernel that th_matmul takes: the ragged GEMM with K in 10 to 16 parts for
+    rows of 3000 columns and more, the few-token kernel for the others
+    (test_gemm_ragged runs the GEMM at their sizes). Three bf16 terms are x
+    exactly; the f32 sums add cols * 2^-24 of sum |w x| at most."""
+    assert route(n, rows, cols)[0] == (RAGGED if cols >= 3000 else FEW)
+    _ragged_case(rows, cols, n, lambda w, x, out: hip.matmul(out, w, x), hip)
+
+
+@pytest.mark.parametrize("rows,cols,n,ksplit", [
+    (1, 8, 33, 1), (63, 64, 64, 1), (64, 72, 65, 1), (64, 72, 65, 2), (65, 72, 17, 2), (65, 1096, 64, 1), (127, 1096, 63, 3),
+    (129, 136, 300, 3), (1003, 520, 130, 1), (1003, 520, 129, 9), (300, 4088, 65, 1), (40, 3000, 80, 16), (5003, 264, 70, 1)])
+def test_gemm_ragged(hip, rows, cols, n, ksplit):
+    """The GEMM for matrices that are not whole tiles, unsplit and in uneven
+    parts: a last row tile of one row, of 63 and whole, a last step of one
+    chunk, tokens past a tile by one. The bound of test_ragged_matmul."""
+    def gemm(w, x, out):
+        check(_test_lib().th_test_gemm_ragged(hip.handle, w.handle, x.handle, n, ksplit, out.handle))
+
+    _ragged_case(rows, cols, n, gemm, hip)
+
+
+@pytest.mark.parametrize("rows,cols,n,ksplit", [(100, 1096, 70, 1), (100, 1096, 70, 5), (65, 72, 33, 1), (129, 520, 130, 9)])
+def test_gemm_ragged_not_finite(hip, rows, cols, n, ksplit):
+    """Infinite and NaN weights and activations, in first, last and middle
+    rows, columns, tokens and parts of K, give what their products and sums in
+    f32 give."""
+    rng = np.random.default_rng(n)
+    wf = bf16_to_f32(normal_bf16(rows * cols, 6, "inf", 0.05)).reshape(rows, cols).copy()
+    x = np.round(rng.standard_normal((n, cols)).astype(np.float32) * 4) / 4 + np.float32(0.125)  # no zero; bf16 exactly
+    wf[0, cols - 1], wf[5, 10], wf[7, cols // 2], wf[7, 30], wf[rows - 1, 0] = np.inf, -np.inf, np.inf, np.nan, np.inf
+    x[1, cols // 3], x[n - 1, cols - 1] = np.inf, np.uint32(0x7f800001).view(np.float32)  # a NaN of low bits only
+    with np.errstate(invalid="ignore"):
+        exp = (wf[None].astype(np.float64) * x[:, None].astype(np.float64)).sum(-1)
+    bx, out = hip.alloc(x.size), hip.alloc(n * rows)
+    hip.write(bx, x)
+    w = hip.upload(Tensor((rows, cols), f32_to_bf16(wf.reshape(-1))))
+    check(_test_lib().th_test_gemm_ragged(hip.handle, w.handle, bx.handle, n, ksplit, out.handle))
+    got = hip.read(out).reshape(n, rows).astype(np.float64)
+    assert np.array_equal(np.isnan(got), np.isnan(exp))
+    infinite = np.isinf(exp)
+    assert np.array_equal(got[infinite], exp[infinite]) and np.all(np.isfinite(got[np.isfinite(exp)]))
+
+
+def _test_lib():
+    lib = C.CDLL(str(LIB_PATH))
+    lib.th_test_gemm_ragged.argtypes = [C.c_void_p, C.c_void_p, C.c_void_p, C.c_size_t, C.c_int, C.c_void_p]
+    return lib
+
+
+def _ragged_case(rows, cols, n, product, hip):
     rng = np.random.default_rng(rows + cols + n)
     w = normal_bf16(rows * cols, 5, "ragged", 0.05)
     x = rng.standard_normal((n, cols)).astype(np.float32)
@@ -342,7 +395,7 @@ def test_ragged_matmul(hip, rows, cols, n):
     bx, out = hip.alloc(x.size), hip.alloc(n * rows)
     hip.write(bx, x)
     hip.write(out, np.full(n * rows, np.nan, np.float32))
-    hip.matmul(out, hip.upload(Tensor((rows, cols), w)), bx)
+    product(hip.upload(Tensor((rows, cols), w)), bx, out)
     got = hip.read(out).reshape(n, rows)
     assert np.all(np.abs(got - exp) <= cols * 2.0**-24 * size)
 

@@ -43,6 +43,7 @@ TEST_SIGNATURES = {
     "th_test_gemm_silu": [_P, _P, _P, _P, _SZ, _P],
     "th_test_add_rmsnorm_parts": [_P, _P, _P, _SZ, _P, _F, _P],
     "th_test_attention_prefill": [_P, _P, _P, _P, _SZ, _SZ, _SZ, _SZ, _SZ, C.c_int, _P],
+    "th_test_gemm_ragged": [_P, _P, _P, _SZ, C.c_int, _P],
     "th_test_matmul_route": [_SZ, _SZ, _SZ, C.POINTER(C.c_int), C.POINTER(C.c_int)],
     "th_test_few_preferred": [_SZ, _SZ, _SZ, C.c_int, C.POINTER(C.c_int)],
     "th_test_few_together": [_SZ, _SZ, _SZ, _SZ, _SZ, C.POINTER(C.c_int)],
@@ -331,8 +332,9 @@ def test_step_attention_split(hip, tlib, nh, nkv, ctx, max_len, kv_bf16):
                                          ("0.6b", 1000, 5), ("0.6b", 970, 32), ("4b", 512, 32), ("4b", 450, 7),
                                          ("narrow", 12288, 0), ("narrow", 12200, 96)])
 def test_gemm_qkv(hip, tlib, shape, n, pos):
-    """The head tile (32 tokens x one head) and, for the narrow shape, the
-    256 x 256 tile (a wave a head of 64 tokens; 12200 tokens leave the last
+    """The tile of 32 tokens x one head (100 tokens), of 64 (0.6B, 512) and of
+    128 (0.6B from 970, 4B from 450), with whole and partial 32-key slices,
+    aligned and not; and, for the narrow shape, the 256 x 256 tile (a wave a head of 64 tokens; 12200 tokens leave the last
     token tile ragged, its last V^T slice partly past the tokens)."""
     H, nh, nkv, _ = NARROW if shape == "narrow" else SHAPES[shape]
     hd, qd, kvd = 128, nh * 128, nkv * 128
@@ -403,9 +405,12 @@ def _check_planes(got, dk, dv, pos, n, nkv, L):
 
 
 @pytest.mark.parametrize("H,I,n", [(1024, 3072, 100), (1024, 3072, 512), (2560, 9728, 100), (256, 3072, 8000),
-                                   (1024, 3072, 250), (1024, 3072, 1000), (2560, 9728, 256), (512, 3200, 300)])
+                                   (1024, 3072, 250), (1024, 3072, 1000), (2560, 9728, 256), (512, 3200, 300),
+                                   (256, 16448, 64)])
 def test_gemm_silu(hip, tlib, H, I, n):
-    """The 0.6B and 4B shapes take the 64 x 64 and 128 x 128 tiles; 8000
+    """The small tile (3072 at 100 tokens; its two-stage form 16448 at 64), 64 x
+    128 (3072 at 250, 3200 at 300), 64 x 192 (3072 at 512 and 1000), 128 x 128
+    (9728); 8000
     tokens x 2 x 3072 rows, 768 tiles of 256 x 256, the largest tile with its
     SiLU epilogue in registers (against float64 products there: the oracle's
     matmul would take minutes)."""

@@ -433,4 +433,17 @@ int th_test_attention_splits(size_t n, size_t n_heads, size_t n_kv_heads, size_t
     return TH_OK;
 }
 
+int th_test_gemm_ragged(th_device *dev, const th_weight *w, const th_buffer *x, size_t n, int ksplit, th_buffer *out) {
+    TH_REQUIRE(dev && w && x && out, "th_test_gemm_ragged: null argument");
+    const size_t rows = (size_t)rows_of(w), cols = (size_t)cols_of(w);
+    TH_REQUIRE(n > 0 && x->len == n * cols && out->len == n * rows && th::gemm_ragged_supported(n, rows, cols),
+               "x and out hold n rows, of whole 8s of columns");
+    TH_REQUIRE(ksplit >= 1 && (size_t)(ksplit - 1) * 64 < cols && (size_t)ksplit * n * rows <= th::kPartFloats,
+               "a part of K has a step of 64 columns, and the partials fit");
+    TH_HIP(th::launch_gemm_ragged(dev->stream, x->ptr, n, cols, w->ptr, rows, out->ptr, dev->part, ksplit));
+    if (ksplit > 1) TH_HIP(th::launch_splitk_sum(dev->stream, dev->part, out->ptr, n * rows, ksplit));
+    TH_HIP(hipStreamSynchronize(dev->stream));
+    return TH_OK;
+}
+
 }  // extern "C"
