@@ -1,10 +1,12 @@
 /*
  * titania_hip_test.h: test-only entry points of the hip device library.
  *
- * Each runs one fused kernel of the decode step or of the prefill on caller
- * buffers, so that a test can hold it to the per-kernel bar (relative error
- * <= 1e-3) against the oracle's composition of the reference's primitives
- * (model/cpu.rs). They are not part of the Device boundary (titania_hip.h),
+ * Those that take a device each run one kernel of the decode step, of the
+ * prefill or of the ragged products on caller buffers, so that a test can hold
+ * it to the per-kernel bar (relative error <= 1e-3) against the oracle's
+ * composition of the reference's primitives (model/cpu.rs). Those that take
+ * sizes alone answer which kernel and how many splits such a call takes, and
+ * need no GPU. They are not part of the Device boundary (titania_hip.h),
  * the forward and decode paths never call them, and they may allocate and
  * wait. Caches are f32, laid out [kv_head][max_len][128] as the fused path
  * keeps them; the rope table is [max_len][64][cos, sin] (model/model.rs:239-250).
